@@ -253,9 +253,10 @@ int ql_batch_tune(ql_batch *b, int trial_steps, double *step_ms);
 enum { QL_TRANSFORM_FFT = 0, QL_TRANSFORM_DFT_MFMA = 1 };
 int ql_batch_set_transform(ql_batch *b, int NZ, int transform);
 /* Substep tail of the NZ group: the column reduction and the mean-field
- * kernel as two launches (QL_TAIL_TWO_KERNELS, the default) or one launch with
- * a workgroup per mean field and run (QL_TAIL_FUSED: fixed steps, NZ <= 128,
- * at most 65536 / NZ partial rows per run, else QL_ERR_ARG).  Both sum the
+ * kernel as two launches (QL_TAIL_TWO_KERNELS) or one launch with a workgroup
+ * per mean field and run (QL_TAIL_FUSED: fixed steps, NZ <= 128, at most
+ * 65536 / NZ partial rows per run, else QL_ERR_ARG; the default for FP64 sets
+ * of few runs at NZ <= 64, by the measured rule of default_shape).  Both sum the
  * stress / EMF partial rows in the same order: the results are bitwise equal.
  * No counterpart in the reference (its MPI Allreduce, MHD_FullQlin.cpp:386,
  * followed by the mean-field update, :386-423). */

@@ -411,8 +411,11 @@ int create_batch(Batch &b, const ql_params *ps, int nruns)
         QL_HIP(hipMemcpy(g.kzv, r0.h_kz.data(), sizeof(double) * g.nz, hipMemcpyHostToDevice));
         QL_HIP(hipMemcpy(g.tw, htw.data(), sizeof(double2) * g.NZ, hipMemcpyHostToDevice));
         QL_HIP(hipMemcpy(g.tw32, htw32.data(), sizeof(float2) * g.NZ, hipMemcpyHostToDevice));
-        const int line = default_line(g.NZ, b.precision, b.hd);
-        QL_RC(configure(b, g, line, default_target(line)));
+        const Shape sh = default_shape(g.NZ, b.precision, g.nruns, g.modes);
+        QL_RC(configure(b, g, sh.line, sh.target));
+        g.tail = sh.tail;
+        for (const qlk::RunParams &rp : g.h_rp)
+            if (rp.nwg * g.NZ > TAIL_ONE) g.tail = 0;
     }
     return QL_OK;
 }

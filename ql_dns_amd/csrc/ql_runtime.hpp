@@ -54,13 +54,42 @@ constexpr int DEFAULT_LINE = 256, DEFAULT_TARGET = 512;
 
 inline bool valid_NZ(int NZ) { return NZ == 32 || NZ == 64 || NZ == 128 || NZ == 256; }
 inline int mb_for(int NZ, int line) { return (line == LINE_WAVE || NZ >= line) ? 1 : line / NZ; }
-// shape before tuning: the wavefront kernel, which measured fastest at NZ =
-// 128 and 256 for every model and precision (in mixed precision at NZ = 256 it
-// runs the flagged modes in FP64 itself, which beats the workgroup kernel plus
-// its companion: 2672 against 2625 steps/s at 128x128x256), with about one
-// workgroup per CU
-inline int default_line(int NZ, int, bool) { return NZ >= 128 ? LINE_WAVE : DEFAULT_LINE; }
-inline int default_target(int line) { return line == LINE_WAVE ? 256 : DEFAULT_TARGET; }
+// Shape before tuning, by NZ, the group's mode count and its run count; us per
+// FP64 step, old default (line 256, 512 workgroups, two-kernel tail) against
+// the rule's choice, MHD_FullQlin:
+//   NZ >= 128      the wavefront kernel, about one workgroup per CU, for every
+//                  model and precision (64x128x128: 131 -> 109);
+//   NZ = 64        FP64 groups of few runs take it too: 16x16 42.0 -> 36.6,
+//                  32x32 43.7 -> 39.9, 36x60 54.2 -> 45.7, 128x128 113.6 -> 100.4;
+//   NZ = 32        up to 512 modes (16x16 41.4 -> 34.6, 32x32 42.3 -> 36.1); beyond
+//                  that eight modes per pass keep more lanes busy (128x128 74.8
+//                  against 82.7);
+//   few modes      at least 64 workgroups, then four modes each: fewer rows for
+//                  the tail to sum (32x32x64: 124 workgroups 39.9, 248 41.8);
+//   tail           one launch at NZ <= 64 and at most TAIL_ONE / NZ rows per run,
+//                  which saves a launch (2-4 us per step); with more rows (NZ =
+//                  64, 504 rows: 78.4 against 77.5) or longer ones (NZ = 128, 252
+//                  rows: 116 against 109; 60 rows: 55.2 against 53.0) its
+//                  workgroups read too much each.
+// Groups of more than SMALL_SET runs fill the chip and share it with the other
+// groups: there eight (four) modes per pass and two launches measured best (48
+// runs: 160.0 us per step; wavefront kernel at NZ = 64 164.0, one-launch tail
+// 166-172; at 8 runs the one-launch tail won, 97.6 -> 79.0).
+constexpr int SMALL_SET = 4, SMALL_MODES = 512, TAIL_ONE = 16384;
+struct Shape {
+    int line, target, tail;
+};
+inline Shape default_shape(int NZ, int precision, int nruns, int modes)
+{
+    const bool small = precision == QL_PREC_FP64 && nruns <= SMALL_SET;
+    const int tail = small && NZ <= 64 ? 1 : 0;
+    if (NZ >= 128) return Shape{LINE_WAVE, 256, tail};
+    if (small && (NZ == 64 || modes <= SMALL_MODES)) {
+        const int target = modes / 4 < 64 ? 64 : (modes / 4 < 256 ? modes / 4 : 256);
+        return Shape{LINE_WAVE, target, tail};
+    }
+    return Shape{DEFAULT_LINE, DEFAULT_TARGET, tail};
+}
 // the matrix-core transform (QL_TRANSFORM_DFT_MFMA): FP64 workgroup kernel, NZ 32 and 64
 inline bool dft_ok(int NZ, int precision, int line)
 {
