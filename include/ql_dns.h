@@ -256,7 +256,7 @@ int ql_batch_set_transform(ql_batch *b, int NZ, int transform);
  * kernel as two launches (QL_TAIL_TWO_KERNELS) or one launch with a workgroup
  * per mean field and run (QL_TAIL_FUSED: fixed steps, NZ <= 128, at most
  * 65536 / NZ partial rows per run, else QL_ERR_ARG; the default for FP64 sets
- * of few runs at NZ <= 64, by the measured rule of default_shape).  Both sum the
+ * of few runs at NZ <= 64 except MHD_BQlin's).  Both sum the
  * stress / EMF partial rows in the same order: the results are bitwise equal.
  * No counterpart in the reference (its MPI Allreduce, MHD_FullQlin.cpp:386,
  * followed by the mean-field update, :386-423). */

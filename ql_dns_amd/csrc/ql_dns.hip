@@ -411,7 +411,7 @@ int create_batch(Batch &b, const ql_params *ps, int nruns)
         QL_HIP(hipMemcpy(g.kzv, r0.h_kz.data(), sizeof(double) * g.nz, hipMemcpyHostToDevice));
         QL_HIP(hipMemcpy(g.tw, htw.data(), sizeof(double2) * g.NZ, hipMemcpyHostToDevice));
         QL_HIP(hipMemcpy(g.tw32, htw32.data(), sizeof(float2) * g.NZ, hipMemcpyHostToDevice));
-        const Shape sh = default_shape(g.NZ, b.precision, g.nruns, g.modes);
+        const Shape sh = default_shape(g.NZ, b.model, b.precision, g.nruns, g.modes);
         QL_RC(configure(b, g, sh.line, sh.target));
         g.tail = sh.tail;
         for (const qlk::RunParams &rp : g.h_rp)

@@ -70,7 +70,9 @@ inline int mb_for(int NZ, int line) { return (line == LINE_WAVE || NZ >= line) ?
 //                  which saves a launch (2-4 us per step); with more rows (NZ =
 //                  64, 504 rows: 78.4 against 77.5) or longer ones (NZ = 128, 252
 //                  rows: 116 against 109; 60 rows: 55.2 against 53.0) its
-//                  workgroups read too much each.
+//                  workgroups read too much each.  Not MHD_BQlin's, whose
+//                  profile lines the two tails round differently: a run continued
+//                  from its saved state must give the same bits.
 // Groups of more than SMALL_SET runs fill the chip and share it with the other
 // groups: there eight (four) modes per pass and two launches measured best (48
 // runs: 160.0 us per step; wavefront kernel at NZ = 64 164.0, one-launch tail
@@ -79,10 +81,10 @@ constexpr int SMALL_SET = 4, SMALL_MODES = 512, TAIL_ONE = 16384;
 struct Shape {
     int line, target, tail;
 };
-inline Shape default_shape(int NZ, int precision, int nruns, int modes)
+inline Shape default_shape(int NZ, int model, int precision, int nruns, int modes)
 {
     const bool small = precision == QL_PREC_FP64 && nruns <= SMALL_SET;
-    const int tail = small && NZ <= 64 ? 1 : 0;
+    const int tail = small && NZ <= 64 && model != QL_MODEL_MHD_BQLIN ? 1 : 0;
     if (NZ >= 128) return Shape{LINE_WAVE, 256, tail};
     if (small && (NZ == 64 || modes <= SMALL_MODES)) {
         const int target = modes / 4 < 64 ? 64 : (modes / 4 < 256 ? modes / 4 : 256);
