@@ -1171,7 +1171,7 @@ int diagnostics(Batch &b, int run, double t, double out[18])
     f.eta = r.p.eta;
     f.kzfac = r.kzfac;
     f.out = b.dout;
-    qlk::k_diag_final<<<1, 64, 0, b.s>>>(f);
+    qlk::k_diag_final<<<1, qlk::NT, 0, b.s>>>(f);
     QL_HIP(hipGetLastError());
     QL_HIP(hipMemcpyAsync(out, b.dout, sizeof(double) * 18, hipMemcpyDeviceToHost, b.s));
     QL_HIP(hipStreamSynchronize(b.s));
