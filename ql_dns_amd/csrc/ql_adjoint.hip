@@ -61,9 +61,8 @@ void adj_release(Batch &b)
 
 namespace {
 
-constexpr int ADJ_GMAX = 1024;
-
-int adj_line_mb(int NZ) { return NZ >= 128 ? 1 : 128 / NZ; }
+// workgroups of the reverse mode kernel, at most: two per CU
+constexpr int ADJ_GMAX = 512;
 
 int check_adjoint(const Batch &b, const char *who)
 {
@@ -147,12 +146,12 @@ template <int NZ, int MODEL>
 void launch_adj_nz(const qlk::AdjModeArgs &am, const qlk::AdjMFArgs &aa, const qlk::AdjMF2Args &ab, int W,
                    const double *gpart, const qlk::RunParams *rp1, double *grows, hipStream_t st, int stage)
 {
-    constexpr int MB = NZ >= 128 ? 1 : 128 / NZ;
     using P = typename std::conditional<MODEL == 0, qlk::ModelFull, qlk::ModelBQ>::type;
     if (stage == 0) {
         qlk::k_adj_mf_a<NZ, MODEL><<<1, qlk::NT, 0, st>>>(aa);
     } else if (stage == 1) {
-        qlk::k_adj_mode<NZ, MB, P><<<W, qlk::NT, 0, st>>>(am);
+        if (am.mode == qlk::MODE_CN) qlk::k_adj_mode<NZ, P, qlk::MODE_CN><<<W, qlk::NT, 0, st>>>(am);
+        else qlk::k_adj_mode<NZ, P, qlk::MODE_ELIN><<<W, qlk::NT, 0, st>>>(am);
         const int ncols = 8 * NZ + qlk::NGP;
         qlk::k_reduce_cols<<<dim3((ncols + qlk::RED_CW - 1) / qlk::RED_CW, 1), qlk::NT, 0, st>>>(gpart, rp1, ncols, grows);
     } else {
@@ -217,7 +216,7 @@ int adjoint_backward(Batch &b, const double *g_lin, const double *g_mf, double *
     const RunInfo &r = b.runs[0];
     const int NZ = g.NZ, nz = g.nz, nxy = r.nxy, K = A->every;
     const size_t nl = (size_t)nxy * 4 * nz, nm = (size_t)b.nMF * nz;
-    const int MB = adj_line_mb(NZ);
+    const int MB = qlk::NT / NZ;  // modes per pass of the reverse mode kernel
     const int W = std::min((nxy + MB - 1) / MB, ADJ_GMAX);
     const int ncols = 8 * NZ + qlk::NGP;
     if (!A->gu) {

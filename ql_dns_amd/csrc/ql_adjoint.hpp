@@ -47,7 +47,7 @@ __device__ __forceinline__ double neg_abs_pow_d(double x, int p)
     const double a = fabs(x), sg = x < 0 ? -1.0 : (x > 0 ? 1.0 : 0.0);
     if (p == 1) return -sg;
     if (p == 2) return -2.0 * x;
-    return -(double)p * pow(a, (double)(p - 1)) * sg;
+    return -(double)p * pow_call(a, p - 1) * sg;
 }
 
 struct AdjModeArgs {
@@ -72,46 +72,105 @@ struct AdjModeArgs {
     double t_step, dt_step;
 };
 
-// first-pass source of the reverse transforms: compact kz-slot lines
-template <int NZ>
-struct CompactSrc {
-    const double2 *v;  // [line][nz]
+// compact kz-slot lines ([line][LD]) as the first-pass source of an inverse
+// transform (zero in the dealiased band) and the last-pass sink of a forward one
+template <int NZ, int LD>
+struct CompactIO {
+    double2 *v;
     __device__ double2 operator()(int line, int g) const
     {
         using D = Dealias<NZ>;
-        return D::kept(g) ? v[line * D::nz + D::slot(g)] : make_double2(0.0, 0.0);
+        return D::kept(g) ? v[line * LD + D::slot(g)] : make_double2(0.0, 0.0);
+    }
+    __device__ void operator()(int line, int j, double2 x) const
+    {
+        using D = Dealias<NZ>;
+        if (D::kept(j)) v[line * LD + D::slot(j)] = x;
     }
 };
 
+// inverse transform of NL compact lines in buf, in place (lines of LS slots)
+template <int NZ, int NL, int LS, int LD>
+__device__ __forceinline__ void adj_inv(double2 *buf, const double2 *tw)
+{
+    using PL = Plan2<NZ>;
+    const PadIO<NZ, double2> pad{buf};
+    fft_pass_io<NZ, NL, true, PL::R1, 1, true>(tw, CompactIO<NZ, LD>{buf}, pad);
+    fft_pass_io<NZ, NL, true, PL::R2, PL::R1, true>(tw, pad, BufIO<LS, double2>{buf});
+}
+// forward transform of NL lines of LS slots in buf to compact lines, in place
+template <int NZ, int NL, int LS, int LD>
+__device__ __forceinline__ void adj_fwd(double2 *buf, const double2 *tw)
+{
+    using PL = Plan2<NZ>;
+    const PadIO<NZ, double2> pad{buf};
+    fft_pass_io<NZ, NL, false, PL::R1, 1, true>(tw, BufIO<LS, double2>{buf}, pad);
+    fft_pass_io<NZ, NL, false, PL::R2, PL::R1, true>(tw, pad, CompactIO<NZ, LD>{buf});
+}
+
+// dL/dq through the step's driving noise (ql_noise.hpp) of one entry.  The
+// noise is state independent; its ux and bx multipliers sqrt(nf lap2 / lapF)
+// depend on q through lapF = -kx(t)^2 + lap2, d/dq = mult kx t ky / lapF (ky =
+// 0 modes: none); the band mask is held fixed like the remap decision.  A
+// call of its own: the generator's registers are not the mode kernel's
+static __device__ __noinline__ double noise_q_gradient(NoiseParams np, double q, double tn, double dt,
+                                                       double kx0, double ky, double kz2, int mode, int slot,
+                                                       double2 gux, double2 gbx)
+{
+    const double kxn = rn_add(kx0, rn_mul(rn_mul(q, tn), ky));
+    const double lap2n = rn_add(rn_mul(-ky, ky), kz2);
+    const double lapF = rn_add(rn_mul(-kxn, kxn), lap2n);
+    if (!(lapF > -np.hi2 && lapF < -np.lo2)) return 0.0;
+    const double nf = rn_mul(dt, np.nfac);
+    const double mu = sqrt(rn_mul(nf, lap2n) / lapF);
+    double2 z[4];
+    noise_normals(np.seed, tn, mode, slot, z);
+    double gz = 0.0;
+    if (np.drive_u) gz += redot(z[0], gux);
+    if (np.drive_b) gz += redot(z[2], gbx);
+    return mu * kxn * (tn * ky) / lapF * np.sigma * gz;
+}
+
 // P = ModelFull (MHD_FullQlin) or ModelBQ (MHD_BQlin.cpp:117-306: 8 base
 // lines, 5 product lines, By profiles only, no B0z terms, and the dz uz
-// constant of the ky = 0 modes, whose gradient is summed over z per mode)
-template <int NZ, int MB, class P>
-__global__ __launch_bounds__(NT) void k_adj_mode(AdjModeArgs a)
+// constant of the ky = 0 modes, whose gradient is summed over z per mode).
+//
+// A 256-thread workgroup takes MB = 256 / NZ modes at a time, as the forward
+// workgroup kernel does: a thread owns one (mode, kz slot) in the spectral
+// stages, whose state and gradients it keeps in registers, and one (mode, z)
+// in the products.  Two line buffers in LDS (X lines, T lines: 52 KB at NZ =
+// 128, two workgroups per CU) and the two-pass transforms in place in them.
+// The recomputation transforms only the product lines the reverse reads: the
+// momentum lines of MHD_FullQlin (the induction lines enter N linearly with
+// constant factors) and the second line of MHD_BQlin.  Bound by the transforms
+// (21 lines per mode, LDS and FP64 issue).  Against three radix-8 passes over
+// unpadded lines with all 24 transforms and the products in two halves, whole
+// gradients: 64x64x128 RK3CN, 20 steps 16.0 -> 9.7 ms; 32x32x64, 200 steps
+// 43.2 -> 37.3 ms.
+template <int NZ, class P, int MODE>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_adj_mode(AdjModeArgs a)
 {
     constexpr bool BQ = std::is_same<P, ModelBQ>::value;
     using D = Dealias<NZ>;
-    constexpr int NZD = D::nz;
+    constexpr int MB = NT / NZ, NZD = D::nz, NZDP = bank_stride(NZD), LS = bank_stride(NZ);
+    constexpr int NIT = MB * NZD;       // (mode slot, kz slot) items
     constexpr int NLX = P::NLINE * MB;  // 6 (8) lines per mode
-    constexpr int NLT = P::NOUT * MB;   // 6 (5) lines per mode
-    constexpr int HI = MB * 2 * NZ;     // product items (mode, half, z)
-    constexpr int HW = (HI + NT - 1) / NT;
-    constexpr int NBS = P::NB > P::NOUT ? P::NB : P::NOUT;
-    constexpr int GL = BQ ? 4 : 3;      // lines whose gradient one half-item forms
-    __shared__ double2 bufX[NLX * NZ];  // X lines, then dL/dX lines
-    __shared__ double2 bufT[NLT * NZ];  // P -> T, then dL/dP
-    __shared__ double2 uin[MB * 4 * NZD];
-    __shared__ double2 sgu[MB * 4 * NZD];      // dL/du_out rows, then dL/du_in (direct terms)
-    __shared__ double2 sbase[MB * NBS * NZD];  // bases, then dL/dT (compact)
-    __shared__ double2 sdz[MB], sgdz[MB];      // ModelBQ: fac ux at kz = 0 of a ky = 0 mode, and its gradient
-    __shared__ double2 gdzz[BQ ? MB * NZ : 1]; // ModelBQ: per-z terms of that gradient
+    constexpr int NLG = P::NOUT * MB;   // 6 (5) gradient lines per mode
+    constexpr int L0 = BQ ? 1 : 0;      // the product lines the reverse reads: L0 .. L0 + NRD - 1
+    constexpr int NRD = BQ ? 1 : 3;
+    constexpr int XS = Plan2Size<NZ, NLX, LS>::SLOTS, TS = Plan2Size<NZ, NLG, LS>::SLOTS;
+    static_assert(MB * NZ == NT && NIT <= NT, "one item per thread");
+    static_assert(NLX * NZDP <= XS && NLG * NZDP <= TS, "compact lines fit the line buffers");
+    __shared__ double2 bufX[XS];  // bases, X lines, dL/dX lines, their spectra
+    __shared__ double2 bufT[TS];  // products, T, dL/dT, dL/dP lines
     __shared__ double2 tw[NZ];
-    __shared__ double skz[NZD];
-    __shared__ double silF[MB * NZD];
-    __shared__ double skx0[MB], sky[MB], skx[MB];
-    __shared__ int sidx[MB];
-    __shared__ double smfz[NZ * 8];  // [z][profile]
-    __shared__ double sgs[4 * NZ];   // dL/d(stress sums) [slot][z]
+    __shared__ double smfz[P::NMFZ * NZ];  // mean-field profiles [profile][z]
+    __shared__ double sgs[4 * NZ];         // dL/d(EMF / stress sums) [slot][z]
+    __shared__ double skx[MB], sky[MB];
+    __shared__ int sok[MB];
+    __shared__ double2 sdz[MB];               // ModelBQ: fac ux at kz = 0 of a ky = 0 mode
+    constexpr int SEG = NZ < 64 ? NZ : 64;    // lanes of a wavefront on one mode's z points
+    __shared__ double2 sgdz[BQ ? NT / SEG : 1];  // ModelBQ: partial sums of that value's gradient
     const int tid = threadIdx.x;
     const Phys ph = a.ph;
     const double q = ph.q, Om = ph.omega, B0z = ph.B0z;
@@ -123,167 +182,140 @@ __global__ __launch_bounds__(NT) void k_adj_mode(AdjModeArgs a)
     const double qt_old = to_sgpr(rn_mul(q, a.tso)), qdtl_old = to_sgpr(rn_mul(q, a.dtlo));
     const double remap_qt = to_sgpr(rn_mul(q, a.tnew));
     const bool remap_now = a.s == 3 && a.do_remap;
-    for (int k = tid; k < NZ; k += NT) tw[k] = a.tw[k];
-    for (int k = tid; k < NZD; k += NT) skz[k] = a.kzv[k];
-    for (int k = tid; k < NZ * 8; k += NT) smfz[(k % NZ) * 8 + k / NZ] = a.mfz[k];
+
+    // the thread's items, fixed for the whole kernel
+    const bool has_it = tid < NIT;
+    const int imb = tid / NZD, im = tid - imb * NZD;
+    const int zmb = tid / NZ, zz = tid - zmb * NZ;
+    const double kz = has_it ? a.kzv[im] : 0.0, kz2 = -(kz * kz);
+    for (int k = tid; k < P::NMFZ * NZ; k += NT) smfz[k] = a.mfz[k];
     for (int k = tid; k < 4 * NZ; k += NT) sgs[k] = a.gsums[k];
+    if (tid < NZ) tw[tid] = a.tw[tid];
 
     // per-thread gradient accumulators: parameters and z-profile rows
     double gq = 0, gom = 0, gnu = 0, geta = 0, gb0 = 0;
-    double accm[HW][8];
+    double accm[8];
 #pragma unroll
-    for (int p = 0; p < HW; ++p)
-#pragma unroll
-        for (int c = 0; c < 8; ++c) accm[p][c] = 0.0;
+    for (int c = 0; c < 8; ++c) accm[c] = 0.0;
 
     const int ngroups = (a.nxy + MB - 1) / MB;
     for (int g = blockIdx.x; g < ngroups; g += gridDim.x) {
-        // A: rows of this group
-        if (tid < MB) {
-            const int i = g * MB + tid;
-            sidx[tid] = i < a.nxy ? i : -1;
-            if (i < a.nxy) {
-                const double kx0 = a.kx0[i], ky = a.ky[i];
-                skx0[tid] = kx0;
-                sky[tid] = ky;
-                skx[tid] = rn_add(kx0, rn_mul(qt, ky));
-                sdz[tid] = (BQ && ky == 0.0) ? cscale(a.fac, a.u_in[(size_t)i * 4 * NZD]) : make_double2(0.0, 0.0);
-            } else {
-                skx0[tid] = sky[tid] = skx[tid] = 0.0;
-                sdz[tid] = make_double2(0.0, 0.0);
+        // A, B: the item's state row and wavenumbers, the bases (forward
+        // recomputation)
+        const int i = (has_it && g * MB + imb < a.nxy) ? g * MB + imb : -1;
+        const size_t off = (size_t)(i < 0 ? 0 : i) * 4 * NZD + im;
+        const double kx0 = i >= 0 ? a.kx0[i] : 0.0, ky = i >= 0 ? a.ky[i] : 0.0;
+        const double kx = i >= 0 ? rn_add(kx0, rn_mul(qt, ky)) : 0.0;
+        const bool zero = (ky == 0.0 && im == 0);
+        const double lap2 = zero ? 0.0 : (-ky * ky + kz2);
+        const double ilap2 = zero ? 1.0 : 1.0 / lap2;
+        if (has_it) {
+            double2 u[4];
+#pragma unroll
+            for (int f = 0; f < 4; ++f) u[f] = i >= 0 ? a.u_in[off + f * NZD] : make_double2(0.0, 0.0);
+            P::bases(u[0], u[1], u[2], u[3], kx, ky, kz, ilap2, a.fac, bufX + imb * NZDP + im, MB * NZDP);
+            if (im == 0) {
+                skx[imb] = kx;
+                sky[imb] = ky;
+                sok[imb] = i >= 0;
+                sdz[imb] = (BQ && i >= 0 && ky == 0.0) ? cscale(a.fac, u[0]) : make_double2(0.0, 0.0);
             }
         }
-        for (int k = tid; k < MB * 4 * NZD; k += NT) {
-            const int mb = k / (4 * NZD), i = g * MB + mb;
-            const bool ok = i < a.nxy;
-            const size_t off = (size_t)i * 4 * NZD + (k - mb * 4 * NZD);
-            uin[k] = ok ? a.u_in[off] : make_double2(0.0, 0.0);
-            sgu[k] = ok ? a.gu[off] : make_double2(0.0, 0.0);
-        }
         __syncthreads();
+        adj_inv<NZ, NLX, LS, NZDP>(bufX, tw);
 
-        // B, C: bases and inverse transforms (forward recomputation)
-        for (int k = tid; k < MB * NZD; k += NT) {
-            const int mb = k / NZD, m = k % NZD;
-            const double kx = skx[mb], ky = sky[mb], kz = skz[m];
-            const bool zero = (ky == 0.0 && m == 0);
-            const double lap2 = zero ? 0.0 : (-ky * ky + -(kz * kz));
-            const double ilap2 = zero ? 1.0 : 1.0 / lap2;
-            silF[k] = (sidx[mb] == 0 && m == 0) ? 1.0 : 1.0 / (-kx * kx + lap2);
-            const double2 *U = uin + mb * 4 * NZD;
-            P::bases(U[m], U[NZD + m], U[2 * NZD + m], U[3 * NZD + m], kx, ky, kz, ilap2, a.fac,
-                     sbase + mb * P::NB * NZD + m, NZD);
-        }
-        __syncthreads();
-        fft_lines_from<NZ, NLX, true>(bufX, tw, LineSrc<NZ, P, double2>{sbase, skz});
-
-        // D, E: products and forward transforms (forward recomputation)
-        for (int item = tid; item < HI; item += NT) {
-            const int mb = item / (2 * NZ), rem = item % (2 * NZ);
-            const int part = rem / NZ, z = rem % NZ;
+        // D, E: the product lines the reverse reads and their transforms
+        const double zkx = skx[zmb], zky = sky[zmb];
+        const bool zok = sok[zmb] != 0;
+        double2 *X = bufX + zmb * LS + zz;  // line l at X[l * MB * LS]
+        double2 *Y = bufT + zmb * LS + zz;
+        {
             double2 prod[3];
-            double racc[2];
-            P::products(part, bufX + mb * P::NLINE * NZ + z, NZ, smfz + z * 8, skx[mb], sky[mb],
-                        imul(skx[mb], sdz[mb]), prod, racc);
+            double racc[2], mf[P::NMFZ];
 #pragma unroll
-            for (int c = 0; c < 3; ++c)
-                if (c < P::nprod(part)) bufT[(mb * P::NOUT + P::out_line(part, c)) * NZ + z] = prod[c];
+            for (int c = 0; c < P::NMFZ; ++c) mf[c] = smfz[c * NZ + zz];
+            P::products(0, X, MB * LS, mf, zkx, zky, imul(zkx, sdz[zmb]), prod, racc);
+#pragma unroll
+            for (int c = 0; c < NRD; ++c) Y[c * MB * LS] = prod[L0 + c];
         }
         __syncthreads();
-        fft_lines<NZ, NLT, false>(bufT, tw);
+        adj_fwd<NZ, NRD * MB, LS, NZDP>(bufT, tw);
 
         // F: substep update and RHS assembly in reverse, per (mode, kz slot)
-        for (int k = tid; k < MB * NZD; k += NT) {
-            const int mb = k / NZD, m = k % NZD;
-            const int i = sidx[mb];
-            double2 *GT = sbase + mb * P::NOUT * NZD + m;  // dL/dT, compact [line][nz]
-            if (i < 0) {
-                for (int o = 0; o < P::NOUT; ++o) GT[o * NZD] = make_double2(0.0, 0.0);
-                continue;
-            }
-            const double kx = skx[mb], ky = sky[mb], kz = skz[m];
-            const double kz2 = -(kz * kz);
-            double2 *Gu = sgu + mb * 4 * NZD + m;
-            const double2 *U = uin + mb * 4 * NZD + m;
-            const double2 ux = U[0], ze = U[NZD], bx = U[2 * NZD], et = U[3 * NZD];
+        double2 *GT = bufT + imb * NZDP + im;  // T (line c at c * MB * NZDP), then dL/dT
+        if (has_it && i < 0)
+            for (int o = 0; o < P::NOUT; ++o) GT[o * MB * NZDP] = make_double2(0.0, 0.0);
+        if (i >= 0) {
+            double2 u[4];
+#pragma unroll
+            for (int f = 0; f < 4; ++f) u[f] = a.u_in[off + f * NZD];
+            const double2 ux = u[0], ze = u[1], bx = u[2], et = u[3];
             double2 gout[4], GN[4], gdir[4];
-            const bool hit = remap_now && remap_hit(remap_qt, a.remap_thr, skx0[mb], ky);
-            for (int f = 0; f < 4; ++f) gout[f] = hit ? make_double2(0.0, 0.0) : Gu[f * NZD];
-            // the step's driving noise (ql_noise.hpp) is state independent; its
-            // ux and bx multipliers sqrt(nf lap2 / lapF) depend on q through
-            // lapF = -kx(t)^2 + lap2, d/dq = mult kx t ky / lapF (ky = 0 modes:
-            // none); the band mask is held fixed like the remap decision
-            if (a.noise && a.s == 3 && !hit && a.np.sigma != 0.0 && ky != 0.0) {
-                const NoiseParams &np = a.np;
-                const double tn = a.t_step;
-                const double kxn = rn_add(skx0[mb], rn_mul(rn_mul(q, tn), ky));
-                const double lap2n = rn_add(rn_mul(-ky, ky), kz2);
-                const double lapF = rn_add(rn_mul(-kxn, kxn), lap2n);
-                if (lapF > -np.hi2 && lapF < -np.lo2) {
-                    const double nf = rn_mul(a.dt_step, np.nfac);
-                    const double mu = sqrt(rn_mul(nf, lap2n) / lapF);
-                    double2 z[4];
-                    noise_normals(np.seed, tn, i, m, z);
-                    double gz = 0.0;
-                    if (np.drive_u) gz += redot(z[0], gout[0]);
-                    if (np.drive_b) gz += redot(z[2], gout[2]);
-                    gq += mu * kxn * (tn * ky) / lapF * np.sigma * gz;
+            const bool hit = remap_now && remap_hit(remap_qt, a.remap_thr, kx0, ky);
+#pragma unroll
+            for (int f = 0; f < 4; ++f) gout[f] = hit ? make_double2(0.0, 0.0) : a.gu[off + f * NZD];
+            if (a.noise && a.s == 3 && !hit && a.np.sigma != 0.0 && ky != 0.0)
+                gq += noise_q_gradient(a.np, q, a.t_step, a.dt_step, kx0, ky, kz2, i, im, gout[0], gout[2]);
+            const double kxn = kx + qdtl * ky;
+            const double xn = (-kxn * kxn - ky * ky) + kz2;
+            double xo = 0.0, dxo_dq = 0.0, kxo_e = 0.0;
+            const double kxo = rn_add(kx0, rn_mul(qt_old, ky));
+            if constexpr (MODE == MODE_CN) {
+                if (a.oinit) {
+                    xo = -kxo * kxo + lap2;
+                    kxo_e = kxo;
+                    dxo_dq = a.tso * ky;
+                } else {
+                    kxo_e = kxo + qdtl_old * ky;
+                    xo = (-kxo_e * kxo_e - ky * ky) + kz2;
+                    dxo_dq = (a.tso + a.dtlo) * ky;
                 }
             }
-            const size_t off = (size_t)i * 4 * NZD + m;
+#pragma unroll
             for (int pr = 0; pr < 2; ++pr) {
                 const double coef = pr == 0 ? ph.nu : ph.eta;
-                const double kxn = kx + qdtl * ky;
-                const double xn = (-kxn * kxn - ky * ky) + kz2;
                 const double Ln = P::lin(pr, kxn, ky, kz2, ph);
-                double gLn = 0.0, gLo = 0.0, xo = 0.0, dxo_dq = 0.0, kxo_e = 0.0;
+                double gLn = 0.0, gLo = 0.0;
+                // factors of the update and of the two right-hand sides in it
+                double e, d = 1.0;
+                if constexpr (MODE == MODE_ELIN) {
+                    e = exp(a.linC * Ln);
+                } else {
+                    const double Lo = a.oinit ? P::lin_init(pr, kxo, lap2, ph) : P::lin(pr, kxo_e, ky, kz2, ph);
+                    d = 1.0 / (1.0 - a.linC * Ln);
+                    e = (1 + a.linC * Lo) * d;
+                }
+#pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const int f = 2 * pr + h;
                     const double2 go = gout[f];
                     const double2 gin = (a.s < 3) ? a.gnp[off + f * NZD] : make_double2(0.0, 0.0);
                     const double2 uo = a.u_out[off + f * NZD];
-                    if (a.mode == MODE_ELIN) {
-                        const double e = exp(a.linC * Ln);
+                    if constexpr (MODE == MODE_ELIN) {
                         const double2 mu = cscale(e, go);
                         GN[f] = cadd(cscale(a.nlc1, mu), gin);
                         if (a.s > 1) a.gnp[off + f * NZD] = cscale(a.nlc2, mu);
                         gdir[f] = mu;
                         gLn += a.linC * redot(uo, go);
                     } else {
-                        double Lo;
-                        const double kxo = rn_add(skx0[mb], rn_mul(qt_old, ky));
-                        if (a.oinit) {
-                            const double lap2 = (ky == 0.0 && m == 0) ? 0.0 : (-ky * ky + kz2);
-                            xo = -kxo * kxo + lap2;
-                            kxo_e = kxo;
-                            dxo_dq = a.tso * ky;
-                            Lo = P::lin_init(pr, kxo, lap2, ph);
-                        } else {
-                            kxo_e = kxo + qdtl_old * ky;
-                            xo = (-kxo_e * kxo_e - ky * ky) + kz2;
-                            dxo_dq = (a.tso + a.dtlo) * ky;
-                            Lo = P::lin(pr, kxo_e, ky, kz2, ph);
-                        }
-                        const double d = 1.0 / (1.0 - a.linC * Ln);
                         GN[f] = cadd(cscale(a.nlc1 * d, go), gin);
                         if (a.s > 1) a.gnp[off + f * NZD] = cscale(a.nlc2 * d, go);
-                        gdir[f] = cscale((1 + a.linC * Lo) * d, go);
+                        gdir[f] = cscale(e, go);
                         gLn += a.linC * d * redot(uo, go);
-                        gLo += a.linC * d * redot(U[f * NZD], go);
+                        gLo += a.linC * d * redot(u[f], go);
                     }
                 }
                 // L = coef * op(x): coefficient and kx(t) = kx0 + q t ky dependence
-                const double gc = gLn * opv(xn) + (a.mode == MODE_CN ? gLo * opv(xo) : 0.0);
+                const double gc = gLn * opv(xn) + (MODE == MODE_CN ? gLo * opv(xo) : 0.0);
                 if (pr == 0) gnu += gc;
                 else geta += gc;
                 gq += gLn * coef * opd(xn) * (-2.0 * kxn) * ((a.ts + a.dtl) * ky);
-                if (a.mode == MODE_CN) gq += gLo * coef * opd(xo) * (-2.0 * kxo_e) * dxo_dq;
+                if (MODE == MODE_CN) gq += gLo * coef * opd(xo) * (-2.0 * kxo_e) * dxo_dq;
             }
+            const double ilapF = (i == 0 && im == 0) ? 1.0 : 1.0 / (-kx * kx + lap2);
             if constexpr (!BQ) {
                 // RHS assembly in reverse (MHD_FullQlin.cpp:283-285, :303-305)
-                const double2 *Tm = bufT + mb * P::NOUT * NZ + D::pad(m);
-                const double2 T1 = Tm[0], T2 = Tm[NZ], T3 = Tm[2 * NZ];
-                const double ilapF = silF[k];
+                const double2 T1 = GT[0], T2 = GT[MB * NZDP], T3 = GT[2 * MB * NZDP];
                 double gkx = 0.0;
                 // N_ux = ilapF s + i B0z kz bx - T1,  s = 2 kx ky q ux + i 2 Om kz ze - kx^2 T1 - kx ky T2 - kx kz T3
                 double2 s = cscale(2.0 * kx * ky * q, ux);
@@ -305,7 +337,7 @@ __global__ __launch_bounds__(NT) void k_adj_mode(AdjModeArgs a)
                     dsk = csub(dsk, cscale(kz, T3));
                     gkx += redot(dsk, Gs);
                 }
-                if (!(i == 0 && m == 0)) gkx += redot(s, GN[0]) * 2.0 * kx * ilapF * ilapF;
+                if (!(i == 0 && im == 0)) gkx += redot(s, GN[0]) * 2.0 * kx * ilapF * ilapF;
                 gq += redot(cscale(2.0 * kx * ky, ux), Gs);
                 gom += redot(imul(2.0 * kz, ze), Gs);
                 gb0 += redot(imul(kz, bx), GN[0]);
@@ -319,36 +351,31 @@ __global__ __launch_bounds__(NT) void k_adj_mode(AdjModeArgs a)
                 gb0 += redot(imul(kz, et), GN[1]);
                 // N_bx = i B0z kz ux - T4
                 gdir[0] = cadd(gdir[0], imul(-B0z * kz, GN[2]));
-                const double2 GT3 = cscale(-1.0, GN[2]);
                 gb0 += redot(imul(kz, ux), GN[2]);
                 // N_et = -i q kz bx + i B0z kz ze - i kz T5 + i ky T6
                 gdir[2] = cadd(gdir[2], imul(q * kz, GN[3]));
                 gdir[1] = cadd(gdir[1], imul(-B0z * kz, GN[3]));
-                const double2 GT4 = imul(kz, GN[3]);
-                const double2 GT5 = imul(-ky, GN[3]);
                 gq += redot(imul(-kz, bx), GN[3]);
                 gb0 += redot(imul(kz, ze), GN[3]);
                 gq += gkx * (a.ts * ky);
                 GT[0] = GT0;
-                GT[NZD] = GT1;
-                GT[2 * NZD] = GT2;
-                GT[3 * NZD] = GT3;
-                GT[4 * NZD] = GT4;
-                GT[5 * NZD] = GT5;
+                GT[MB * NZDP] = GT1;
+                GT[2 * MB * NZDP] = GT2;
+                GT[3 * MB * NZDP] = cscale(-1.0, GN[2]);
+                GT[4 * MB * NZDP] = imul(kz, GN[3]);
+                GT[5 * MB * NZDP] = imul(-ky, GN[3]);
             } else {
                 // MHD_BQlin.cpp:160-162, :177-178, :185, :200-201 in reverse:
                 // N_ux = T1 + ilapF (s + T2), s = 2 kx ky q ux + i 2 Om kz ze;
                 // N_ze = T4 + i (q - 2 Om) kz ux; N_bx = T3; N_et = T5 - i q kz bx
-                const double2 *Tm = bufT + mb * P::NOUT * NZ + D::pad(m);
-                const double2 T2 = Tm[NZ];
-                const double ilapF = silF[k];
+                const double2 T2 = GT[0];  // the only line transformed
                 double gkx = 0.0;
                 const double2 s = cadd(cscale(2.0 * kx * ky * q, ux), imul(2.0 * Om * kz, ze));
                 const double2 Gs = cscale(ilapF, GN[0]);
                 gdir[0] = cadd(gdir[0], cscale(2.0 * kx * ky * q, Gs));
                 gdir[1] = cadd(gdir[1], imul(-2.0 * Om * kz, Gs));
                 gkx += redot(cscale(2.0 * ky * q, ux), Gs);
-                if (!(i == 0 && m == 0)) gkx += redot(cadd(s, T2), GN[0]) * 2.0 * kx * ilapF * ilapF;
+                if (!(i == 0 && im == 0)) gkx += redot(cadd(s, T2), GN[0]) * 2.0 * kx * ilapF * ilapF;
                 gq += redot(cscale(2.0 * kx * ky, ux), Gs);
                 gom += redot(imul(2.0 * kz, ze), Gs);
                 gdir[0] = cadd(gdir[0], imul(-(q - 2.0 * Om) * kz, GN[1]));
@@ -358,279 +385,198 @@ __global__ __launch_bounds__(NT) void k_adj_mode(AdjModeArgs a)
                 gq += redot(imul(-kz, bx), GN[3]);
                 gq += gkx * (a.ts * ky);
                 GT[0] = GN[0];
-                GT[NZD] = Gs;
-                GT[2 * NZD] = GN[2];
-                GT[3 * NZD] = GN[1];
-                GT[4 * NZD] = GN[3];
+                GT[MB * NZDP] = Gs;
+                GT[2 * MB * NZDP] = GN[2];
+                GT[3 * MB * NZDP] = GN[1];
+                GT[4 * MB * NZDP] = GN[3];
             }
-            for (int f = 0; f < 4; ++f) Gu[f * NZD] = gdir[f];
+            // the direct terms wait in the gradient itself for J
+#pragma unroll
+            for (int f = 0; f < 4; ++f) a.gu[off + f * NZD] = gdir[f];
         }
         __syncthreads();
 
         // G: adjoint of the forward transforms = padded inverse transforms
-        fft_lines_from<NZ, NLT, true>(bufT, tw, CompactSrc<NZ>{sbase});
+        adj_inv<NZ, NLG, LS, NZDP>(bufT, tw);
 
-        // H: products and EMF / stress terms in reverse, per (mode, half, z):
-        // half 0 owns the u lines (ux uy uz), half 1 the b lines (bx by bz)
-        double2 gX[HW][GL];
+        // H: products and EMF / stress terms in reverse, per (mode, z); the X
+        // lines of the thread's z point become their gradients
+        double2 gdz = make_double2(0.0, 0.0);
+        if (!zok) {
 #pragma unroll
-        for (int p = 0; p < HW; ++p) {
-            const int item = tid + p * NT;
-            if (HI % NT != 0 && item >= HI) continue;
-            const int mb = item / (2 * NZ), rem = item % (2 * NZ);
-            const int h = rem / NZ, z = rem % NZ;
-#pragma unroll
-            for (int c = 0; c < GL; ++c) gX[p][c] = make_double2(0.0, 0.0);
-            if (BQ && h == 0) gdzz[mb * NZ + z] = make_double2(0.0, 0.0);
-            if (sidx[mb] < 0) continue;
-            if constexpr (BQ) {
-                // MHD_BQlin products (MHD_BQlin.cpp:153-201, :219-240) in reverse;
-                // X lines ux ze bx et uy uz by bz, P lines: By i ky bx,
-                // dzBy 2 kx ky bz, By i ky ux, (zeta), (eta)
-                const double2 *X = bufX + mb * P::NLINE * NZ + z;
-                const double2 ux = X[0], ze = X[NZ], bx = X[2 * NZ], et = X[3 * NZ];
-                const double2 uy = X[4 * NZ], uz = X[5 * NZ], by = X[6 * NZ], bz = X[7 * NZ];
-                const double2 *GPp = bufT + mb * P::NOUT * NZ + z;
-                const double2 G0 = GPp[0], G1 = GPp[NZ], G2 = GPp[2 * NZ], G3 = GPp[3 * NZ], G4 = GPp[4 * NZ];
-                const double *mf = smfz + z * 8;
-                const double By = mf[0], dzBy = mf[1], dzdzBy = mf[2];
-                const double kx = skx[mb], ky = sky[mb];
-                const double ftfac = (ky == 0.0 ? 1.0 : 2.0) * a.rsf;
-                const double g0 = ftfac * sgs[z], g1 = ftfac * sgs[NZ + z];  // EMF x, EMF y
-                double gkx = 0.0;
-                if (h == 0) {
-                    // ux, ze, uy, uz; dz uz = -i kx ux - i ky uy + dzc enters the
-                    // eta product as dzBy (-2 dz uz - i kx ux)
-                    const double2 dzuz = cadd(cadd(imul(-kx, ux), imul(-ky, uy)), imul(kx, sdz[mb]));
-                    const double2 t2 = csub(cscale(-2.0, dzuz), imul(kx, ux));
-                    gX[p][0] = cadd(cadd(imul(-ky * By, G2), imul(-kx * dzBy, G4)), cscale(g0, bz));
-                    gX[p][1] = imul(-ky * By, G4);
-                    gX[p][2] = cadd(imul(-2.0 * ky * dzBy, G4), cscale(g1, bz));
-                    gX[p][3] = csub(cscale(-dzdzBy, G4), cadd(cscale(g0, bx), cscale(g1, by)));
-                    gdzz[mb * NZ + z] = cscale(-2.0 * dzBy, G4);
-                    accm[p][0] += redot(imul(ky, ux), G2) + redot(imul(ky, ze), G4);
-                    accm[p][1] += redot(t2, G4);
-                    accm[p][2] -= redot(uz, G4);
-                    gkx += redot(imul(dzBy, ux), G4);
-                } else {
-                    // bx, et, by, bz
-                    gX[p][0] = csub(cadd(imul(-ky * By, G0), imul(kx * dzBy, G3)), cscale(g0, uz));
-                    gX[p][1] = imul(-ky * By, G3);
-                    gX[p][2] = cscale(-g1, uz);
-                    gX[p][3] = cadd(cadd(cscale(2.0 * kx * ky * dzBy, G1), cscale(dzdzBy, G3)),
-                                    cadd(cscale(g0, ux), cscale(g1, uy)));
-                    accm[p][0] += redot(imul(ky, bx), G0) + redot(imul(ky, et), G3);
-                    accm[p][1] += redot(cscale(2.0 * kx * ky, bz), G1) + redot(imul(-kx, bx), G3);
-                    accm[p][2] += redot(bz, G3);
-                    gkx += redot(cscale(2.0 * ky * dzBy, bz), G1) + redot(imul(-dzBy, bx), G3);
-                }
-                gq += gkx * (a.ts * ky);
-                continue;
-            }
-            const double2 *X = bufX + mb * P::NLINE * NZ + z;
-            const double2 u0 = X[0], u1 = X[NZ], u2 = X[2 * NZ], b0 = X[3 * NZ], b1 = X[4 * NZ], b2 = X[5 * NZ];
-            const double2 *GPp = bufT + mb * P::NOUT * NZ + z;
-            const double2 G0 = GPp[0], G1 = GPp[NZ], G2 = GPp[2 * NZ], G3 = GPp[3 * NZ], G4 = GPp[4 * NZ],
-                          G5 = GPp[5 * NZ];
-            const double *mf = smfz + z * 8;
-            const double MBx = mf[0], dzMBx = mf[1], MBy = mf[2], dzMBy = mf[3];
-            const double MUx = mf[4], dzMUx = mf[5], MUy = mf[6], dzMUy = mf[7];
-            const double kx = skx[mb], ky = sky[mb];
-            const double aU = kx * MUx + ky * MUy, aB = kx * MBx + ky * MBy;
-            const double ftfac = (ky == 0.0 ? 1.0 : 2.0) * a.rsf;
-            const double g0 = ftfac * sgs[z], g1 = ftfac * sgs[NZ + z], g2 = ftfac * sgs[2 * NZ + z],
-                         g3 = ftfac * sgs[3 * NZ + z];
+            for (int l = 0; l < P::NLINE; ++l) X[l * MB * LS] = make_double2(0.0, 0.0);
+        } else if constexpr (BQ) {
+            // MHD_BQlin products (MHD_BQlin.cpp:153-201, :219-240) in reverse;
+            // X lines ux ze bx et uy uz by bz, P lines: By i ky bx,
+            // dzBy 2 kx ky bz, By i ky ux, (zeta), (eta)
+            const double2 ux = X[0], ze = X[MB * LS], bx = X[2 * MB * LS], et = X[3 * MB * LS];
+            const double2 uy = X[4 * MB * LS], uz = X[5 * MB * LS], by = X[6 * MB * LS], bz = X[7 * MB * LS];
+            const double2 G0 = Y[0], G1 = Y[MB * LS], G2 = Y[2 * MB * LS], G3 = Y[3 * MB * LS], G4 = Y[4 * MB * LS];
+            const double By = smfz[zz], dzBy = smfz[NZ + zz], dzdzBy = smfz[2 * NZ + zz];
+            const double ftfac = (zky == 0.0 ? 1.0 : 2.0) * a.rsf;
+            const double g0 = ftfac * sgs[zz], g1 = ftfac * sgs[NZ + zz];  // EMF x, EMF y
             double gkx = 0.0;
-            if (h == 0) {
-                // u0 (0), u1 (1), u2 (2)
-                double2 Gu0 = cadd(imul(-aU, G0), imul(aB, G3));
-                double2 Gu1 = cadd(imul(-aU, G1), imul(aB, G4));
-                double2 Gu2 = cadd(cadd(cscale(dzMUx, G0), cscale(dzMUy, G1)), imul(-aU, G2));
-                Gu2 = cadd(Gu2, cadd(cadd(cscale(dzMBx, G3), cscale(dzMBy, G4)), imul(aB, G5)));
-                // EMF x, y (slots 0, 1) and stresses (slots 2, 3:
-                // -Re(uz conj(ux)), -Re(uz conj(uy)) before their z-derivative)
-                Gu0 = cadd(Gu0, cscale(g0, b2));
-                Gu2 = csub(Gu2, cadd(cscale(g0, b0), cscale(g1, b1)));
-                Gu1 = cadd(Gu1, cscale(g1, b2));
-                Gu0 = csub(Gu0, cscale(g2, u2));
-                Gu1 = csub(Gu1, cscale(g3, u2));
-                Gu2 = csub(Gu2, cadd(cscale(g2, u0), cscale(g3, u1)));
-                gX[p][0] = Gu0;
-                gX[p][1] = Gu1;
-                gX[p][2] = Gu2;
-                // mean-field profile and kx gradients from the first three products
-                const double gaU = redot(imul(1.0, u0), G0) + redot(imul(1.0, u1), G1) + redot(imul(1.0, u2), G2);
-                const double gaB = redot(imul(-1.0, b0), G0) + redot(imul(-1.0, b1), G1) + redot(imul(-1.0, b2), G2);
-                accm[p][5] += redot(u2, G0);   // dz MUx
-                accm[p][1] -= redot(b2, G0);   // dz MBx
-                accm[p][7] += redot(u2, G1);   // dz MUy
-                accm[p][3] -= redot(b2, G1);   // dz MBy
-                accm[p][4] += kx * gaU;
-                accm[p][6] += ky * gaU;
-                accm[p][0] += kx * gaB;
-                accm[p][2] += ky * gaB;
-                gkx += MUx * gaU + MBx * gaB;
-            } else {
-                // b0 (0), b1 (1), b2 (2)
-                double2 Gb0 = cadd(imul(aB, G0), imul(-aU, G3));
-                double2 Gb1 = cadd(imul(aB, G1), imul(-aU, G4));
-                double2 Gb2 = cadd(cadd(cscale(-dzMBx, G0), cscale(-dzMBy, G1)), imul(aB, G2));
-                Gb2 = cadd(Gb2, cadd(cadd(cscale(-dzMUx, G3), cscale(-dzMUy, G4)), imul(-aU, G5)));
-                Gb2 = cadd(Gb2, cadd(cscale(g0, u0), cscale(g1, u1)));
-                Gb0 = csub(Gb0, cscale(g0, u2));
-                Gb1 = csub(Gb1, cscale(g1, u2));
-                // stresses: +Re(bz conj(bx)), +Re(bz conj(by))
-                Gb0 = cadd(Gb0, cscale(g2, b2));
-                Gb1 = cadd(Gb1, cscale(g3, b2));
-                Gb2 = cadd(Gb2, cadd(cscale(g2, b0), cscale(g3, b1)));
-                gX[p][0] = Gb0;
-                gX[p][1] = Gb1;
-                gX[p][2] = Gb2;
-                const double gaU = redot(imul(1.0, b0), G3) + redot(imul(1.0, b1), G4) + redot(imul(1.0, b2), G5);
-                const double gaB = redot(imul(-1.0, u0), G3) + redot(imul(-1.0, u1), G4) + redot(imul(-1.0, u2), G5);
-                accm[p][1] += redot(u2, G3);   // dz MBx
-                accm[p][5] -= redot(b2, G3);   // dz MUx
-                accm[p][3] += redot(u2, G4);   // dz MBy
-                accm[p][7] -= redot(b2, G4);   // dz MUy
-                accm[p][4] += kx * gaU;
-                accm[p][6] += ky * gaU;
-                accm[p][0] += kx * gaB;
-                accm[p][2] += ky * gaB;
-                gkx += MUx * gaU + MBx * gaB;
-            }
-            gq += gkx * (a.ts * ky);
+            // ux, ze, uy, uz; dz uz = -i kx ux - i ky uy + dzc enters the
+            // eta product as dzBy (-2 dz uz - i kx ux)
+            const double2 dzuz = cadd(cadd(imul(-zkx, ux), imul(-zky, uy)), imul(zkx, sdz[zmb]));
+            const double2 t2 = csub(cscale(-2.0, dzuz), imul(zkx, ux));
+            X[0] = cadd(cadd(imul(-zky * By, G2), imul(-zkx * dzBy, G4)), cscale(g0, bz));
+            X[MB * LS] = imul(-zky * By, G4);
+            X[4 * MB * LS] = cadd(imul(-2.0 * zky * dzBy, G4), cscale(g1, bz));
+            X[5 * MB * LS] = csub(cscale(-dzdzBy, G4), cadd(cscale(g0, bx), cscale(g1, by)));
+            gdz = cscale(-2.0 * dzBy, G4);
+            accm[0] += redot(imul(zky, ux), G2) + redot(imul(zky, ze), G4);
+            accm[1] += redot(t2, G4);
+            accm[2] -= redot(uz, G4);
+            gkx += redot(imul(dzBy, ux), G4);
+            // bx, et, by, bz
+            X[2 * MB * LS] = csub(cadd(imul(-zky * By, G0), imul(zkx * dzBy, G3)), cscale(g0, uz));
+            X[3 * MB * LS] = imul(-zky * By, G3);
+            X[6 * MB * LS] = cscale(-g1, uz);
+            X[7 * MB * LS] = cadd(cadd(cscale(2.0 * zkx * zky * dzBy, G1), cscale(dzdzBy, G3)),
+                                  cadd(cscale(g0, ux), cscale(g1, uy)));
+            accm[0] += redot(imul(zky, bx), G0) + redot(imul(zky, et), G3);
+            accm[1] += redot(cscale(2.0 * zkx * zky, bz), G1) + redot(imul(-zkx, bx), G3);
+            accm[2] += redot(bz, G3);
+            gkx += redot(cscale(2.0 * zky * dzBy, bz), G1) + redot(imul(-dzBy, bx), G3);
+            gq += gkx * (a.ts * zky);
+        } else {
+            const double2 u0 = X[0], u1 = X[MB * LS], u2 = X[2 * MB * LS];
+            const double2 b0 = X[3 * MB * LS], b1 = X[4 * MB * LS], b2 = X[5 * MB * LS];
+            const double2 G0 = Y[0], G1 = Y[MB * LS], G2 = Y[2 * MB * LS];
+            const double2 G3 = Y[3 * MB * LS], G4 = Y[4 * MB * LS], G5 = Y[5 * MB * LS];
+            const double *mf = smfz + zz;
+            const double MBx = mf[0], dzMBx = mf[NZ], MBy = mf[2 * NZ], dzMBy = mf[3 * NZ];
+            const double MUx = mf[4 * NZ], dzMUx = mf[5 * NZ], MUy = mf[6 * NZ], dzMUy = mf[7 * NZ];
+            const double aU = zkx * MUx + zky * MUy, aB = zkx * MBx + zky * MBy;
+            const double ftfac = (zky == 0.0 ? 1.0 : 2.0) * a.rsf;
+            const double g0 = ftfac * sgs[zz], g1 = ftfac * sgs[NZ + zz], g2 = ftfac * sgs[2 * NZ + zz],
+                         g3 = ftfac * sgs[3 * NZ + zz];
+            // u0 (0), u1 (1), u2 (2)
+            double2 Gu0 = cadd(imul(-aU, G0), imul(aB, G3));
+            double2 Gu1 = cadd(imul(-aU, G1), imul(aB, G4));
+            double2 Gu2 = cadd(cadd(cscale(dzMUx, G0), cscale(dzMUy, G1)), imul(-aU, G2));
+            Gu2 = cadd(Gu2, cadd(cadd(cscale(dzMBx, G3), cscale(dzMBy, G4)), imul(aB, G5)));
+            // EMF x, y (slots 0, 1) and stresses (slots 2, 3:
+            // -Re(uz conj(ux)), -Re(uz conj(uy)) before their z-derivative)
+            Gu0 = cadd(Gu0, cscale(g0, b2));
+            Gu2 = csub(Gu2, cadd(cscale(g0, b0), cscale(g1, b1)));
+            Gu1 = cadd(Gu1, cscale(g1, b2));
+            Gu0 = csub(Gu0, cscale(g2, u2));
+            Gu1 = csub(Gu1, cscale(g3, u2));
+            Gu2 = csub(Gu2, cadd(cscale(g2, u0), cscale(g3, u1)));
+            X[0] = Gu0;
+            X[MB * LS] = Gu1;
+            X[2 * MB * LS] = Gu2;
+            // b0 (0), b1 (1), b2 (2)
+            double2 Gb0 = cadd(imul(aB, G0), imul(-aU, G3));
+            double2 Gb1 = cadd(imul(aB, G1), imul(-aU, G4));
+            double2 Gb2 = cadd(cadd(cscale(-dzMBx, G0), cscale(-dzMBy, G1)), imul(aB, G2));
+            Gb2 = cadd(Gb2, cadd(cadd(cscale(-dzMUx, G3), cscale(-dzMUy, G4)), imul(-aU, G5)));
+            Gb2 = cadd(Gb2, cadd(cscale(g0, u0), cscale(g1, u1)));
+            Gb0 = csub(Gb0, cscale(g0, u2));
+            Gb1 = csub(Gb1, cscale(g1, u2));
+            // stresses: +Re(bz conj(bx)), +Re(bz conj(by))
+            Gb0 = cadd(Gb0, cscale(g2, b2));
+            Gb1 = cadd(Gb1, cscale(g3, b2));
+            Gb2 = cadd(Gb2, cadd(cscale(g2, b0), cscale(g3, b1)));
+            X[3 * MB * LS] = Gb0;
+            X[4 * MB * LS] = Gb1;
+            X[5 * MB * LS] = Gb2;
+            // mean-field profile and kx gradients: the momentum products, then
+            // the induction products
+            double gaU = redot(imul(1.0, u0), G0) + redot(imul(1.0, u1), G1) + redot(imul(1.0, u2), G2);
+            double gaB = redot(imul(-1.0, b0), G0) + redot(imul(-1.0, b1), G1) + redot(imul(-1.0, b2), G2);
+            gaU += redot(imul(1.0, b0), G3) + redot(imul(1.0, b1), G4) + redot(imul(1.0, b2), G5);
+            gaB += redot(imul(-1.0, u0), G3) + redot(imul(-1.0, u1), G4) + redot(imul(-1.0, u2), G5);
+            accm[0] += zkx * gaB;
+            accm[1] += redot(u2, G3) - redot(b2, G0);  // dz MBx
+            accm[2] += zky * gaB;
+            accm[3] += redot(u2, G4) - redot(b2, G1);  // dz MBy
+            accm[4] += zkx * gaU;
+            accm[5] += redot(u2, G0) - redot(b2, G3);  // dz MUx
+            accm[6] += zky * gaU;
+            accm[7] += redot(u2, G1) - redot(b2, G4);  // dz MUy
+            gq += (MUx * gaU + MBx * gaB) * (a.ts * zky);
         }
-        __syncthreads();
+        if constexpr (BQ) {
+            // the dz uz constant's gradient summed over z: within a wavefront
+            // here, over a mode's wavefronts by its reader in J
 #pragma unroll
-        for (int p = 0; p < HW; ++p) {
-            const int item = tid + p * NT;
-            if (HI % NT != 0 && item >= HI) continue;
-            const int mb = item / (2 * NZ), rem = item % (2 * NZ);
-            const int h = rem / NZ, z = rem % NZ;
-            double2 *Y = bufX + mb * P::NLINE * NZ + z;
-            if constexpr (BQ) {
-                // lines: ux ze bx et uy uz by bz; half 0 the u side, half 1 the b side
-                const int l0 = h ? 2 : 0;
-                Y[l0 * NZ] = gX[p][0];
-                Y[(l0 + 1) * NZ] = gX[p][1];
-                Y[(l0 + 4) * NZ] = gX[p][2];
-                Y[(l0 + 5) * NZ] = gX[p][3];
-            } else {
-                // lines: u0 u1 u2 b0 b1 b2
-                const int l0 = h ? 3 : 0;
-                Y[l0 * NZ] = gX[p][0];
-                Y[(l0 + 1) * NZ] = gX[p][1];
-                Y[(l0 + 2) * NZ] = gX[p][2];
-            }
-        }
-        // ModelBQ: the dz uz constant's gradient of each mode, summed over z
-        // in order
-        if (BQ && tid < MB) {
-            double2 sg = make_double2(0.0, 0.0);
-            for (int z = 0; z < NZ; ++z) sg = cadd(sg, gdzz[tid * NZ + z]);
-            sgdz[tid] = sg;
+            for (int o = SEG / 2; o > 0; o >>= 1)
+                gdz = cadd(gdz, make_double2(__shfl_xor(gdz.x, o), __shfl_xor(gdz.y, o)));
+            if (tid % SEG == 0) sgdz[tid / SEG] = gdz;
         }
         __syncthreads();
 
         // I: adjoint of the padded inverse transforms = truncated forward transforms
-        fft_lines<NZ, NLX, false>(bufX, tw);
+        adj_fwd<NZ, NLX, LS, NZDP>(bufX, tw);
 
         // J: base fields in reverse; total dL/du_in
-        for (int k = tid; k < MB * NZD; k += NT) {
-            const int mb = k / NZD, m = k % NZD;
-            const int i = sidx[mb];
-            if (i < 0) continue;
-            const double kx = skx[mb], ky = sky[mb], kz = skz[m];
-            const bool zero = (ky == 0.0 && m == 0);
-            const double ilap2 = zero ? 1.0 : 1.0 / (-ky * ky + -(kz * kz));
-            if constexpr (!BQ) {
-                const double2 *GL = bufX + mb * P::NLINE * NZ + D::pad(m);
-                const double2 GB0 = GL[0], GB1 = GL[NZ], GB2 = GL[2 * NZ];
-                const double2 GB3 = GL[3 * NZ], GB4 = GL[4 * NZ], GB5 = GL[5 * NZ];
-                const double2 *U = uin + mb * 4 * NZD + m;
-                const double2 ux = U[0], bx = U[2 * NZD];
-                const double f = a.fac;
-                double2 *Gu = sgu + mb * 4 * NZD + m;
-                // uy = (ky kx ux + i kz ze) ilap2, uz = (kx kz ux - i ky ze) ilap2 (and b likewise)
-                const double2 Gux = cscale(f, cadd(GB0, cadd(cscale(ky * kx * ilap2, GB1), cscale(kx * kz * ilap2, GB2))));
-                const double2 Gze = cscale(f, cadd(imul(-kz * ilap2, GB1), imul(ky * ilap2, GB2)));
-                const double2 Gbx = cscale(f, cadd(GB3, cadd(cscale(ky * kx * ilap2, GB4), cscale(kx * kz * ilap2, GB5))));
-                const double2 Get = cscale(f, cadd(imul(-kz * ilap2, GB4), imul(ky * ilap2, GB5)));
-                const double gkx = f * (redot(cscale(ky * ilap2, ux), GB1) + redot(cscale(kz * ilap2, ux), GB2) +
-                                        redot(cscale(ky * ilap2, bx), GB4) + redot(cscale(kz * ilap2, bx), GB5));
-                gq += gkx * (a.ts * ky);
-                const size_t off = (size_t)i * 4 * NZD + m;
-                a.gu[off] = cadd(Gu[0], Gux);
-                a.gu[off + NZD] = cadd(Gu[NZD], Gze);
-                a.gu[off + 2 * NZD] = cadd(Gu[2 * NZD], Gbx);
-                a.gu[off + 3 * NZD] = cadd(Gu[3 * NZD], Get);
-            } else {
-                // bases ux ze bx et uy uz by bz: uy = (ky kx ux + i kz ze) ilap2,
-                // uz = (kx kz ux - i ky ze) ilap2 (and b likewise), all times fac
-                const double2 *GL = bufX + mb * P::NLINE * NZ + D::pad(m);
-                const double2 GB0 = GL[0], GB1 = GL[NZ], GB2 = GL[2 * NZ], GB3 = GL[3 * NZ];
-                const double2 GB4 = GL[4 * NZ], GB5 = GL[5 * NZ], GB6 = GL[6 * NZ], GB7 = GL[7 * NZ];
-                const double2 *U = uin + mb * 4 * NZD + m;
-                const double2 ux = U[0], bx = U[2 * NZD];
-                const double f = a.fac;
-                double2 *Gu = sgu + mb * 4 * NZD + m;
-                double2 Gux = cscale(f, cadd(GB0, cadd(cscale(ky * kx * ilap2, GB4), cscale(kx * kz * ilap2, GB5))));
-                const double2 Gze = cscale(f, cadd(GB1, cadd(imul(-kz * ilap2, GB4), imul(ky * ilap2, GB5))));
-                const double2 Gbx = cscale(f, cadd(GB2, cadd(cscale(ky * kx * ilap2, GB6), cscale(kx * kz * ilap2, GB7))));
-                const double2 Get = cscale(f, cadd(GB3, cadd(imul(-kz * ilap2, GB6), imul(ky * ilap2, GB7))));
-                double gkx = f * (redot(cscale(ky * ilap2, ux), GB4) + redot(cscale(kz * ilap2, ux), GB5) +
-                                  redot(cscale(ky * ilap2, bx), GB6) + redot(cscale(kz * ilap2, bx), GB7));
-                if (zero) {
-                    // dzc = i kx (fac ux at kz = 0) of a ky = 0 mode
-                    const double2 Gd = sgdz[mb];
-                    Gux = cadd(Gux, imul(-kx * f, Gd));
-                    gkx += redot(imul(1.0, sdz[mb]), Gd);
-                }
-                gq += gkx * (a.ts * ky);
-                const size_t off = (size_t)i * 4 * NZD + m;
-                a.gu[off] = cadd(Gu[0], Gux);
-                a.gu[off + NZD] = cadd(Gu[NZD], Gze);
-                a.gu[off + 2 * NZD] = cadd(Gu[2 * NZD], Gbx);
-                a.gu[off + 3 * NZD] = cadd(Gu[3 * NZD], Get);
+        if (i >= 0) {
+            const double2 *GL = bufX + imb * NZDP + im;  // line l at GL[l * MB * NZDP]
+            const double f = a.fac;
+            const double2 ux = a.u_in[off], bx = a.u_in[off + 2 * NZD];
+            // the y, z bases: uy = (ky kx ux + i kz ze) ilap2, uz = (kx kz ux - i ky ze)
+            // ilap2 (and b likewise), all bases times fac
+            const double2 GBx = GL[0], GBy = GL[(BQ ? 4 : 1) * MB * NZDP], GBz = GL[(BQ ? 5 : 2) * MB * NZDP];
+            const double2 Gbx_ = GL[(BQ ? 2 : 3) * MB * NZDP], Gby_ = GL[(BQ ? 6 : 4) * MB * NZDP],
+                          Gbz_ = GL[(BQ ? 7 : 5) * MB * NZDP];
+            const double2 G1z = BQ ? GL[MB * NZDP] : make_double2(0.0, 0.0);      // the zeta base
+            const double2 G3e = BQ ? GL[3 * MB * NZDP] : make_double2(0.0, 0.0);  // the eta base
+            double2 Gux = cscale(f, cadd(GBx, cadd(cscale(ky * kx * ilap2, GBy), cscale(kx * kz * ilap2, GBz))));
+            double2 Gze = cadd(imul(-kz * ilap2, GBy), imul(ky * ilap2, GBz));
+            const double2 Gbx = cscale(f, cadd(Gbx_, cadd(cscale(ky * kx * ilap2, Gby_), cscale(kx * kz * ilap2, Gbz_))));
+            double2 Get = cadd(imul(-kz * ilap2, Gby_), imul(ky * ilap2, Gbz_));
+            if constexpr (BQ) {
+                Gze = cadd(G1z, Gze);
+                Get = cadd(G3e, Get);
             }
+            Gze = cscale(f, Gze);
+            Get = cscale(f, Get);
+            double gkx = f * (redot(cscale(ky * ilap2, ux), GBy) + redot(cscale(kz * ilap2, ux), GBz) +
+                              redot(cscale(ky * ilap2, bx), Gby_) + redot(cscale(kz * ilap2, bx), Gbz_));
+            if (BQ && zero) {
+                // dzc = i kx (fac ux at kz = 0) of a ky = 0 mode
+                double2 Gd = sgdz[imb * (NZ / SEG)];
+#pragma unroll
+                for (int w = 1; w < NZ / SEG; ++w) Gd = cadd(Gd, sgdz[imb * (NZ / SEG) + w]);
+                Gux = cadd(Gux, imul(-kx * f, Gd));
+                gkx += redot(imul(1.0, sdz[imb]), Gd);
+            }
+            gq += gkx * (a.ts * ky);
+            const double2 total[4] = {Gux, Gze, Gbx, Get};
+#pragma unroll
+            for (int fl = 0; fl < 4; ++fl) a.gu[off + fl * NZD] = cadd(a.gu[off + fl * NZD], total[fl]);
         }
         __syncthreads();
     }
 
-    // partial row of this workgroup: z-profile gradients summed over mode slots
-    // and halves in a fixed order, then the parameter gradients
-    // (four profile lines at a time: 2 MB x 4 x NZ doubles fit the X lines)
+    // partial row of this workgroup: the z-profile gradients summed over the
+    // mode slots, then the parameter gradients over the threads, both in a
+    // fixed order
     double *red = reinterpret_cast<double *>(bufX);
-    static_assert(2 * MB * 4 * NZ * sizeof(double) <= sizeof(bufX), "reduction fits the X lines");
+    static_assert((8 * NT + 5 * (NT / 64)) * sizeof(double) <= sizeof(bufX), "reduction fits the X lines");
     double *row = a.gpart + (size_t)blockIdx.x * (8 * NZ + NGP);
 #pragma unroll
-    for (int c0 = 0; c0 < 8; c0 += 4) {
+    for (int c = 0; c < 8; ++c) red[(zmb * 8 + c) * NZ + zz] = accm[c];
+    double gp[5] = {gq, gom, gnu, geta, gb0};
 #pragma unroll
-        for (int p = 0; p < HW; ++p) {
-            const int item = tid + p * NT;
-            if (HI % NT != 0 && item >= HI) continue;
-            const int mbh = item / NZ, z = item % NZ;  // (mode slot, half) pair, z
-#pragma unroll
-            for (int c = 0; c < 4; ++c) red[(mbh * 4 + c) * NZ + z] = accm[p][c0 + c];
-        }
-        __syncthreads();
-        for (int k = tid; k < 4 * NZ; k += NT) {
-            double s = 0.0;
-            for (int mbh = 0; mbh < 2 * MB; ++mbh) s += red[mbh * 4 * NZ + k];
-            row[c0 * NZ + k] = s;
-        }
-        __syncthreads();
+    for (int c = 0; c < 5; ++c) {
+        const double t = wave_sum(gp[c]);
+        if (tid % 64 == 0) red[8 * NT + c * (NT / 64) + tid / 64] = t;
     }
-    red[0 * NT + tid] = gq;
-    red[1 * NT + tid] = gom;
-    red[2 * NT + tid] = gnu;
-    red[3 * NT + tid] = geta;
-    red[4 * NT + tid] = gb0;
     __syncthreads();
+    for (int k = tid; k < 8 * NZ; k += NT) {
+        double s = 0.0;
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) s += red[mb * 8 * NZ + k];
+        row[k] = s;
+    }
     if (tid < NGP) {
         double s = 0.0;
         if (tid < 5)
-            for (int k = 0; k < NT; ++k) s += red[tid * NT + k];
+            for (int w = 0; w < NT / 64; ++w) s += red[8 * NT + tid * (NT / 64) + w];
         row[8 * NZ + tid] = s;
     }
 }
