@@ -5,9 +5,9 @@
 // ql_adjoint_forward runs the steps exactly as ql_steps does (the same kernels
 // and launch shape, so the same bits) and stores the state every `every`
 // steps.  ql_adjoint_backward walks the segments backwards: it restores a
-// checkpoint, recomputes the segment's substeps eagerly while keeping every
-// substep state (3 every + 1 states), then runs the reverse substeps
-// (ql_adjoint.hpp) from the last to the first.  It returns dL/d(state at the
+// checkpoint, recomputes the segment's substeps eagerly, each writing its state,
+// mean fields and profiles to buffers of its own (3 every + 1 states), then runs
+// the reverse substeps (ql_adjoint.hpp) from the last to the first.  It returns dL/d(state at the
 // start of the forward) and dL/d(q, omega, nu, eta, B0z) for the caller's
 // dL/d(final state); the context is left at the final state of the forward.
 #include <algorithm>
@@ -19,10 +19,13 @@
 
 namespace qlh {
 
+// Everything one context's gradients need.  It stays with the context, so that
+// a loop of gradients allocates once; a forward with other steps or spacing
+// gives back what no longer fits (adj_fit).
 struct AdjState {
+    bool valid = false;  // a forward has completed
     int nsteps = 0, every = 0, nseg = 0;
     bool noise = false;  // the forward was driven
-    double t_end = 0.0;
     // checkpoints at segment starts (index nseg: the final state); with
     // variable steps also the step taken last and the profile maxima the next
     // step's dt comes from
@@ -34,26 +37,34 @@ struct AdjState {
     };
     std::vector<Ck> ck;
     double t_init = 0.0;
-    // substep states of one segment; with driving noise also each step's
-    // state after substep 3 before the noise and the remap
+    // substep states, mean fields and profiles of one segment; with driving
+    // noise also each step's state after substep 3 before the noise and the
+    // remap
     double2 *st_u = nullptr, *st_mf = nullptr, *st_pre = nullptr;
-    double *st_kx0 = nullptr;
+    double *st_kx0 = nullptr, *st_mfz = nullptr;
     // adjoint buffers
     double2 *gu = nullptr, *gnp = nullptr, *gM = nullptr, *gnmp = nullptr;
     double *gsums = nullptr, *gpart = nullptr, *grows = nullptr, *gpar_mf = nullptr, *gpar = nullptr;
-    double *mfz = nullptr;
     qlk::RunParams *rp1 = nullptr;  // one run, rows [0, W) (column reduction)
     int W = 0;
 };
+
+namespace {
+void free_ck(AdjState::Ck &c) { dfree(c.u), dfree(c.mf), dfree(c.kx0), dfree(c.pm); }
+void free_segment(AdjState *A)
+{
+    dfree(A->st_u), dfree(A->st_mf), dfree(A->st_kx0), dfree(A->st_pre), dfree(A->st_mfz);
+}
+}  // namespace
 
 void adj_release(Batch &b)
 {
     AdjState *A = b.adj;
     if (!A) return;
-    for (auto &c : A->ck) dfree(c.u), dfree(c.mf), dfree(c.kx0), dfree(c.pm);
-    dfree(A->st_u), dfree(A->st_mf), dfree(A->st_kx0), dfree(A->st_pre);
+    for (auto &c : A->ck) free_ck(c);
+    free_segment(A);
     dfree(A->gu), dfree(A->gnp), dfree(A->gM), dfree(A->gnmp);
-    dfree(A->gsums), dfree(A->gpart), dfree(A->grows), dfree(A->gpar_mf), dfree(A->gpar), dfree(A->mfz);
+    dfree(A->gsums), dfree(A->gpart), dfree(A->grows), dfree(A->gpar_mf), dfree(A->gpar);
     dfree(A->rp1);
     delete A;
     b.adj = nullptr;
@@ -94,18 +105,27 @@ int save_ck(Batch &b, AdjState::Ck &c, double t)
     return QL_OK;
 }
 
-int load_ck(Batch &b, const AdjState::Ck &c)
+// the state and clock history of a checkpoint, the state into u, mf and the
+// profiles mfz
+int load_ck(Batch &b, const AdjState::Ck &c, double2 *u, double2 *mf, double *mfz)
 {
     Group &g = b.groups[0];
     const size_t nl = (size_t)g.modes * 4 * g.nz, nm = (size_t)b.nMF * g.nz;
-    QL_HIP(hipMemcpyAsync(g.u, c.u, sizeof(double2) * nl, hipMemcpyDeviceToDevice, b.s));
-    QL_HIP(hipMemcpyAsync(g.mf, c.mf, sizeof(double2) * nm, hipMemcpyDeviceToDevice, b.s));
+    QL_HIP(hipMemcpyAsync(u, c.u, sizeof(double2) * nl, hipMemcpyDeviceToDevice, b.s));
+    QL_HIP(hipMemcpyAsync(mf, c.mf, sizeof(double2) * nm, hipMemcpyDeviceToDevice, b.s));
     QL_HIP(hipMemcpyAsync(g.kx0, c.kx0, sizeof(double) * g.modes, hipMemcpyDeviceToDevice, b.s));
     QL_HIP(hipMemcpyAsync(g.pm, c.pm, sizeof(double) * qlk::PM_STRIDE, hipMemcpyDeviceToDevice, b.s));
     b.t_prev = c.t_prev;
     b.dt_last = c.dt_last;
     b.old_init = c.old_init;
-    return refresh_profiles(b, g, b.s);
+    qlk::MFArgs m = mf_args(b, g);
+    m.mode = qlk::MODE_PROFILES;
+    m.mf = mf;
+    m.mfz = mfz;
+    m.mfn_out = g.mfN1;
+    launch_mf(g, m, b.s);
+    QL_HIP(hipGetLastError());
+    return QL_OK;
 }
 
 // substep times of the forward (sub_times in ql_kernels.hpp, same roundings);
@@ -143,54 +163,86 @@ HostTimes host_times(double t, double t_prev, int old_init, double t_init, doubl
 }
 
 template <int NZ, int MODEL>
-void launch_adj_nz(const qlk::AdjModeArgs &am, const qlk::AdjMFArgs &aa, const qlk::AdjMF2Args &ab, int W,
-                   const double *gpart, const qlk::RunParams *rp1, double *grows, hipStream_t st, int stage)
+void launch_adj_mode_nz(const qlk::AdjModeArgs &am, int W, const qlk::RunParams *rp1, double *grows, hipStream_t st)
 {
     using P = typename std::conditional<MODEL == 0, qlk::ModelFull, qlk::ModelBQ>::type;
-    if (stage == 0) {
-        qlk::k_adj_mf_a<NZ, MODEL><<<1, qlk::NT, 0, st>>>(aa);
-    } else if (stage == 1) {
-        if (am.mode == qlk::MODE_CN) qlk::k_adj_mode<NZ, P, qlk::MODE_CN><<<W, qlk::NT, 0, st>>>(am);
-        else qlk::k_adj_mode<NZ, P, qlk::MODE_ELIN><<<W, qlk::NT, 0, st>>>(am);
-        const int ncols = 8 * NZ + qlk::NGP;
-        qlk::k_reduce_cols<<<dim3((ncols + qlk::RED_CW - 1) / qlk::RED_CW, 1), qlk::NT, 0, st>>>(gpart, rp1, ncols, grows);
-    } else {
-        qlk::k_adj_mf_b<NZ, MODEL><<<1, qlk::NT, 0, st>>>(ab);
-    }
+    if (am.mode == qlk::MODE_CN) qlk::k_adj_mode<NZ, P, qlk::MODE_CN><<<W, qlk::NT, 0, st>>>(am);
+    else qlk::k_adj_mode<NZ, P, qlk::MODE_ELIN><<<W, qlk::NT, 0, st>>>(am);
+    const int ncols = 8 * NZ + qlk::NGP;
+    qlk::k_reduce_cols<<<dim3((ncols + qlk::RED_CW - 1) / qlk::RED_CW, 1), qlk::NT, 0, st>>>(am.gpart, rp1, ncols, grows);
 }
 
 template <int MODEL>
-void launch_adj_m(int NZ, const qlk::AdjModeArgs &am, const qlk::AdjMFArgs &aa, const qlk::AdjMF2Args &ab, int W,
-                  const double *gpart, const qlk::RunParams *rp1, double *grows, hipStream_t st, int stage)
+void launch_adj_mode_m(int NZ, const qlk::AdjModeArgs &am, int W, const qlk::RunParams *rp1, double *grows, hipStream_t st)
 {
     switch (NZ) {
-    case 32: launch_adj_nz<32, MODEL>(am, aa, ab, W, gpart, rp1, grows, st, stage); break;
-    case 64: launch_adj_nz<64, MODEL>(am, aa, ab, W, gpart, rp1, grows, st, stage); break;
-    case 128: launch_adj_nz<128, MODEL>(am, aa, ab, W, gpart, rp1, grows, st, stage); break;
-    default: launch_adj_nz<256, MODEL>(am, aa, ab, W, gpart, rp1, grows, st, stage); break;
+    case 32: launch_adj_mode_nz<32, MODEL>(am, W, rp1, grows, st); break;
+    case 64: launch_adj_mode_nz<64, MODEL>(am, W, rp1, grows, st); break;
+    case 128: launch_adj_mode_nz<128, MODEL>(am, W, rp1, grows, st); break;
+    default: launch_adj_mode_nz<256, MODEL>(am, W, rp1, grows, st); break;
     }
 }
 
-void launch_adj(int NZ, int model, const qlk::AdjModeArgs &am, const qlk::AdjMFArgs &aa, const qlk::AdjMF2Args &ab,
-                int W, const double *gpart, const qlk::RunParams *rp1, double *grows, hipStream_t st, int stage)
+// the reverse mode kernel and the column sums of its partial rows
+int launch_adj_mode(int NZ, int model, const qlk::AdjModeArgs &am, int W, const qlk::RunParams *rp1, double *grows,
+                    hipStream_t st)
 {
-    if (model == QL_MODEL_MHD_BQLIN) launch_adj_m<1>(NZ, am, aa, ab, W, gpart, rp1, grows, st, stage);
-    else launch_adj_m<0>(NZ, am, aa, ab, W, gpart, rp1, grows, st, stage);
+    if (model == QL_MODEL_MHD_BQLIN) launch_adj_mode_m<1>(NZ, am, W, rp1, grows, st);
+    else launch_adj_mode_m<0>(NZ, am, W, rp1, grows, st);
+    QL_HIP(hipGetLastError());
+    return QL_OK;
+}
+
+template <int NZ>
+void launch_adj_mf_nz(int model, const qlk::AdjMFArgs &a, hipStream_t st)
+{
+    if (model == QL_MODEL_MHD_BQLIN) qlk::k_adj_mf<NZ, 1><<<1, qlk::NT, 0, st>>>(a);
+    else qlk::k_adj_mf<NZ, 0><<<1, qlk::NT, 0, st>>>(a);
+}
+
+int launch_adj_mf(int NZ, int model, const qlk::AdjMFArgs &a, hipStream_t st)
+{
+    switch (NZ) {
+    case 32: launch_adj_mf_nz<32>(model, a, st); break;
+    case 64: launch_adj_mf_nz<64>(model, a, st); break;
+    case 128: launch_adj_mf_nz<128>(model, a, st); break;
+    default: launch_adj_mf_nz<256>(model, a, st); break;
+    }
+    QL_HIP(hipGetLastError());
+    return QL_OK;
+}
+
+// The context's AdjState for a forward of nsteps with checkpoints every `every`
+// steps: buffers of an earlier forward are kept where they fit and given back
+// where they do not
+int adj_fit(Batch &b, int nsteps, int every, bool noise)
+{
+    if (!b.adj) b.adj = new AdjState();
+    AdjState *A = b.adj;
+    A->valid = false;
+    if (A->every != every || A->noise != noise) {
+        QL_HIP(hipStreamSynchronize(b.s));
+        free_segment(A);
+    }
+    A->nsteps = nsteps;
+    A->every = every;
+    A->nseg = (nsteps + every - 1) / every;
+    A->noise = noise;
+    if ((int)A->ck.size() > A->nseg + 1) {
+        QL_HIP(hipStreamSynchronize(b.s));
+        for (size_t k = A->nseg + 1; k < A->ck.size(); ++k) free_ck(A->ck[k]);
+    }
+    A->ck.resize(A->nseg + 1);
+    return QL_OK;
 }
 
 int adjoint_forward(Batch &b, int nsteps, int every, double *t_inout)
 {
     QL_RC(check_adjoint(b, "ql_adjoint_forward"));
     if (nsteps < 1 || every < 1) return fail(QL_ERR_ARG, "ql_adjoint_forward: nsteps=%d, every=%d", nsteps, every);
-    adj_release(b);
-    AdjState *A = new AdjState();
-    b.adj = A;
-    A->nsteps = nsteps;
-    A->every = every;
-    A->nseg = (nsteps + every - 1) / every;
-    A->noise = b.groups[0].noise;
+    QL_RC(adj_fit(b, nsteps, every, b.groups[0].noise));
+    AdjState *A = b.adj;
     A->t_init = b.t_init;
-    A->ck.resize(A->nseg + 1);
     double t = *t_inout;
     for (int sg = 0; sg < A->nseg; ++sg) {
         QL_RC(save_ck(b, A->ck[sg], t));
@@ -199,7 +251,7 @@ int adjoint_forward(Batch &b, int nsteps, int every, double *t_inout)
     }
     QL_RC(save_ck(b, A->ck[A->nseg], t));
     QL_HIP(hipStreamSynchronize(b.s));
-    A->t_end = t;
+    A->valid = true;
     *t_inout = t;
     return QL_OK;
 }
@@ -209,7 +261,7 @@ int adjoint_backward(Batch &b, const double *g_lin, const double *g_mf, double *
 {
     QL_RC(check_adjoint(b, "ql_adjoint_backward"));
     AdjState *A = b.adj;
-    if (!A) return fail(QL_ERR_STATE, "ql_adjoint_backward: no ql_adjoint_forward on this context");
+    if (!A || !A->valid) return fail(QL_ERR_STATE, "ql_adjoint_backward: no ql_adjoint_forward on this context");
     if (A->noise != b.groups[0].noise)
         return fail(QL_ERR_STATE, "ql_adjoint_backward: the driving noise changed since ql_adjoint_forward");
     Group &g = b.groups[0];
@@ -219,30 +271,31 @@ int adjoint_backward(Batch &b, const double *g_lin, const double *g_mf, double *
     const int MB = qlk::NT / NZ;  // modes per pass of the reverse mode kernel
     const int W = std::min((nxy + MB - 1) / MB, ADJ_GMAX);
     const int ncols = 8 * NZ + qlk::NGP;
-    if (!A->gu) {
+    if (!A->st_u) {
         QL_RC(dalloc(&A->st_u, nl * (3 * K + 1)));
         QL_RC(dalloc(&A->st_mf, nm * (3 * K + 1)));
         QL_RC(dalloc(&A->st_kx0, (size_t)nxy * K));
+        // zeroed: MHD_BQlin writes 3 of the 8 profile lines
+        QL_RC(dalloc(&A->st_mfz, (size_t)8 * NZ * (3 * K + 1)));
         if (g.noise) QL_RC(dalloc(&A->st_pre, nl * K));
+    }
+    if (!A->rp1) {
         QL_RC(dalloc(&A->gu, nl));
         QL_RC(dalloc(&A->gnp, nl));
         QL_RC(dalloc(&A->gM, nm));
         QL_RC(dalloc(&A->gnmp, nm));
-        QL_RC(dalloc(&A->gsums, (size_t)4 * NZ));
-        QL_HIP(hipMemset(A->gsums, 0, sizeof(double) * 4 * NZ));  // MHD_BQlin fills 2 of the 4 lines
+        QL_RC(dalloc(&A->gsums, (size_t)4 * NZ));  // zeroed: MHD_BQlin fills 2 of the 4 lines
         QL_RC(dalloc(&A->gpart, (size_t)W * ncols));
         QL_RC(dalloc(&A->grows, (size_t)ncols));
         QL_RC(dalloc(&A->gpar_mf, (size_t)qlk::NGP));
         QL_RC(dalloc(&A->gpar, (size_t)qlk::NGP));
-        QL_RC(dalloc(&A->mfz, (size_t)8 * NZ));
-        // MHD_BQlin writes 3 of the 8 profile lines; the others stay zero
-        QL_HIP(hipMemset(A->mfz, 0, sizeof(double) * 8 * NZ));
-        QL_RC(dalloc(&A->rp1, 1));
         qlk::RunParams rp = g.h_rp[0];
         rp.wg_off = 0;
         rp.nwg = W;
-        QL_HIP(hipMemcpy(A->rp1, &rp, sizeof(rp), hipMemcpyHostToDevice));
+        rp.wg_off2 = rp.nwg2 = 0;
         A->W = W;
+        QL_RC(dalloc(&A->rp1, 1));
+        QL_HIP(hipMemcpy(A->rp1, &rp, sizeof(rp), hipMemcpyHostToDevice));
     }
     // HD_fullU runs the MHD_FullQlin kernels with b = B = 0 on the internal
     // four-field layout: its caller's (ux, zeta) and (Ux, Uy) gradients sit at
@@ -268,22 +321,35 @@ int adjoint_backward(Batch &b, const double *g_lin, const double *g_mf, double *
     QL_HIP(hipMemsetAsync(A->gpar, 0, sizeof(double) * qlk::NGP, b.s));
 
     const bool cn = (b.integrator == QL_INT_RK3CN);
+    // the clock advances on the device through a segment; variable steps and
+    // driven ones need the host's times step by step
+    const bool stepwise = b.vdt || g.noise;
+    bool have_rows = false;  // a reverse substep's sums wait for their z-profile adjoint
+    qlk::AdjMFArgs aa{};
+    aa.gpar_total = A->gpar;
+    aa.fac = 1.0 / NZ;
+    aa.gM = A->gM;
+    aa.gnmp = A->gnmp;
+    aa.kzv = g.kzv;
+    aa.tw = g.tw;
+    aa.gsums = A->gsums;
+    aa.gpar = A->gpar_mf;
+    aa.ph = g.h_rp[0].ph;
+    aa.mode = cn ? qlk::MODE_CN : qlk::MODE_ELIN;
     for (int sg = A->nseg - 1; sg >= 0; --sg) {
         const int n = std::min(K, A->nsteps - sg * K);
-        // recompute the segment, keeping every substep state
-        QL_RC(load_ck(b, A->ck[sg]));
+        // recompute the segment, every substep into the next slot
+        QL_RC(load_ck(b, A->ck[sg], A->st_u, A->st_mf, A->st_mfz));
         double t = A->ck[sg].t;
         std::vector<double> st_t(n), st_tp(n), st_dt(n), st_dtl(n);
         std::vector<int> st_oi(n);
-        QL_HIP(hipMemcpyAsync(A->st_u, g.u, sizeof(double2) * nl, hipMemcpyDeviceToDevice, b.s));
-        QL_HIP(hipMemcpyAsync(A->st_mf, g.mf, sizeof(double2) * nm, hipMemcpyDeviceToDevice, b.s));
         for (int k = 0; k < n; ++k) {
             st_t[k] = t;
             st_tp[k] = b.t_prev;
             st_oi[k] = b.old_init;
             QL_HIP(hipMemcpyAsync(A->st_kx0 + (size_t)k * nxy, g.kx0, sizeof(double) * nxy, hipMemcpyDeviceToDevice,
                                   b.s));
-            QL_RC(set_clock(b, t));
+            if (k == 0 || stepwise) QL_RC(set_clock(b, t));
             // with variable steps the device chose the step from the profile
             // maxima, as in the forward (ql_step); the reverse takes it as given
             double dt = b.dt;
@@ -295,17 +361,16 @@ int adjoint_backward(Batch &b, const double *g_lin, const double *g_mf, double *
             st_dt[k] = dt;
             st_dtl[k] = b.vdt ? b.dt_last : dt;
             for (int s = 1; s <= 3; ++s) {
-                // with noise the step's remap follows the noise (main.cpp:111-123)
-                QL_RC(enqueue_substep(b, g, s, s == 3 && !g.noise, false, b.s));
-                if (s == 3 && g.noise) {
-                    QL_HIP(hipMemcpyAsync(A->st_pre + (size_t)k * nl, g.u, sizeof(double2) * nl,
-                                          hipMemcpyDeviceToDevice, b.s));
-                    QL_RC(launch_noise(g, false, t, dt, true, r.p.remap != 0, b.s));
-                }
                 const size_t j = (size_t)3 * k + s;
-                QL_HIP(hipMemcpyAsync(A->st_u + j * nl, g.u, sizeof(double2) * nl, hipMemcpyDeviceToDevice, b.s));
-                QL_HIP(hipMemcpyAsync(A->st_mf + j * nm, mf_after_substep(b, g, s), sizeof(double2) * nm,
-                                      hipMemcpyDeviceToDevice, b.s));
+                const SubBuffers bf{A->st_u + (j - 1) * nl, A->st_mf + (j - 1) * nm, A->st_u + j * nl,
+                                    A->st_mf + j * nm, A->st_mfz + (j - 1) * 8 * NZ, A->st_mfz + j * 8 * NZ};
+                // with noise the step's remap follows the noise (main.cpp:111-123)
+                QL_RC(enqueue_substep(b, g, s, s == 3 && !g.noise, !stepwise, b.s, &bf));
+                if (s == 3 && g.noise) {
+                    QL_HIP(hipMemcpyAsync(A->st_pre + (size_t)k * nl, A->st_u + j * nl, sizeof(double2) * nl,
+                                          hipMemcpyDeviceToDevice, b.s));
+                    QL_RC(launch_noise(g, A->st_u + j * nl, false, t, dt, true, r.p.remap != 0, b.s));
+                }
             }
             b.t_prev = t;
             b.dt_last = dt;
@@ -331,32 +396,16 @@ int adjoint_backward(Batch &b, const double *g_lin, const double *g_mf, double *
                     nlc1 = A2 * dt;
                     nlc2 = B2 * dt;
                 }
-                // z-profiles of the substep's mean fields
-                qlk::MFArgs pm = mf_args(b, g);
-                pm.mode = qlk::MODE_PROFILES;
-                pm.mf = A->st_mf + jin * nm;
-                pm.mfz = A->mfz;
-                pm.mfn_out = g.mfN1;
-                pm.advance = 0;
-                pm.vdt = pm.rec = 0;  // profiles only: no CFL records, no clock
-                launch_mf(g, pm, b.s);
-                QL_HIP(hipGetLastError());
-
-                qlk::AdjMFArgs aa{};
-                aa.gM = A->gM;
-                aa.gnmp = A->gnmp;
+                // the substep reversed before: its z-profiles; this one: its
+                // mean fields
+                aa.rows = have_rows ? A->grows : nullptr;
                 aa.M_in = A->st_mf + jin * nm;
                 aa.M_out = A->st_mf + jout * nm;
-                aa.kzv = g.kzv;
-                aa.tw = g.tw;
-                aa.gsums = A->gsums;
-                aa.gpar = A->gpar_mf;
-                aa.ph = g.h_rp[0].ph;
-                aa.mode = cn ? qlk::MODE_CN : qlk::MODE_ELIN;
                 aa.s = s;
                 aa.linC = lc;
                 aa.nlc1 = nlc1;
                 aa.nlc2 = nlc2;
+                QL_RC(launch_adj_mf(NZ, b.model, aa, b.s));
 
                 qlk::AdjModeArgs am{};
                 am.u_in = A->st_u + jin * nl;
@@ -368,7 +417,7 @@ int adjoint_backward(Batch &b, const double *g_lin, const double *g_mf, double *
                 am.ky = g.ky;
                 am.kzv = g.kzv;
                 am.tw = g.tw;
-                am.mfz = A->mfz;
+                am.mfz = A->st_mfz + jin * 8 * NZ;
                 am.gsums = A->gsums;
                 am.gpart = A->gpart;
                 am.ph = g.h_rp[0].ph;
@@ -392,24 +441,16 @@ int adjoint_backward(Batch &b, const double *g_lin, const double *g_mf, double *
                 if (g.noise) am.np = g.h_np[0];
                 am.t_step = st_t[k];
                 am.dt_step = dt;
-
-                qlk::AdjMF2Args ab{};
-                ab.gM = A->gM;
-                ab.rows = A->grows;
-                ab.gpar_mf = A->gpar_mf;
-                ab.gpar_total = A->gpar;
-                ab.kzv = g.kzv;
-                ab.tw = g.tw;
-                ab.fac = 1.0 / NZ;
-                for (int stage = 0; stage < 3; ++stage) {
-                    launch_adj(NZ, b.model, am, aa, ab, A->W, A->gpart, A->rp1, A->grows, b.s, stage);
-                    QL_HIP(hipGetLastError());
-                }
+                QL_RC(launch_adj_mode(NZ, b.model, am, A->W, A->rp1, A->grows, b.s));
+                have_rows = true;
             }
         }
     }
+    aa.rows = have_rows ? A->grows : nullptr;
+    aa.s = 0;
+    QL_RC(launch_adj_mf(NZ, b.model, aa, b.s));
     // leave the context at the forward's final state
-    QL_RC(load_ck(b, A->ck[A->nseg]));
+    QL_RC(load_ck(b, A->ck[A->nseg], g.u, g.mf, g.mfz));
     if (b.hd) {
         QL_HIP(hipStreamSynchronize(b.s));
         QL_HIP(hipMemcpy(hl.data(), A->gu, sizeof(double2) * nl, hipMemcpyDeviceToHost));

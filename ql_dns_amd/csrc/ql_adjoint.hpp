@@ -15,18 +15,18 @@
 // versa, so the reverse pass reuses the forward transform code unchanged.
 //
 // One reverse substep (host sequence, ql_adjoint.hip):
-//   k_adj_mf_a    one workgroup: mean-field update and mean-field RHS in
-//                 reverse, drive (EMF / stress) reverse down to dL/d(stress
-//                 z-profiles) by an inverse transform;
+//   k_adj_mf      one workgroup: z-profile adjoint of the substep reversed
+//                 before into dL/dM and parameter gradient accumulation, then
+//                 mean-field update and mean-field RHS in reverse, drive (EMF /
+//                 stress) reverse down to dL/d(stress z-profiles) by an inverse
+//                 transform;
 //   k_adj_mode    per mode: recompute the forward lines and products, then
 //                 reverse the update, the RHS assembly, the forward transforms,
 //                 the mean-field x fluctuation products and the EMF / stress
 //                 products, the inverse transforms and the base fields; per
 //                 workgroup partial rows of dL/d(mean-field z-profiles) and of
 //                 the parameter gradients;
-//   k_reduce_cols column sum of those rows;
-//   k_adj_mf_b    one workgroup: z-profile adjoint into dL/dM, parameter
-//                 gradient accumulation.
+//   k_reduce_cols column sum of those rows.
 // The remap decision (MHD_FullQlin.cpp:470-472) is piecewise constant in q and
 // enters as a fixed mask.
 #pragma once
@@ -144,9 +144,8 @@ static __device__ __noinline__ double noise_q_gradient(NoiseParams np, double q,
 // momentum lines of MHD_FullQlin (the induction lines enter N linearly with
 // constant factors) and the second line of MHD_BQlin.  Bound by the transforms
 // (21 lines per mode, LDS and FP64 issue).  Against three radix-8 passes over
-// unpadded lines with all 24 transforms and the products in two halves, whole
-// gradients: 64x64x128 RK3CN, 20 steps 16.0 -> 9.7 ms; 32x32x64, 200 steps
-// 43.2 -> 37.3 ms.
+// unpadded lines with all 24 transforms and the products in two halves (rocprof,
+// us): 64x64x128 RK3CN 132.8 -> 36.8, 32x32x64 RK3CN_Elin 19.8 -> 14.2.
 template <int NZ, class P, int MODE>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_adj_mode(AdjModeArgs a)
 {
@@ -582,110 +581,170 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_
 }
 
 // ---------------------------------------------------------------------------
-// mean fields in reverse, part A (one workgroup)
+// mean fields in reverse, one workgroup between the mode kernels of two
+// reverse substeps: first the z-profile adjoint of the substep just reversed
+// (rows), then the update, RHS and drive of the next one (s).  Two two-pass
+// transforms between separate LDS regions; latency-bound, like k_meanfield (32x32x64:
+// 5.5 us, 8.7 for the two launches it replaces).
 // ---------------------------------------------------------------------------
 struct AdjMFArgs {
+    // z-profile part (rows null: none): adds the profiles' gradient to gM and
+    // the substep's parameter gradients (rows' and gpar's) to gpar_total
+    const double *rows;  // reduced partial rows [8 NZ + NGP]
+    double *gpar_total;  // [NGP]
+    double fac;
+    // update part (s = 0: none)
     double2 *gM;           // in: dL/dM_out; out: dL/dM_in without the z-profile path
     double2 *gnmp;         // in (s < 3): dL/dNM_s; out (s > 1): dL/dNM_{s-1}
     const double2 *M_in, *M_out;
     const double *kzv;
     const double2 *tw;
     double *gsums;         // out: dL/d(EMF / stress z-profiles) [4][NZ]
-    double *gpar;          // out: parameter-gradient partials [NGP]
+    double *gpar;          // parameter-gradient partials [NGP] of the substep's mean fields
     Phys ph;
     int mode, s;
     double linC, nlc1, nlc2;
 };
 
 // MODEL 0: MHD_FullQlin (Bx, By, Ux, Uy); 1: MHD_BQlin (Bx, By: N_Bx = EMF x,
-// N_By = -q Bx + EMF y, both with eta kz^2, MHD_BQlin.cpp:274-280)
+// N_By = -q Bx + EMF y, both with eta kz^2, MHD_BQlin.cpp:274-280).  The
+// z-profiles are mfz_l = Re(inverse(pad(c_l M))) with c = fac (l even) or
+// i fac kz (l odd) (MHD_FullQlin.cpp:180-198); MHD_BQlin's are By, dz By, dz^2
+// By with c = fac, i fac kz, -fac kz^2 (MHD_BQlin.cpp:122-127), Bx has none.
 template <int NZ, int MODEL>
-__global__ __launch_bounds__(NT) void k_adj_mf_a(AdjMFArgs a)
+__global__ __launch_bounds__(NT) void k_adj_mf(AdjMFArgs a)
 {
     using D = Dealias<NZ>;
+    using PL = Plan2<NZ>;
     constexpr int NZD = D::nz, HALF = D::half;
-    constexpr int NM = MODEL == 0 ? 4 : 2;
-    __shared__ double2 buf[4 * NZ];
+    constexpr int NM = MODEL == 0 ? 4 : 2, NP = MODEL == 0 ? 8 : 3;
+    constexpr int KW = (NM * NZD + NT - 1) / NT;
+    __shared__ double2 padb[8 * PadIO<NZ, double2>::LP];
+    __shared__ double2 line[8 * NZ];
     __shared__ double2 tw[NZ];
     __shared__ double skz[NZD];
-    __shared__ double2 sGN[4 * NZD], sdir[4 * NZD];
-    __shared__ double red[5][NT];
+    __shared__ double2 sGN[4 * NZD], sM[4 * NZD];
+    __shared__ double red[5][NT / 64];
     const int tid = threadIdx.x;
     const Phys ph = a.ph;
-    for (int k = tid; k < NZ; k += NT) tw[k] = a.tw[k];
-    for (int k = tid; k < NZD; k += NT) skz[k] = a.kzv[k];
+    const PadIO<NZ, double2> pad{padb};
+    const BufIO<NZ, double2> lines{line};
+    // loads of both parts first, so that they are in flight together
+    double2 g[KW], gin[KW], Mo[KW], Mi[KW];
+#pragma unroll
+    for (int w = 0; w < KW; ++w) {
+        const int k = tid + w * NT;
+        const bool ok = k < NM * NZD, up = ok && a.s > 0;
+        g[w] = ok ? a.gM[k] : make_double2(0.0, 0.0);
+        gin[w] = (up && a.s < 3) ? a.gnmp[k] : make_double2(0.0, 0.0);
+        Mo[w] = up ? a.M_out[k] : make_double2(0.0, 0.0);
+        Mi[w] = up ? a.M_in[k] : make_double2(0.0, 0.0);
+    }
+    if (tid < NZ) tw[tid] = a.tw[tid];
+    if (tid < NZD) skz[tid] = a.kzv[tid];
+    if (a.rows && tid < NGP) a.gpar_total[tid] += a.gpar[tid] + a.rows[8 * NZ + tid];
     __syncthreads();
+    if (a.rows) {
+        const double *R = a.rows;
+        const auto ld = [R](int l, int j) { return make_double2(R[l * NZ + j], 0.0); };
+        fft_pass_io<NZ, NP, false, PL::R1, 1, false>(tw, ld, pad);
+        fft_pass_io<NZ, NP, false, PL::R2, PL::R1, false>(tw, pad, lines);
+#pragma unroll
+        for (int w = 0; w < KW; ++w) {
+            const int k = tid + w * NT;
+            if (k >= NM * NZD) continue;
+            const int f = k / NZD, m = k % NZD;
+            const double kz = skz[m];
+            const int j = D::pad(m);
+            if (MODEL == 0) {
+                g[w] = cadd(g[w], cadd(cscale(a.fac, line[(2 * f) * NZ + j]),
+                                       imul(-a.fac * kz, line[(2 * f + 1) * NZ + j])));
+            } else if (f == 1) {
+                double2 G = cadd(cscale(a.fac, line[j]), imul(-a.fac * kz, line[NZ + j]));
+                g[w] = cadd(g[w], cadd(G, cscale(-a.fac * kz * kz, line[2 * NZ + j])));
+            }
+        }
+    }
+    if (a.s == 0) {
+#pragma unroll
+        for (int w = 0; w < KW; ++w)
+            if (tid + w * NT < NM * NZD) a.gM[tid + w * NT] = g[w];
+        return;
+    }
     double gq = 0, gom = 0, gnu = 0, geta = 0, gb0 = 0;
+    double2 dir[KW];
     // update in reverse (RK3CN_Elin.cpp:109-112 / RK3CN.cpp:112-115)
-    for (int k = tid; k < NM * NZD; k += NT) {
+#pragma unroll
+    for (int w = 0; w < KW; ++w) {
+        const int k = tid + w * NT;
+        dir[w] = make_double2(0.0, 0.0);
+        if (k >= NM * NZD) continue;
         const int f = k / NZD, m = k % NZD;
         const double kz2 = -(skz[m] * skz[m]);
         const double coef = f < 2 ? ph.eta : ph.nu;
         const double L = ph.quasilinear ? coef * kz2 : 0.0;
-        const double2 g = a.gM[k];
-        const double2 gin = (a.s < 3) ? a.gnmp[k] : make_double2(0.0, 0.0);
-        double2 GN, dir;
+        double2 GN;
         double gL;
         if (a.mode == MODE_ELIN) {
-            const double2 mu = cscale(exp(a.linC * L), g);
-            GN = cadd(cscale(a.nlc1, mu), gin);
+            const double2 mu = cscale(exp(a.linC * L), g[w]);
+            GN = cadd(cscale(a.nlc1, mu), gin[w]);
             if (a.s > 1) a.gnmp[k] = cscale(a.nlc2, mu);
-            dir = mu;
-            gL = a.linC * redot(a.M_out[k], g);
+            dir[w] = mu;
+            gL = a.linC * redot(Mo[w], g[w]);
         } else {
             const double d = 1.0 / (1.0 - a.linC * L);
-            GN = cadd(cscale(a.nlc1 * d, g), gin);
-            if (a.s > 1) a.gnmp[k] = cscale(a.nlc2 * d, g);
-            dir = cscale((1 + a.linC * L) * d, g);
-            gL = a.linC * d * (redot(a.M_in[k], g) + redot(a.M_out[k], g));
+            GN = cadd(cscale(a.nlc1 * d, g[w]), gin[w]);
+            if (a.s > 1) a.gnmp[k] = cscale(a.nlc2 * d, g[w]);
+            dir[w] = cscale((1 + a.linC * L) * d, g[w]);
+            gL = a.linC * d * (redot(Mi[w], g[w]) + redot(Mo[w], g[w]));
         }
         if (ph.quasilinear) {
             if (f < 2) geta += gL * kz2;
             else gnu += gL * kz2;
         }
         sGN[k] = ph.quasilinear ? GN : make_double2(0.0, 0.0);
-        sdir[k] = dir;
+        sM[k] = Mi[w];
     }
     __syncthreads();
     // mean-field RHS in reverse (MHD_FullQlin.cpp:411-423)
-    for (int k = tid; k < NM * NZD; k += NT) {
+#pragma unroll
+    for (int w = 0; w < KW; ++w) {
+        const int k = tid + w * NT;
+        if (k >= NM * NZD) continue;
         const int f = k / NZD, m = k % NZD;
         const double kz = skz[m];
+        double2 G = dir[w];
         if constexpr (MODEL == 1) {
-            double2 G = sdir[k];
             if (f == 0) {
                 G = cadd(G, cscale(-ph.q, sGN[NZD + m]));
-                gq += redot(cscale(-1.0, a.M_in[m]), sGN[NZD + m]);
+                gq += redot(cscale(-1.0, sM[m]), sGN[NZD + m]);
             }
             a.gM[k] = G;
-            continue;
-        }
-        const double2 N0 = sGN[m], N1 = sGN[NZD + m], N2 = sGN[2 * NZD + m], N3 = sGN[3 * NZD + m];
-        double2 G = sdir[k];
-        if (f == 0) G = cadd(G, cadd(cscale(-ph.q, N1), imul(-ph.B0z * kz, N2)));
-        else if (f == 1) G = cadd(G, imul(-ph.B0z * kz, N3));
-        else if (f == 2) G = cadd(G, cadd(imul(-ph.B0z * kz, N0), cscale(ph.q - 2.0 * ph.omega, N3)));
-        else G = cadd(G, cadd(imul(-ph.B0z * kz, N1), cscale(2.0 * ph.omega, N2)));
-        a.gM[k] = G;
-        if (f == 0) {
-            const double2 M0 = a.M_in[m], M1 = a.M_in[NZD + m], M2 = a.M_in[2 * NZD + m], M3 = a.M_in[3 * NZD + m];
-            gq += redot(cscale(-1.0, M0), N1) + redot(M2, N3);
-            gom += redot(cscale(2.0, M3), N2) + redot(cscale(-2.0, M2), N3);
-            gb0 += redot(imul(kz, M2), N0) + redot(imul(kz, M3), N1) + redot(imul(kz, M0), N2) +
-                   redot(imul(kz, M1), N3);
+        } else {
+            const double2 N0 = sGN[m], N1 = sGN[NZD + m], N2 = sGN[2 * NZD + m], N3 = sGN[3 * NZD + m];
+            if (f == 0) G = cadd(G, cadd(cscale(-ph.q, N1), imul(-ph.B0z * kz, N2)));
+            else if (f == 1) G = cadd(G, imul(-ph.B0z * kz, N3));
+            else if (f == 2) G = cadd(G, cadd(imul(-ph.B0z * kz, N0), cscale(ph.q - 2.0 * ph.omega, N3)));
+            else G = cadd(G, cadd(imul(-ph.B0z * kz, N1), cscale(2.0 * ph.omega, N2)));
+            a.gM[k] = G;
+            if (f == 0) {
+                const double2 M0 = sM[m], M1 = sM[NZD + m], M2 = sM[2 * NZD + m], M3 = sM[3 * NZD + m];
+                gq += redot(cscale(-1.0, M0), N1) + redot(M2, N3);
+                gom += redot(cscale(2.0, M3), N2) + redot(cscale(-2.0, M2), N3);
+                gb0 += redot(imul(kz, M2), N0) + redot(imul(kz, M3), N1) + redot(imul(kz, M0), N2) +
+                       redot(imul(kz, M1), N3);
+            }
         }
     }
     // drive in reverse: Hermitian fill and x i kz of every line (the EMF,
     // MHD_FullQlin.cpp:326-336, and the stresses before their z-derivative),
     // then the forward transform's adjoint (an inverse transform) of the
     // real stress profiles
-    for (int k = tid; k < NM * NZ; k += NT) {
-        const int f = k / NZ, n = k % NZ;
+    const auto src = [&](int f, int n) {
         double2 v = make_double2(0.0, 0.0);
         if (n < HALF) {
             const double c = skz[n];
-            const double2 d0 = sGN[f * NZD + n];
-            v = imul(-c, d0);
+            v = imul(-c, sGN[f * NZD + n]);
             const int mm = 2 * HALF - 1 - n;  // slot filled with conj of this one
             if (n >= 1 && mm < NZD) {
                 double2 d1 = sGN[f * NZD + mm];
@@ -693,72 +752,25 @@ __global__ __launch_bounds__(NT) void k_adj_mf_a(AdjMFArgs a)
                 v = cadd(v, imul(-c, d1));
             }
         }
-        buf[k] = v;
+        return v;
+    };
+    double *gs = a.gsums;
+    const auto out = [gs](int l, int i, double2 v) { gs[l * NZ + i] = v.x; };
+    fft_pass_io<NZ, NM, true, PL::R1, 1, false>(tw, src, pad);
+    fft_pass_io<NZ, NM, true, PL::R2, PL::R1, false>(tw, pad, out);
+    const double gp[5] = {gq, gom, gnu, geta, gb0};
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+        const double t = wave_sum(gp[c]);
+        if (tid % 64 == 0) red[c][tid / 64] = t;
     }
-    __syncthreads();
-    fft_lines<NZ, NM, true>(buf, tw);
-    for (int k = tid; k < NM * NZ; k += NT) a.gsums[k] = buf[k].x;
-    red[0][tid] = gq;
-    red[1][tid] = gom;
-    red[2][tid] = gnu;
-    red[3][tid] = geta;
-    red[4][tid] = gb0;
     __syncthreads();
     if (tid < NGP) {
         double s = 0.0;
         if (tid < 5)
-            for (int k = 0; k < NT; ++k) s += red[tid][k];
+            for (int w = 0; w < NT / 64; ++w) s += red[tid][w];
         a.gpar[tid] = s;
     }
-}
-
-// ---------------------------------------------------------------------------
-// mean fields in reverse, part B (one workgroup): the z-profiles
-// mfz_l = Re(inverse(pad(c_l M))) with c = fac (l even) or i fac kz (l odd)
-// (MHD_FullQlin.cpp:180-198), and the parameter-gradient sum of the substep
-// ---------------------------------------------------------------------------
-struct AdjMF2Args {
-    double2 *gM;
-    const double *rows;     // reduced partial rows [8 NZ + NGP]
-    const double *gpar_mf;  // [NGP] from k_adj_mf_a
-    double *gpar_total;     // [NGP], accumulated
-    const double *kzv;
-    const double2 *tw;
-    double fac;
-};
-
-// MHD_BQlin: profiles By, dz By, dz^2 By = Re(inverse(pad(c_l By))) with
-// c = fac, i fac kz, -fac kz^2 (MHD_BQlin.cpp:122-127); Bx has none
-template <int NZ, int MODEL>
-__global__ __launch_bounds__(NT) void k_adj_mf_b(AdjMF2Args a)
-{
-    using D = Dealias<NZ>;
-    constexpr int NZD = D::nz;
-    __shared__ double2 buf[8 * NZ];
-    __shared__ double2 tw[NZ];
-    const int tid = threadIdx.x;
-    for (int k = tid; k < NZ; k += NT) tw[k] = a.tw[k];
-    for (int k = tid; k < 8 * NZ; k += NT) buf[k] = make_double2(a.rows[k], 0.0);
-    __syncthreads();
-    fft_lines<NZ, 8, false>(buf, tw);
-    if constexpr (MODEL == 1) {
-        for (int m = tid; m < NZD; m += NT) {
-            const double kz = a.kzv[m];
-            const int j = D::pad(m);
-            double2 G = cadd(cscale(a.fac, buf[j]), imul(-a.fac * kz, buf[NZ + j]));
-            G = cadd(G, cscale(-a.fac * kz * kz, buf[2 * NZ + j]));
-            a.gM[NZD + m] = cadd(a.gM[NZD + m], G);
-        }
-    } else {
-        for (int k = tid; k < 4 * NZD; k += NT) {
-            const int f = k / NZD, m = k % NZD;
-            const double kz = a.kzv[m];
-            const int j = D::pad(m);
-            const double2 G = cadd(cscale(a.fac, buf[(2 * f) * NZ + j]), imul(-a.fac * kz, buf[(2 * f + 1) * NZ + j]));
-            a.gM[k] = cadd(a.gM[k], G);
-        }
-    }
-    if (tid < NGP) a.gpar_total[tid] += a.gpar_mf[tid] + a.rows[8 * NZ + tid];
 }
 
 }  // namespace qlk

@@ -596,6 +596,7 @@ qlk::ModeArgs mode_args(const Batch &b, const Group &g)
 {
     qlk::ModeArgs a{};
     a.u = g.u;
+    a.u_out = g.u;
     a.kx0 = g.kx0;
     a.ky = g.ky;
     a.kzv = g.kzv;
@@ -676,10 +677,10 @@ qlk::MFArgs mf_args(const Batch &b, const Group &g)
     return m;
 }
 
-int launch_noise(Group &g, bool use_clock, double t, double dt, bool noise, bool remap, hipStream_t st)
+int launch_noise(Group &g, double2 *u, bool use_clock, double t, double dt, bool noise, bool remap, hipStream_t st)
 {
     qlk::NoiseArgs a{};
-    a.u = g.u;
+    a.u = u;
     a.kx0 = g.kx0;
     a.ky = g.ky;
     a.kzv = g.kzv;
@@ -807,8 +808,11 @@ int refresh_profiles(Batch &b, Group &g, hipStream_t st, bool rec)
 
 // One substep s (1..3) of RK3CN_Elin::Step (RK3CN_Elin.cpp:290-378) or
 // RK3CN::Step (RK3CN.cpp:92-193) for one group; times come from the group's
-// clock, which the last substep advances when `advance` is set.
-int enqueue_substep(Batch &b, Group &g, int s, bool remap_after, bool advance, hipStream_t st)
+// clock, which the last substep advances when `advance` is set.  The state, mean
+// fields and profiles are the group's own, or with `bf` read from and written
+// to its buffers (the adjoint's recomputation keeps every substep; the step's
+// noise is then the caller's).
+int enqueue_substep(Batch &b, Group &g, int s, bool remap_after, bool advance, hipStream_t st, const SubBuffers *bf)
 {
     const bool cn = (b.integrator == QL_INT_RK3CN);
     const double dt = b.dt;
@@ -827,7 +831,7 @@ int enqueue_substep(Batch &b, Group &g, int s, bool remap_after, bool advance, h
     }
     // with driving noise the step ends with the noise kernel, which remaps
     // after it (main.cpp:112-123)
-    const bool noisy = g.noise && advance && s == 3;
+    const bool noisy = g.noise && advance && s == 3 && !bf;
     qlk::ModeArgs a = mode_args(b, g);
     a.s = s;
     a.mode = cn ? qlk::MODE_CN : qlk::MODE_ELIN;
@@ -852,8 +856,16 @@ int enqueue_substep(Batch &b, Group &g, int s, bool remap_after, bool advance, h
         m.mf_in = mf_after_substep(b, g, s == 1 ? 3 : s - 1);
         m.mf = const_cast<double2 *>(mf_after_substep(b, g, s));
     }
+    if (bf) {
+        a.u = bf->u_in;
+        a.u_out = bf->u_out;
+        a.mfz = bf->mfz_in;
+        m.mf_in = bf->mf_in;
+        m.mf = bf->mf_out;
+        m.mfz = bf->mfz_out;
+    }
     QL_RC(enqueue_sequence(b, g, a, m, st));
-    if (noisy) QL_RC(launch_noise(g, true, 0.0, 0.0, true, remap_after, st));
+    if (noisy) QL_RC(launch_noise(g, g.u, true, 0.0, 0.0, true, remap_after, st));
     return QL_OK;
 }
 
@@ -1913,7 +1925,7 @@ int ql_batch_driving_noise(ql_batch *bt, double t, double dt)
     if (!bt) return fail(QL_ERR_ARG, "ql_batch_driving_noise: null handle");
     Batch &b = bt->b;
     for (Group &g : b.groups)
-        if (g.noise) QL_RC(launch_noise(g, false, t, dt, true, false, b.s));
+        if (g.noise) QL_RC(launch_noise(g, g.u, false, t, dt, true, false, b.s));
     QL_HIP(hipStreamSynchronize(b.s));
     return QL_OK;
 }

@@ -87,7 +87,8 @@ struct Clock {
 };
 
 struct ModeArgs {
-    double2 *u;             // state [modes][4][nz], updated in place (MODE_ELIN/CN)
+    const double2 *u;       // state [modes][4][nz] at the substep start
+    double2 *u_out;         // the updated state (MODE_ELIN/CN): u itself, or another buffer
     double2 *n_out;         // RHS out (nullable)
     const double2 *n_prev;  // previous substep RHS (nullable)
     double *lin_out;        // linear operator out (MODE_RHS, nullable)

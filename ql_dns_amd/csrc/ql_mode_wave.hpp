@@ -375,8 +375,8 @@ __device__ __forceinline__ void mode_wave_body(const ModeArgs &a)
                         un1 = cadd(s1, cscale(co, u1));
                     }
                     if (hit) un0 = un1 = make_double2(0.0, 0.0);
-                    a.u[off0] = un0;
-                    a.u[off1] = un1;
+                    a.u_out[off0] = un0;
+                    a.u_out[off1] = un1;
                     if (a.n_out) {
                         a.n_out[off0] = N0;
                         a.n_out[off1] = N1;

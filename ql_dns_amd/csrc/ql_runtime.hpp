@@ -221,11 +221,17 @@ int sync_all(Batch &b);
 int set_clock(Batch &b, double t);
 int set_clock_runs(Batch &b, const double *t_runs);
 int read_clock(Batch &b, qlk::Clock *c);
-int enqueue_substep(Batch &b, Group &g, int s, bool remap_after, bool advance, hipStream_t st);
-bool fused_tail(const Batch &b, const Group &g);
-const double2 *mf_after_substep(const Batch &b, const Group &g, int s);
+// where a substep reads and writes instead of the group's own buffers
+struct SubBuffers {
+    const double2 *u_in, *mf_in;
+    double2 *u_out, *mf_out;
+    const double *mfz_in;
+    double *mfz_out;
+};
+int enqueue_substep(Batch &b, Group &g, int s, bool remap_after, bool advance, hipStream_t st,
+                    const SubBuffers *bf = nullptr);
 void launch_mf(const Group &g, const qlk::MFArgs &m, hipStream_t st);
-int launch_noise(Group &g, bool use_clock, double t, double dt, bool noise, bool remap, hipStream_t st);
+int launch_noise(Group &g, double2 *u, bool use_clock, double t, double dt, bool noise, bool remap, hipStream_t st);
 qlk::MFArgs mf_args(const Batch &b, const Group &g);
 int refresh_profiles(Batch &b, Group &g, hipStream_t st, bool rec = false);
 int run_steps(Batch &b, int nsteps, double *t_inout);
