@@ -45,8 +45,6 @@ struct AdjState {
     // adjoint buffers
     double2 *gu = nullptr, *gnp = nullptr, *gM = nullptr, *gnmp = nullptr;
     double *gsums = nullptr, *gpart = nullptr, *grows = nullptr, *gpar_mf = nullptr, *gpar = nullptr;
-    qlk::RunParams *rp1 = nullptr;  // one run, rows [0, W) (column reduction)
-    int W = 0;
 };
 
 namespace {
@@ -65,7 +63,6 @@ void adj_release(Batch &b)
     free_segment(A);
     dfree(A->gu), dfree(A->gnp), dfree(A->gM), dfree(A->gnmp);
     dfree(A->gsums), dfree(A->gpart), dfree(A->grows), dfree(A->gpar_mf), dfree(A->gpar);
-    dfree(A->rp1);
     delete A;
     b.adj = nullptr;
 }
@@ -163,32 +160,31 @@ HostTimes host_times(double t, double t_prev, int old_init, double t_init, doubl
 }
 
 template <int NZ, int MODEL>
-void launch_adj_mode_nz(const qlk::AdjModeArgs &am, int W, const qlk::RunParams *rp1, double *grows, hipStream_t st)
+void launch_adj_mode_nz(const qlk::AdjModeArgs &am, int W, double *grows, hipStream_t st)
 {
     using P = typename std::conditional<MODEL == 0, qlk::ModelFull, qlk::ModelBQ>::type;
     if (am.mode == qlk::MODE_CN) qlk::k_adj_mode<NZ, P, qlk::MODE_CN><<<W, qlk::NT, 0, st>>>(am);
     else qlk::k_adj_mode<NZ, P, qlk::MODE_ELIN><<<W, qlk::NT, 0, st>>>(am);
     const int ncols = 8 * NZ + qlk::NGP;
-    qlk::k_reduce_cols<<<dim3((ncols + qlk::RED_CW - 1) / qlk::RED_CW, 1), qlk::NT, 0, st>>>(am.gpart, rp1, ncols, grows);
+    qlk::k_reduce_cols<<<dim3((ncols + qlk::RED_CW - 1) / qlk::RED_CW, 1), qlk::NT, 0, st>>>(am.gpart, nullptr, W, ncols, grows);
 }
 
 template <int MODEL>
-void launch_adj_mode_m(int NZ, const qlk::AdjModeArgs &am, int W, const qlk::RunParams *rp1, double *grows, hipStream_t st)
+void launch_adj_mode_m(int NZ, const qlk::AdjModeArgs &am, int W, double *grows, hipStream_t st)
 {
     switch (NZ) {
-    case 32: launch_adj_mode_nz<32, MODEL>(am, W, rp1, grows, st); break;
-    case 64: launch_adj_mode_nz<64, MODEL>(am, W, rp1, grows, st); break;
-    case 128: launch_adj_mode_nz<128, MODEL>(am, W, rp1, grows, st); break;
-    default: launch_adj_mode_nz<256, MODEL>(am, W, rp1, grows, st); break;
+    case 32: launch_adj_mode_nz<32, MODEL>(am, W, grows, st); break;
+    case 64: launch_adj_mode_nz<64, MODEL>(am, W, grows, st); break;
+    case 128: launch_adj_mode_nz<128, MODEL>(am, W, grows, st); break;
+    default: launch_adj_mode_nz<256, MODEL>(am, W, grows, st); break;
     }
 }
 
 // the reverse mode kernel and the column sums of its partial rows
-int launch_adj_mode(int NZ, int model, const qlk::AdjModeArgs &am, int W, const qlk::RunParams *rp1, double *grows,
-                    hipStream_t st)
+int launch_adj_mode(int NZ, int model, const qlk::AdjModeArgs &am, int W, double *grows, hipStream_t st)
 {
-    if (model == QL_MODEL_MHD_BQLIN) launch_adj_mode_m<1>(NZ, am, W, rp1, grows, st);
-    else launch_adj_mode_m<0>(NZ, am, W, rp1, grows, st);
+    if (model == QL_MODEL_MHD_BQLIN) launch_adj_mode_m<1>(NZ, am, W, grows, st);
+    else launch_adj_mode_m<0>(NZ, am, W, grows, st);
     QL_HIP(hipGetLastError());
     return QL_OK;
 }
@@ -279,7 +275,7 @@ int adjoint_backward(Batch &b, const double *g_lin, const double *g_mf, double *
         QL_RC(dalloc(&A->st_mfz, (size_t)8 * NZ * (3 * K + 1)));
         if (g.noise) QL_RC(dalloc(&A->st_pre, nl * K));
     }
-    if (!A->rp1) {
+    if (!A->gpar) {
         QL_RC(dalloc(&A->gu, nl));
         QL_RC(dalloc(&A->gnp, nl));
         QL_RC(dalloc(&A->gM, nm));
@@ -289,13 +285,6 @@ int adjoint_backward(Batch &b, const double *g_lin, const double *g_mf, double *
         QL_RC(dalloc(&A->grows, (size_t)ncols));
         QL_RC(dalloc(&A->gpar_mf, (size_t)qlk::NGP));
         QL_RC(dalloc(&A->gpar, (size_t)qlk::NGP));
-        qlk::RunParams rp = g.h_rp[0];
-        rp.wg_off = 0;
-        rp.nwg = W;
-        rp.wg_off2 = rp.nwg2 = 0;
-        A->W = W;
-        QL_RC(dalloc(&A->rp1, 1));
-        QL_HIP(hipMemcpy(A->rp1, &rp, sizeof(rp), hipMemcpyHostToDevice));
     }
     // HD_fullU runs the MHD_FullQlin kernels with b = B = 0 on the internal
     // four-field layout: its caller's (ux, zeta) and (Ux, Uy) gradients sit at
@@ -441,7 +430,7 @@ int adjoint_backward(Batch &b, const double *g_lin, const double *g_mf, double *
                 if (g.noise) am.np = g.h_np[0];
                 am.t_step = st_t[k];
                 am.dt_step = dt;
-                QL_RC(launch_adj_mode(NZ, b.model, am, A->W, A->rp1, A->grows, b.s));
+                QL_RC(launch_adj_mode(NZ, b.model, am, W, A->grows, b.s));
                 have_rows = true;
             }
         }

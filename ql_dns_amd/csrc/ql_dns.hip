@@ -665,6 +665,8 @@ qlk::MFArgs mf_args(const Batch &b, const Group &g)
     m.drive = g.drive;
     m.mfz = g.mfz;
     m.runs = g.rp;
+    m.one_run = g.nruns == 1;
+    m.ph1 = g.h_rp[0].ph;
     m.kzv = g.kzv;
     m.tw = g.tw;
     m.clock = g.clock;
@@ -785,8 +787,9 @@ int enqueue_sequence(Batch &b, Group &g, const qlk::ModeArgs &a, const qlk::MFAr
         launch_fused_tail(g, m, a.partials, st);
         QL_HIP(hipGetLastError());
     } else {
+        const int own_rows = g.nruns == 1 && g.h_rp[0].nwg2 == 0 ? g.h_rp[0].nwg : 0;
         qlk::k_reduce_cols<<<dim3((ncols + qlk::RED_CW - 1) / qlk::RED_CW, g.nruns), qlk::NT, 0, st>>>(
-            a.partials, g.rp, ncols, const_cast<double *>(m.sums));
+            a.partials, g.rp, own_rows, ncols, const_cast<double *>(m.sums));
         QL_HIP(hipGetLastError());
         launch_mf(g, m, st);
         QL_HIP(hipGetLastError());

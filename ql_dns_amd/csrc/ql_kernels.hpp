@@ -278,16 +278,30 @@ __device__ __forceinline__ void clock_advance(Clock *c)
 // Neumaier compensation.  A block (blockIdx.y = run) owns RED_CW columns; its
 // NT / RED_CW row chunks are summed in row order by separate threads and then
 // added in chunk order, so the result does not depend on scheduling.  No
-// cross-block communication (no fences, no atomics).
+// cross-block communication (no fences, no atomics).  A set of one run passes
+// its row count (own_rows; 0: read the run table), and the mean-field kernel its
+// physics, as launch arguments: one load latency less in each of the two short
+// launches (200 steps of 64x128x128 22.85 -> 22.6 ms, 100 of 36x60x64 MHD_BQlin
+// with noise 6.04 -> 5.86).
 // ---------------------------------------------------------------------------
 constexpr int RED_CW = 16;  // columns per block (4, 8 and 32 measured slower)
 
 [[maybe_unused]] static __global__ __launch_bounds__(NT) void k_reduce_cols(const double *__restrict__ part, const RunParams *__restrict__ runs,
-                                                    int ncols, double *__restrict__ sums)
+                                                    int own_rows, int ncols, double *__restrict__ sums)
 {
     constexpr int CW = RED_CW, CH = NT / CW;
     __shared__ double red[CH][CW + 1], red2[CH][CW + 1];
-    const RunParams &rp = runs[blockIdx.y];
+    RunParams rp;
+    if (own_rows) {
+        rp.nwg = own_rows;
+        rp.wg_off = rp.wg_off2 = rp.nwg2 = 0;
+    } else {
+        const RunParams &r = runs[blockIdx.y];
+        rp.nwg = r.nwg;
+        rp.wg_off = r.wg_off;
+        rp.nwg2 = r.nwg2;
+        rp.wg_off2 = r.wg_off2;
+    }
     const int cl = threadIdx.x % CW, chunk = threadIdx.x / CW;
     const int c = blockIdx.x * CW + cl;
     const int nrows = rp.nwg + rp.nwg2;
@@ -362,18 +376,12 @@ constexpr int AMP_NT = 1024;
     for (int l = tid; l < rp.nxy; l += AMP_NT) hi[rp.mode_off + l] = (double)amp[rp.mode_off + l] >= thr ? 1 : 0;
 }
 
-// sum over the workgroup's threads in a fixed order (every thread gets it)
-__device__ __forceinline__ double block_sum(double v, double *red)
+// sum over the 64 lanes of a wavefront in a fixed order (every lane gets it)
+__device__ __forceinline__ double wave_sum(double v)
 {
-    const int tid = threadIdx.x;
-    __syncthreads();
-    red[tid] = v;
-    __syncthreads();
-    for (int w = NT / 2; w > 0; w >>= 1) {
-        if (tid < w) red[tid] += red[tid + w];
-        __syncthreads();
-    }
-    return red[0];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    return v;
 }
 
 // ---------------------------------------------------------------------------
@@ -388,11 +396,12 @@ struct MFArgs {
     double2 *drive;           // [runs][nMF][nz]
     double *mfz;              // profiles out [runs][8][NZ]
     const RunParams *runs;
+    Phys ph1;                 // the physics of a set of one run (one_run != 0)
     const double *kzv;
     const double2 *tw;
     Clock *clock;  // advanced by dt when advance != 0 (last substep of a step)
     double *pm;    // profile maxima [runs][PM_STRIDE]
-    int model, nMF, mode, advance;
+    int model, nMF, mode, advance, one_run;
     int s, vdt;    // substep; variable steps (coefficients from the clock)
     int rec;       // record the CFL quantities in pm (variable steps, or on request)
     double fac, linC, nlc1, nlc2;
@@ -411,16 +420,16 @@ struct MFShared {
     double ssum[4 * NZ];      // summed stress / EMF z-profiles
     double2 smf[4 * NZD];     // mean fields at the start of the substep
     double2 sprev[4 * NZD];   // previous substep's mean-field RHS
-    double2 sdrive[4 * NZD];  // drives (HD_fullU records)
     double2 smfn[4 * NZD];    // updated mean fields
-    double red[NT];           // block sums
+    double pm[PM_STRIDE];     // CFL record
+    double red[5][NT / 64];   // its sums, per wavefront
 };
 
 // Inputs of the mean-field kernel (twiddles, wavenumbers, mean fields,
 // previous RHS, summed profiles) into LDS, every load issued before the first
 // store so that they are in flight together; meanfield_body starts with the
 // barrier that makes them visible.
-template <int NZ, int MODE, int MODEL>
+template <int NZ, int MODE, int MODEL, bool REC>
 __device__ __forceinline__ void meanfield_load(const MFArgs &a, int run, MFShared<NZ> &sh)
 {
     constexpr int NZD = Dealias<NZ>::nz;
@@ -447,6 +456,8 @@ __device__ __forceinline__ void meanfield_load(const MFArgs &a, int run, MFShare
         const int k = tid + w * NT;
         su[w] = (upd && k < nsum) ? a.sums[(size_t)run * nsum + k] : 0.0;
     }
+    const double pv = (REC && tid < PM_STRIDE) ? a.pm[(size_t)run * PM_STRIDE + tid] : 0.0;
+    if (REC && tid < PM_STRIDE) sh.pm[tid] = pv;
 #pragma unroll
     for (int w = 0; w < TW; ++w)
         if (tid + w * NT < NZ) sh.tw[tid + w * NT] = t[w];
@@ -525,42 +536,66 @@ __device__ __forceinline__ void meanfield_body(const MFArgs &a, int run, MFShare
     constexpr int NZD = D::nz, HALF = D::half;
     constexpr int MW = (4 * NZD + NT - 1) / NT;  // mean-field slots per thread
     const int tid = threadIdx.x;
-    double *pm = a.pm + (size_t)run * PM_STRIDE;
     StepCoefs cf{a.linC, a.nlc1, a.nlc2};
     if (REC && a.vdt && MODE != MODE_PROFILES && a.s > 0) cf = step_coefs(a.clock[run].dt, a.s, MODE == MODE_CN);
     const double linC = cf.linC, nlc1 = cf.nlc1, nlc2 = cf.nlc2;
-    // the right-hand side of this substep read the profiles of the current
-    // state (Calculate_CFL reads those, MHD_FullQlin.cpp:772)
     const bool rec = REC && a.rec != 0;
-    if (rec && MODE != MODE_PROFILES && tid < 8) pm[PM_RHS + tid] = pm[PM_CUR + tid];
-    if (rec && MODE != MODE_PROFILES && tid == 8) pm[PM_E_RHS] = pm[PM_E_CUR];
     const bool hd = rec && a.runs[run].hd != 0;
-    // mean |kz^2 Ux_drive|, mean |kz^2 Uy_drive| of a drive (HD_fullU.cpp:619)
-    auto drive_means = [&](const double2 *d) {
-        double sx = 0.0, sy = 0.0;
-        for (int m = tid; m < NZD; m += NT) {
-            const double k2 = -(sh.skz[m] * sh.skz[m]);
-            const double2 dx = d[2 * NZD + m], dy = d[3 * NZD + m];
-            sx += hypot(dx.x * k2, dx.y * k2);
-            sy += hypot(dy.x * k2, dy.y * k2);
+    // the CFL record is kept in LDS and HD_fullU's sums are reduced together by
+    // shuffles at the end (five sums by trees of eight barriers each and the
+    // record in memory: 10.1 us at 64x128x128 with variable steps, now 8.1)
+    // HD_fullU's sums: |kz^2 Ux_drive|, |kz^2 Uy_drive| of a drive
+    // (HD_fullU.cpp:619), |MUx|^2, |MUy|^2 over z (:618), |kz^2 Ux| (:619)
+    double sum[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    auto add_drive = [&](int f, int m, double2 d) {
+        const double k2 = -(sh.skz[m] * sh.skz[m]);
+        if (f == 2) sum[0] += hypot(d.x * k2, d.y * k2);
+        if (f == 3) sum[1] += hypot(d.x * k2, d.y * k2);
+    };
+    // the sums over the workgroup, in a fixed order, into the record; then the
+    // record to memory (n: how many of the sums were formed)
+    auto record = [&](int n) {
+        if (!rec) return;
+        if (hd) {
+#pragma unroll
+            for (int c = 0; c < 5; ++c) {
+                const double t = wave_sum(sum[c]);
+                if (tid % 64 == 0) sh.red[c][tid / 64] = t;
+            }
         }
-        sx = block_sum(sx, sh.red);
-        sy = block_sum(sy, sh.red);
-        if (tid == 0) {
-            pm[PM_DUX] = sx / NZD;
-            pm[PM_DUY] = sy / NZD;
+        __syncthreads();
+        if (hd && tid == 0) {
+#pragma unroll
+            for (int c = 0; c < 5; ++c) {
+                sum[c] = sh.red[c][0];
+#pragma unroll
+                for (int w = 1; w < NT / 64; ++w) sum[c] += sh.red[c][w];
+            }
+            sh.pm[PM_DUX] = sum[0] / NZD;
+            sh.pm[PM_DUY] = sum[1] / NZD;
+            if (n == 5) {
+                sh.pm[PM_E_CUR] = sum[2] + sum[3];
+                sh.pm[PM_UX] = sum[4] / NZD;
+            }
         }
+        __syncthreads();
+        if (tid < PM_STRIDE) a.pm[(size_t)run * PM_STRIDE + tid] = sh.pm[tid];
     };
     // the substep's mode kernel, the only reader of the clock, has finished;
     // dt is read above, before this block can change it (the next step's dt is
     // written at the end)
     if (a.advance && tid == 0) clock_advance(a.clock + run);
-    const Phys ph = a.runs[run].ph;
+    Phys ph = a.ph1;
+    if (!a.one_run) ph = a.runs[run].ph;
     const int nMF = NMF_OF(MODEL), nslot = nMF * NZD;
     const size_t mo = (size_t)run * nslot;
     const PadIO<NZ, double2> pad{sh.pad};
     const BufIO<NZ, double2> lines{sh.line};
     __syncthreads();  // the inputs meanfield_load stored
+    // the right-hand side of this substep read the profiles of the current
+    // state (Calculate_CFL reads those, MHD_FullQlin.cpp:772)
+    if (rec && MODE != MODE_PROFILES && tid < 8) sh.pm[PM_RHS + tid] = sh.pm[PM_CUR + tid];
+    if (rec && MODE != MODE_PROFILES && tid == 8) sh.pm[PM_E_RHS] = sh.pm[PM_E_CUR];
 
     if (MODE != MODE_PROFILES) {
         // forward transform of the summed z-profiles (real lines)
@@ -582,19 +617,23 @@ __device__ __forceinline__ void meanfield_body(const MFArgs &a, int run, MFShare
             mf_slot<NZD, HALF, MODE, MODEL>(f, m, sh.line + f * NZ, sh.skz, sh.smf, ph, a.mfn_prev != nullptr,
                                             sh.sprev[k], linC, nlc1, nlc2, Dv, N, Mn);
             a.drive[mo + k] = Dv;
-            if (hd) sh.sdrive[k] = Dv;
+            if (hd) add_drive(f, m, Dv);
             a.mfn_out[mo + k] = N;
             if (MODE == MODE_RHS) continue;
             a.mf[mo + k] = Mn;
             sh.smfn[k] = Mn;
         }
+        if (MODE == MODE_RHS) {
+            record(2);
+            return;
+        }
         __syncthreads();
-        if (hd) drive_means(sh.sdrive);
-        if (MODE == MODE_RHS) return;
     } else {
-        for (int k = tid; k < nslot; k += NT) sh.smfn[k] = sh.smf[k];
+        for (int k = tid; k < nslot; k += NT) {
+            sh.smfn[k] = sh.smf[k];
+            if (hd) add_drive(k / NZD, k % NZD, a.drive[mo + k]);  // the last rhs's drive
+        }
         __syncthreads();
-        if (hd) drive_means(a.drive + mo);  // the last rhs's drive
     }
     // real-space profiles for the next rhs (MHD_FullQlin.cpp:180-198,
     // MHD_BQlin.cpp:122-127): fac1D * ifft(pad(...)), real part; for
@@ -639,35 +678,23 @@ __device__ __forceinline__ void meanfield_body(const MFArgs &a, int run, MFShare
         }
 #pragma unroll
         for (int o = 16; o > 0; o >>= 1) m2 = fmax(m2, __shfl_xor(m2, o, 32));
-        if (j0 == 0) pm[PM_CUR + l] = sqrt(m2);
+        if (j0 == 0) sh.pm[PM_CUR + l] = sqrt(m2);
     }
     if (hd) {
-        // |MUx|^2 + |MUy|^2 summed over z (HD_fullU.cpp:618) and mean |kz^2 Ux|
-        // of the current state (:619)
-        double ex = 0.0, ey = 0.0, su = 0.0;
         for (int j = tid; j < NZ; j += NT) {
             const double2 x = sh.line[4 * NZ + j], y = sh.line[6 * NZ + j];
-            ex += x.x * x.x + x.y * x.y;
-            ey += y.x * y.x + y.y * y.y;
+            sum[2] += x.x * x.x + x.y * x.y;
+            sum[3] += y.x * y.x + y.y * y.y;
         }
         for (int m = tid; m < NZD; m += NT) {
             const double k2 = -(sh.skz[m] * sh.skz[m]);
             const double2 u = sh.smfn[2 * NZD + m];
-            su += hypot(u.x * k2, u.y * k2);
-        }
-        ex = block_sum(ex, sh.red);
-        ey = block_sum(ey, sh.red);
-        su = block_sum(su, sh.red);
-        if (tid == 0) {
-            pm[PM_E_CUR] = ex + ey;
-            pm[PM_UX] = su / NZD;
+            sum[4] += hypot(u.x * k2, u.y * k2);
         }
     }
-    if (REC && a.vdt && a.advance) {
-        __syncthreads();
-        // the run's next step dt (RK3CN_Elin.cpp:76-80)
-        if (tid == 0) a.clock[run].dt = cfl_dt(pm, a.runs[run], MODEL);
-    }
+    record(5);
+    // the run's next step dt (RK3CN_Elin.cpp:76-80)
+    if (REC && a.vdt && a.advance && tid == 0) a.clock[run].dt = cfl_dt(sh.pm, a.runs[run], MODEL);
 }
 
 // one workgroup per run (blockIdx.x); the substep mode, the model and
@@ -679,7 +706,7 @@ template <int NZ, int MODE, int MODEL, bool REC>
 __global__ __launch_bounds__(NT) void k_meanfield(MFArgs a)
 {
     __shared__ MFShared<NZ> sh;
-    meanfield_load<NZ, MODE, MODEL>(a, blockIdx.x, sh);
+    meanfield_load<NZ, MODE, MODEL, REC>(a, blockIdx.x, sh);
     meanfield_body<NZ, MODE, MODEL, REC>(a, blockIdx.x, sh);
 }
 
@@ -917,14 +944,6 @@ struct DiagFinalArgs {
     double Lz, totalN2, nu, eta, kzfac;
     double *out;  // [18]
 };
-
-// sum over the 64 lanes of a wavefront in a fixed order (every lane gets it)
-__device__ __forceinline__ double wave_sum(double v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
 
 // MHD_FullQlin.cpp:560-676, one workgroup: a thread per partial row and per
 // mean-field slot, the DIAG_SUMS sums over lanes by shuffles and over the
