@@ -221,3 +221,42 @@ def test_noise_and_remap_match_oracle():
     lg, mg, kg = g.get_state()
     assert np.array_equal(kg, ko) and not np.array_equal(kg, k_init)
     assert rel_err(mg, mo) < TOL and rel_err(lg, lo) < TOL
+
+
+@pytest.mark.parametrize("NX,NY,target", [(2, 2, 1), (6, 6, 3), (4, 10, 1 << 30)])
+@pytest.mark.parametrize("NZ", [128, 256])
+@pytest.mark.parametrize("model", [0, 1, 2])
+def test_z_lines_in_registers_match_oracle(model, NZ, NX, NY, target):
+    """The FP64 transforms at NZ = 128 and 256, whose lines pass between the rows
+    of a wavefront: every kept z mode of every field and of the mean fields set,
+    so that a line, point or band edge taken for another shows; one wavefront
+    for all modes, a partly filled workgroup, one mode per wavefront.
+
+    Bar: two 256-point transforms in FP64 (8 stages, a few eps each: 1e-14 of
+    the largest value) and three-term products around them, 100 times that."""
+    from ql_dns_amd.capi import QLContext
+    from ql_dns_amd.ic import initial_state, mode_tables
+    from oracle.oracle import Oracle
+    p = _params(model=model, NX=NX, NY=NY, NZ=NZ)
+    lin, mf = initial_state(p)
+    kx0, ky = mode_tables(p)[:2]
+    held = np.broadcast_to(((kx0 != 0) | (ky != 0))[:, None, None], lin.shape).copy()  # not the (0, 0) mode,
+    held[ky == 0, ::2, 0] = False  # and not the compressive slots
+    rng = np.random.default_rng(17 * NZ + model)
+    nzl = lin.shape[-1] // 2  # kz order 0..nzl, -nzl..-1
+    kz = np.r_[0:nzl + 1, nzl:0:-1]
+
+    def spectra(shape):
+        return (rng.standard_normal(shape) + 1j * rng.standard_normal(shape)) / (1.0 + kz)
+
+    lin, mf = np.where(held, spectra(lin.shape), 0.0), spectra(mf.shape)
+    mf[:, 0] = 0.0
+    mf[:, nzl + 1:] = np.conj(mf[:, nzl:0:-1])  # real profiles
+    o, g = Oracle.from_params(p, nthreads=8), QLContext(p)
+    g.set_config(NZ, WAVE, target)
+    for x in (o, g):
+        x.set_state(lin, mf)
+        x.linear_ops_init(0.0)
+    for a, b in zip(g.rhs(0.37, 0.011), o.rhs(0.37, 0.011)):
+        assert rel_err(a, b) < 1e-12
+    assert rel_err(g.drive(), o.drive()) < 1e-12
