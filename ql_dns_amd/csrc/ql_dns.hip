@@ -722,16 +722,20 @@ const double2 *mf_after_substep(const Batch &b, const Group &g, int s)
     return s == 1 ? g.mfc1 : g.mfc2;
 }
 
+// the partial rows of a set of one run without a companion launch, which its tail
+// takes as a launch argument (0: the tail reads the run table)
+int own_rows(const Group &g) { return g.nruns == 1 && g.h_rp[0].nwg2 == 0 ? g.h_rp[0].nwg : 0; }
+
 template <int NZ>
 void launch_fused_tail_t(const Group &g, const qlk::MFArgs &m, const double *part, hipStream_t st)
 {
     const dim3 grid(m.nMF, g.nruns);
     if (m.model == QL_MODEL_MHD_BQLIN) {
-        if (m.mode == qlk::MODE_CN) qlk::k_mf_fused<NZ, qlk::MODE_CN, 1><<<grid, qlk::MFF_T, 0, st>>>(m, part);
-        else qlk::k_mf_fused<NZ, qlk::MODE_ELIN, 1><<<grid, qlk::MFF_T, 0, st>>>(m, part);
+        if (m.mode == qlk::MODE_CN) qlk::k_mf_fused<NZ, qlk::MODE_CN, 1><<<grid, qlk::MFF_T, 0, st>>>(m, part, own_rows(g));
+        else qlk::k_mf_fused<NZ, qlk::MODE_ELIN, 1><<<grid, qlk::MFF_T, 0, st>>>(m, part, own_rows(g));
     } else {
-        if (m.mode == qlk::MODE_CN) qlk::k_mf_fused<NZ, qlk::MODE_CN, 0><<<grid, qlk::MFF_T, 0, st>>>(m, part);
-        else qlk::k_mf_fused<NZ, qlk::MODE_ELIN, 0><<<grid, qlk::MFF_T, 0, st>>>(m, part);
+        if (m.mode == qlk::MODE_CN) qlk::k_mf_fused<NZ, qlk::MODE_CN, 0><<<grid, qlk::MFF_T, 0, st>>>(m, part, own_rows(g));
+        else qlk::k_mf_fused<NZ, qlk::MODE_ELIN, 0><<<grid, qlk::MFF_T, 0, st>>>(m, part, own_rows(g));
     }
 }
 
@@ -787,9 +791,8 @@ int enqueue_sequence(Batch &b, Group &g, const qlk::ModeArgs &a, const qlk::MFAr
         launch_fused_tail(g, m, a.partials, st);
         QL_HIP(hipGetLastError());
     } else {
-        const int own_rows = g.nruns == 1 && g.h_rp[0].nwg2 == 0 ? g.h_rp[0].nwg : 0;
         qlk::k_reduce_cols<<<dim3((ncols + qlk::RED_CW - 1) / qlk::RED_CW, g.nruns), qlk::NT, 0, st>>>(
-            a.partials, g.rp, own_rows, ncols, const_cast<double *>(m.sums));
+            a.partials, g.rp, own_rows(g), ncols, const_cast<double *>(m.sums));
         QL_HIP(hipGetLastError());
         launch_mf(g, m, st);
         QL_HIP(hipGetLastError());

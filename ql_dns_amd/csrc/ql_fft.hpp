@@ -12,6 +12,7 @@
 // mixed-precision path).
 #pragma once
 #include <hip/hip_runtime.h>
+#include <type_traits>
 
 namespace qlk {
 

@@ -285,6 +285,21 @@ __device__ __forceinline__ void clock_advance(Clock *c)
 // with noise 6.04 -> 5.86).
 // ---------------------------------------------------------------------------
 constexpr int RED_CW = 16;  // columns per block (4, 8 and 32 measured slower)
+// Rows in flight per thread: all of a chunk's up to 256 rows.  A chunk of up to
+// RED_FEW rows (a run of up to 64) is summed without the larger batch's empty
+// places, eight FP64 instructions each of every wavefront, and chunks without
+// rows are left out: short runs' tails are bound by such instructions and by load
+// latency (100 CN steps of 16x16x32 with k_mf_fused 3.42 -> 3.08 ms, one step 113.6 ->
+// 109.8 us; zeros add nothing, so the bits stay)
+constexpr int RED_FEW = 4, RED_BATCH = 16;
+
+// s + e <- s + e + v, e the rounding errors of the running sum s
+__device__ __forceinline__ void neumaier(double &s, double &e, double v)
+{
+    const double t = s + v;
+    e += (fabs(s) >= fabs(v)) ? ((s - t) + v) : ((v - t) + s);
+    s = t;
+}
 
 [[maybe_unused]] static __global__ __launch_bounds__(NT) void k_reduce_cols(const double *__restrict__ part, const RunParams *__restrict__ runs,
                                                     int own_rows, int ncols, double *__restrict__ sums)
@@ -307,33 +322,33 @@ constexpr int RED_CW = 16;  // columns per block (4, 8 and 32 measured slower)
     const int nrows = rp.nwg + rp.nwg2;
     const int per = (nrows + CH - 1) / CH;
     const int r0 = chunk * per, r1 = min(nrows, chunk * per + per);
-    constexpr int B = 256 / CH;  // rows in flight per thread (one batch up to 256 rows)
     double s = 0.0, e = 0.0;
-    if (c < ncols) {
+    // in batches of B rows in flight; rows past r1 count as zeros, which change nothing
+    auto add_rows = [&](auto batch) {
+        constexpr int B = decltype(batch)::value;
         for (int r = r0; r < r1; r += B) {
             double v[B];
 #pragma unroll
             for (int k = 0; k < B; ++k) v[k] = (r + k < r1) ? part[(size_t)run_row(rp, r + k) * ncols + c] : 0.0;
 #pragma unroll
-            for (int k = 0; k < B; ++k) {
-                const double t = s + v[k];
-                e += (fabs(s) >= fabs(v[k])) ? ((s - t) + v[k]) : ((v[k] - t) + s);
-                s = t;
-            }
+            for (int k = 0; k < B; ++k) neumaier(s, e, v[k]);
         }
+    };
+    if (c < ncols) {
+        if (per <= RED_FEW) add_rows(std::integral_constant<int, RED_FEW>{});
+        else add_rows(std::integral_constant<int, RED_BATCH>{});
     }
     red[chunk][cl] = s;
     red2[chunk][cl] = e;
     __syncthreads();
     if (chunk == 0 && c < ncols) {
         double t = 0.0, te = 0.0;
-        for (int k = 0; k < CH; ++k) {
-            const double v = red[k][cl];
-            const double u = t + v;
-            te += (fabs(t) >= fabs(v)) ? ((t - u) + v) : ((v - u) + t);
-            te += red2[k][cl];
-            t = u;
-        }
+        for (int k0 = 0; k0 < CH && k0 * per < nrows; k0 += RED_FEW)  // the chunks that hold rows
+#pragma unroll
+            for (int k = k0; k < k0 + RED_FEW; ++k) {
+                neumaier(t, te, red[k][cl]);
+                te += red2[k][cl];
+            }
         sums[(size_t)blockIdx.y * ncols + c] = t + te;
     }
 }
@@ -720,7 +735,8 @@ __global__ __launch_bounds__(NT) void k_meanfield(MFArgs a)
 // the other fields at the substep start, which other workgroups of the launch
 // update, so the update is written to another buffer than the one read
 // (a.mf_in -> a.mf).  Substep updates with fixed steps and no CFL records only
-// (the profile maxima and HD_fullU's records combine the fields).
+// (the profile maxima and HD_fullU's records combine the fields).  A set of one
+// run passes its row count and physics as launch arguments (own_rows, a.ph1).
 // ---------------------------------------------------------------------------
 constexpr int MFF_T = 1024;          // threads per workgroup
 constexpr int RED_CH = NT / RED_CW;  // row chunks per column, as k_reduce_cols
@@ -740,7 +756,7 @@ struct MFFShared {
 };
 
 template <int NZ, int MODE, int MODEL>
-__global__ __launch_bounds__(MFF_T) void k_mf_fused(MFArgs a, const double *__restrict__ part)
+__global__ __launch_bounds__(MFF_T) void k_mf_fused(MFArgs a, const double *__restrict__ part, int own_rows)
 {
     static_assert(MODE == MODE_ELIN || MODE == MODE_CN, "substep updates");
     __shared__ MFFShared<NZ> sh;
@@ -749,10 +765,21 @@ __global__ __launch_bounds__(MFF_T) void k_mf_fused(MFArgs a, const double *__re
     constexpr int NZD = D::nz, HALF = D::half;
     constexpr int NPAIR = NZ * RED_CH;                    // (column, chunk) pairs of the field
     constexpr int NP = (NPAIR + MFF_T - 1) / MFF_T;       // pairs per thread
-    constexpr int B = 16;                                 // rows of a pair in flight
     static_assert(4 * NZD <= MFF_T && NZ <= MFF_T, "one table entry per thread");
     const int f = blockIdx.x, run = blockIdx.y, tid = threadIdx.x;
-    const RunParams &rp = a.runs[run];
+    RunParams rp;
+    if (own_rows) {
+        rp.ph = a.ph1;
+        rp.nwg = own_rows;
+        rp.wg_off = rp.wg_off2 = rp.nwg2 = 0;
+    } else {
+        const RunParams &r = a.runs[run];
+        rp.ph = r.ph;
+        rp.nwg = r.nwg;
+        rp.wg_off = r.wg_off;
+        rp.nwg2 = r.nwg2;
+        rp.wg_off2 = r.wg_off2;
+    }
     const Phys ph = rp.ph;
     const int nMF = NMF_OF(MODEL), ncols = nMF * NZ, nslot = nMF * NZD;
     const size_t mo = (size_t)run * nslot;
@@ -776,24 +803,25 @@ __global__ __launch_bounds__(MFF_T) void k_mf_fused(MFArgs a, const double *__re
         r1[q] = act ? min(nrows, r0[q] + per) : r0[q];
         s[q] = e[q] = 0.0;
     }
-    for (int j = 0; j < per; j += B) {
-        double v[NP][B];
+    auto add_rows = [&](auto batch) {
+        constexpr int B = decltype(batch)::value;
+        for (int j = 0; j < per; j += B) {
+            double v[NP][B];
 #pragma unroll
-        for (int q = 0; q < NP; ++q)
+            for (int q = 0; q < NP; ++q)
 #pragma unroll
-            for (int k = 0; k < B; ++k) {
-                const int r = r0[q] + j + k;
-                v[q][k] = r < r1[q] ? part[(size_t)run_row(rp, r) * ncols + col[q]] : 0.0;
-            }
+                for (int k = 0; k < B; ++k) {
+                    const int r = r0[q] + j + k;
+                    v[q][k] = r < r1[q] ? part[(size_t)run_row(rp, r) * ncols + col[q]] : 0.0;
+                }
 #pragma unroll
-        for (int q = 0; q < NP; ++q)
+            for (int q = 0; q < NP; ++q)
 #pragma unroll
-            for (int k = 0; k < B; ++k) {
-                const double t = s[q] + v[q][k];
-                e[q] += (fabs(s[q]) >= fabs(v[q][k])) ? ((s[q] - t) + v[q][k]) : ((v[q][k] - t) + s[q]);
-                s[q] = t;
-            }
-    }
+                for (int k = 0; k < B; ++k) neumaier(s[q], e[q], v[q][k]);
+        }
+    };
+    if (per <= RED_FEW) add_rows(std::integral_constant<int, RED_FEW>{});
+    else add_rows(std::integral_constant<int, RED_BATCH>{});
 #pragma unroll
     for (int q = 0; q < NP; ++q) {
         const int pq = tid + q * MFF_T;
@@ -812,13 +840,12 @@ __global__ __launch_bounds__(MFF_T) void k_mf_fused(MFArgs a, const double *__re
     __syncthreads();
     if (tid < NZ) {
         double t = 0.0, te = 0.0;
-        for (int k = 0; k < RED_CH; ++k) {
-            const double v = sh.red[k][tid];
-            const double u = t + v;
-            te += (fabs(t) >= fabs(v)) ? ((t - u) + v) : ((v - u) + t);
-            te += sh.red2[k][tid];
-            t = u;
-        }
+        for (int k0 = 0; k0 < RED_CH && k0 * per < nrows; k0 += RED_FEW)  // the chunks that hold rows
+#pragma unroll
+            for (int k = k0; k < k0 + RED_FEW; ++k) {
+                neumaier(t, te, sh.red[k][tid]);
+                te += sh.red2[k][tid];
+            }
         sh.ssum[tid] = t + te;
     }
     __syncthreads();

@@ -163,3 +163,23 @@ def test_fused_tail_refusals():
     with pytest.raises(QLError):
         c.set_tail(64, 1)  # no such group
     c.close()
+
+
+@pytest.mark.parametrize("rows", [1, 16, 17, 63, 64, 65, 120])
+def test_partial_row_counts_match_oracle(rows):
+    """Both tails over row counts at the edges of the summation's 16 chunks and of
+    the small batch (64 rows): states and drives within the shapes' bar against the
+    oracle, 1e-10, and bitwise equal between the tails."""
+    from ql_dns_amd.ic import initial_state
+    from oracle.oracle import Oracle
+    p = _p(NX=16, NY=16, NZ=32, Ly=1.0)  # 120 modes
+    out = [_run(p, tail, n=4, shape=(64, rows)) for tail in (1, 0)]
+    _equal(*out)
+    o = Oracle.from_params(p, nthreads=4)
+    o.set_state(*initial_state(p))
+    o.linear_ops_init(0.0)
+    assert o.steps(4, 0.0) == out[0][0]
+    lin, mf, kx0 = o.get_state()
+    assert np.array_equal(out[0][3], kx0)
+    for got, want in ((out[0][1], lin), (out[0][2], mf), (out[0][4], o.drive())):
+        assert rel_err(got, want) < 1e-10
