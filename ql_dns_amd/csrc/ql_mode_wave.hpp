@@ -366,6 +366,28 @@ __device__ __forceinline__ void mode_wave_body(const ModeArgs &a)
 
     const WgInfo wgi = a.wg[blockIdx.x];
     const int run = wgi.run, g0 = wgi.g0, g1 = wgi.g1, mode_off = wgi.mode_off;
+    // AHEAD: a mode's loads, F's of the previous RHS included, at the end of the
+    // mode before it, the first ahead of the tables, and the state held for F.  At
+    // one slot per lane, where few modes per wavefront leave latency the bound and
+    // the registers are there (100 CN steps of 36x60x64 MHD_BQlin with noise 5.93 ->
+    // 5.75 ms, the gradient of 200 steps of 32x32x64 30.05 -> 29.48); with more
+    // slots they are not (200 steps of 64x128x128 21.8 -> 27.9 ms)
+    constexpr bool AHEAD = KI == 1 && (!SPL || MIXW);
+    double kxl = 0.0, kyl = 0.0;
+    double2 ua[4], na[4];
+    auto load_ahead = [&](int l) {
+        const int i = mode_off + l;
+        kxl = a.kx0[i];
+        kyl = a.ky[i];
+        const size_t o = (size_t)i * 4 * NZD + min(lane, NZD - 1);
+#pragma unroll
+        for (int f = 0; f < 2 * P::NPAIR; ++f) {
+            ua[f] = a.u[o + f * NZD];
+            na[f] = a.n_prev ? a.n_prev[o + f * NZD] : make_double2(0.0, 0.0);
+        }
+    };
+    if constexpr (AHEAD)
+        if (g0 + wave < g1) load_ahead(g0 + wave);
     const RunParams rp = a.runs[run];
     const Phys ph = rp.ph;
     const SubTimes st = sub_times<MODE == MODE_CN>(a, run);
@@ -451,7 +473,7 @@ __device__ __forceinline__ void mode_wave_body(const ModeArgs &a)
             // mode loop instead of in registers across it
             int ln = lane;
             if constexpr (ROWS || NZ >= 256) asm volatile("" : "+v"(ln));
-            const double kx0 = to_sgpr(a.kx0[i]), ky = to_sgpr(a.ky[i]);
+            const double kx0 = to_sgpr(AHEAD ? kxl : a.kx0[i]), ky = to_sgpr(AHEAD ? kyl : a.ky[i]);
             const double kx = to_sgpr(rn_add(kx0, rn_mul(qt, ky)));  // kx(t), MHD_FullQlin.cpp:727
             const size_t row = (size_t)i * 4 * NZD;
 
@@ -463,7 +485,11 @@ __device__ __forceinline__ void mode_wave_body(const ModeArgs &a)
             for (int k = 0; k < KI; ++k) {
                 const size_t o = row + min(lane + k * WAVE, NZD - 1);
     #pragma unroll
-                for (int f = 0; f < 4; ++f) ub[k][f] = f < 2 * P::NPAIR ? a.u[o + f * NZD] : make_double2(0.0, 0.0);
+                for (int f = 0; f < 4; ++f) {
+                    if (f >= 2 * P::NPAIR) ub[k][f] = make_double2(0.0, 0.0);
+                    else if constexpr (AHEAD) ub[k][f] = ua[f];
+                    else ub[k][f] = a.u[o + f * NZD];
+                }
             }
     #pragma unroll
             for (int k = 0; k < KI; ++k) {
@@ -598,6 +624,15 @@ __device__ __forceinline__ void mode_wave_body(const ModeArgs &a)
                     }
     #pragma unroll
                     for (int f = 0; f < 2 * P::NPAIR; ++f) np[f] = nf[k][f];
+                } else if constexpr (AHEAD) {
+                    U0 = ua[0];
+                    U1 = ua[1];
+                    if constexpr (P::NPAIR == 2) {
+                        U2 = ua[2];
+                        U3 = ua[3];
+                    }
+    #pragma unroll
+                    for (int f = 0; f < 2 * P::NPAIR; ++f) np[f] = na[f];
                 } else {
                     U0 = a.u[off];
                     U1 = a.u[off + NZD];
@@ -678,6 +713,8 @@ __device__ __forceinline__ void mode_wave_body(const ModeArgs &a)
         } else {
             pass(C{}, buf, tw, skzr, smfz);
         }
+        if constexpr (AHEAD)
+            if (l + NW < g1) load_ahead(l + NW);
         // the next mode's B overwrites the transformed products F read
         wave_sync();
     }

@@ -165,14 +165,15 @@ def test_fused_tail_refusals():
     c.close()
 
 
-@pytest.mark.parametrize("rows", [1, 16, 17, 63, 64, 65, 120])
-def test_partial_row_counts_match_oracle(rows):
+@pytest.mark.parametrize("NZ,rows", [(32, r) for r in (1, 16, 17, 63, 64, 65, 120)] + [(64, 1), (64, 3), (64, 13)])
+def test_partial_row_counts_match_oracle(NZ, rows):
     """Both tails over row counts at the edges of the summation's 16 chunks and of
-    the small batch (64 rows): states and drives within the shapes' bar against the
-    oracle, 1e-10, and bitwise equal between the tails."""
+    the small batch (64 rows), and the mode kernel's loads ahead over several modes
+    of a wavefront, the last of them not in every wavefront: states and drives within
+    the shapes' bar against the oracle, 1e-10, and bitwise equal between the tails."""
     from ql_dns_amd.ic import initial_state
     from oracle.oracle import Oracle
-    p = _p(NX=16, NY=16, NZ=32, Ly=1.0)  # 120 modes
+    p = _p(NX=16, NY=16, NZ=NZ, Ly=1.0)  # 120 modes
     out = [_run(p, tail, n=4, shape=(64, rows)) for tail in (1, 0)]
     _equal(*out)
     o = Oracle.from_params(p, nthreads=4)
