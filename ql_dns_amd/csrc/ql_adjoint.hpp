@@ -124,7 +124,8 @@ static __device__ __noinline__ double noise_q_gradient(NoiseParams np, double q,
     const double nf = rn_mul(dt, np.nfac);
     const double mu = sqrt(rn_mul(nf, lap2n) / lapF);
     double2 z[4];
-    noise_normals(np.seed, tn, mode, slot, z);
+    noise_normals(np.seed, tn, mode, slot, 0, z);
+    noise_normals(np.seed, tn, mode, slot, 1, z + 2);
     double gz = 0.0;
     if (np.drive_u) gz += redot(z[0], gux);
     if (np.drive_b) gz += redot(z[2], gbx);

@@ -688,7 +688,7 @@ int launch_noise(Group &g, double2 *u, bool use_clock, double t, double dt, bool
     a.kzv = g.kzv;
     a.runs = g.rp;
     a.np = g.np;
-    a.mode_run = g.mode_run;
+    a.mode_run = g.nruns == 1 ? nullptr : g.mode_run;
     a.clock = g.clock;
     a.nz = g.nz;
     a.use_clock = use_clock ? 1 : 0;
@@ -696,7 +696,7 @@ int launch_noise(Group &g, double2 *u, bool use_clock, double t, double dt, bool
     a.do_remap = remap ? 1 : 0;
     a.t_x = t;
     a.dt_x = dt;
-    const int threads = (g.nz + 63) / 64 * 64;  // one thread per kz slot (nz <= 171)
+    const int threads = (2 * g.nz + 63) / 64 * 64;  // one per kz slot and field pair (nz <= 171)
     qlk::k_noise_remap<<<g.modes, threads, 0, st>>>(a);
     QL_HIP(hipGetLastError());
     return QL_OK;
