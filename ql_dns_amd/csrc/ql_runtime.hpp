@@ -205,7 +205,11 @@ template <typename T>
 int dalloc(T **p, size_t n)
 {
     QL_HIP(hipMalloc((void **)p, sizeof(T) * (n ? n : 1)));
+    // the clearing runs on the null stream, which the contexts' streams (created
+    // hipStreamNonBlocking) do not wait for: without the wait it could land after
+    // the first copy into the buffer
     QL_HIP(hipMemset(*p, 0, sizeof(T) * (n ? n : 1)));
+    QL_HIP(hipStreamSynchronize(nullptr));
     return QL_OK;
 }
 
