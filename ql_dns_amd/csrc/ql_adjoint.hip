@@ -16,6 +16,7 @@
 
 #include "ql_adjoint.hpp"
 #include "ql_runtime.hpp"
+#include "ql_state_out.hpp"
 
 namespace qlh {
 
@@ -440,21 +441,9 @@ int adjoint_backward(Batch &b, const double *g_lin, const double *g_mf, double *
     QL_RC(launch_adj_mf(NZ, b.model, aa, b.s));
     // leave the context at the forward's final state
     QL_RC(load_ck(b, A->ck[A->nseg], g.u, g.mf, g.mfz));
-    if (b.hd) {
-        QL_HIP(hipStreamSynchronize(b.s));
-        QL_HIP(hipMemcpy(hl.data(), A->gu, sizeof(double2) * nl, hipMemcpyDeviceToHost));
-        QL_HIP(hipMemcpy(hm.data(), A->gM, sizeof(double2) * nm, hipMemcpyDeviceToHost));
-        if (g_lin0)
-            for (int i = 0; i < nxy; ++i)
-                std::memcpy(g_lin0 + (size_t)i * 2 * nz * 2, &hl[(size_t)i * 4 * nz], sizeof(double2) * 2 * nz);
-        if (g_mf0) std::memcpy(g_mf0, &hm[(size_t)2 * nz], sizeof(double2) * 2 * nz);
-    } else {
-        if (g_lin0) QL_HIP(hipMemcpyAsync(g_lin0, A->gu, sizeof(double2) * nl, hipMemcpyDeviceToHost, b.s));
-        if (g_mf0) QL_HIP(hipMemcpyAsync(g_mf0, A->gM, sizeof(double2) * nm, hipMemcpyDeviceToHost, b.s));
-    }
     double gp[qlk::NGP];
-    QL_HIP(hipMemcpyAsync(gp, A->gpar, sizeof(double) * qlk::NGP, hipMemcpyDeviceToHost, b.s));
-    QL_HIP(hipStreamSynchronize(b.s));
+    QL_RC(state_out(*b.out, b.s, A->gu, nxy, ext_nlin(b) * nz, 4 * nz, g_lin0, A->gM + (size_t)ext_mf0(b) * nz,
+                    ext_nmf(b) * nz, g_mf0, A->gpar, qlk::NGP, gp));
     if (b.hd) gp[3] = gp[4] = 0.0;  // HD_fullU has no eta and no B0z
     if (b.model == QL_MODEL_MHD_BQLIN) {
         // MHD_BQlin rotates at 2 q / 3 whatever omega is (MHD_BQlin.cpp:19): the

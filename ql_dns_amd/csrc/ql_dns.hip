@@ -26,6 +26,7 @@
 #include "ql_mode.hpp"
 #include "ql_mode_wave.hpp"
 #include "ql_runtime.hpp"
+#include "ql_state_out.hpp"
 
 namespace qlh {
 
@@ -65,6 +66,8 @@ void release(Batch &b)
         g.s = nullptr;
     }
     dfree(b.dpart), dfree(b.dout), dfree(b.mfr_tmp);
+    delete b.out;
+    b.out = nullptr;
     for (auto &e : b.ev)
         if (e) (void)hipEventDestroy(e), e = nullptr;
     for (hipEvent_t e : b.tpool) (void)hipEventDestroy(e);
@@ -353,6 +356,12 @@ int create_batch(Batch &b, const ql_params *ps, int nruns)
     QL_RC(dalloc(&b.dpart, (size_t)256 * 6));
     QL_RC(dalloc(&b.dout, (size_t)18));
     QL_RC(dalloc(&b.mfr_tmp, (size_t)4 * 256));
+    size_t lin = 0, tail = sizeof(double) * 4 * 256;
+    for (const RunInfo &r : b.runs) {
+        lin = std::max(lin, sizeof(double2) * r.nxy * ext_nlin(b) * r.nz);
+        tail = std::max(tail, sizeof(double2) * 4 * r.nz + sizeof(double) * std::max(r.nxy, qlk::NT));
+    }
+    QL_RC(staging_create(&b.out, lin, tail));
     for (Group &g : b.groups) {
         if (b.groups.size() > 1) {
             QL_HIP(hipStreamCreateWithFlags(&g.s, hipStreamNonBlocking));
@@ -1044,12 +1053,6 @@ int run_steps(Batch &b, int nsteps, double *t_runs)
     return QL_OK;
 }
 
-// the caller's layout: fluctuation fields per mode, mean fields, and the
-// first internal mean-field slot the caller's mean field 0 is
-int ext_nlin(const Batch &b) { return b.hd ? 2 : 4; }
-int ext_nmf(const Batch &b) { return b.hd ? 2 : b.nMF; }
-int ext_mf0(const Batch &b) { return b.hd ? 2 : 0; }
-
 // [modes][4][nz] <-> [modes][nL][nz] (the internal slots past nL are zero)
 template <class T>
 void lin_to_int(const T *src, T *dst, int modes, int nL, int nz)
@@ -1138,19 +1141,8 @@ int get_state(Batch &b, int run, double *lin, double *mf, double *kx0)
     const RunInfo &r = b.runs[run];
     Group &g = b.groups[r.group];
     const size_t mo = (size_t)r.gi * b.nMF * g.nz;
-    std::vector<double2> tl(b.hd && lin ? (size_t)r.nxy * 4 * g.nz : 0);
-    double2 *dl = b.hd ? tl.data() : reinterpret_cast<double2 *>(lin);
-    if (lin)
-        QL_HIP(hipMemcpyAsync(dl, g.u + (size_t)r.mode_off * 4 * g.nz, sizeof(double2) * (size_t)r.nxy * 4 * g.nz,
-                              hipMemcpyDeviceToHost, b.s));
-    if (mf)
-        QL_HIP(hipMemcpyAsync(mf, g.mf + mo + (size_t)ext_mf0(b) * g.nz, sizeof(double2) * ext_nmf(b) * g.nz,
-                              hipMemcpyDeviceToHost, b.s));
-    if (kx0)
-        QL_HIP(hipMemcpyAsync(kx0, g.kx0 + r.mode_off, sizeof(double) * r.nxy, hipMemcpyDeviceToHost, b.s));
-    QL_HIP(hipStreamSynchronize(b.s));
-    if (b.hd && lin) lin_to_ext(tl.data(), reinterpret_cast<double2 *>(lin), r.nxy, 2, g.nz);
-    return QL_OK;
+    return state_out(*b.out, b.s, g.u + (size_t)r.mode_off * 4 * g.nz, r.nxy, ext_nlin(b) * g.nz, 4 * g.nz, lin,
+                     g.mf + mo + (size_t)ext_mf0(b) * g.nz, ext_nmf(b) * g.nz, mf, g.kx0 + r.mode_off, r.nxy, kx0);
 }
 
 int diagnostics(Batch &b, int run, double t, double out[18])
@@ -1191,8 +1183,7 @@ int diagnostics(Batch &b, int run, double t, double out[18])
     f.out = b.dout;
     qlk::k_diag_final<<<1, qlk::NT, 0, b.s>>>(f);
     QL_HIP(hipGetLastError());
-    QL_HIP(hipMemcpyAsync(out, b.dout, sizeof(double) * 18, hipMemcpyDeviceToHost, b.s));
-    QL_HIP(hipStreamSynchronize(b.s));
+    QL_RC(state_out(*b.out, b.s, nullptr, 0, 1, 1, nullptr, nullptr, 0, nullptr, b.dout, 18, out));
     if (r.hd) {
         // HD_fullU.cpp:463-488: no magnetic quantities, Reynolds stresses are
         // saved as full profiles (ql_drive_real) instead of projections
@@ -1446,9 +1437,7 @@ int profiles_real(Batch &b, const double2 *v, const Group &g, double *out)
     default: qlk::k_mf_real<256><<<1, qlk::NT, 0, b.s>>>(v, n, g.tw, fac, b.mfr_tmp); break;
     }
     QL_HIP(hipGetLastError());
-    QL_HIP(hipMemcpyAsync(out, b.mfr_tmp, sizeof(double) * n * g.NZ, hipMemcpyDeviceToHost, b.s));
-    QL_HIP(hipStreamSynchronize(b.s));
-    return QL_OK;
+    return state_out(*b.out, b.s, nullptr, 0, 1, 1, nullptr, nullptr, 0, nullptr, b.mfr_tmp, n * g.NZ, out);
 }
 
 }  // namespace qlh
@@ -1846,10 +1835,8 @@ int ql_batch_get_drive(ql_batch *bt, int run, double *drive)
     Batch &b = bt->b;
     const RunInfo &r = b.runs[run];
     Group &g = b.groups[r.group];
-    QL_HIP(hipMemcpyAsync(drive, g.drive + (size_t)(r.gi * b.nMF + ext_mf0(b)) * g.nz,
-                          sizeof(double2) * ext_nmf(b) * g.nz, hipMemcpyDeviceToHost, b.s));
-    QL_HIP(hipStreamSynchronize(b.s));
-    return QL_OK;
+    return state_out(*b.out, b.s, nullptr, 0, 1, 1, nullptr, g.drive + (size_t)(r.gi * b.nMF + ext_mf0(b)) * g.nz,
+                     ext_nmf(b) * g.nz, drive, nullptr, 0, nullptr);
 }
 
 int ql_batch_calculate_cfl(ql_batch *bt, int run, double *cfl_over_dt)

@@ -164,6 +164,8 @@ constexpr double TUNE_WARM_MS = 25.0;
 
 struct AdjState;  // adjoint checkpoints and buffers (ql_adjoint.hip)
 
+struct Staging;  // ql_state_out.hpp
+
 struct Batch {
     int model = 0, integrator = 0, precision = 0, device = 0, nMF = 4;
     double amp_tau = MIXED_AMP_TAU;  // mixed precision: FP64 from this fraction of a run's largest mode
@@ -199,6 +201,7 @@ struct Batch {
     std::vector<hipEvent_t> tpool;
     size_t tused = 0;
     AdjState *adj = nullptr;
+    Staging *out = nullptr;  // pinned memory results leave through
 };
 
 template <typename T>
@@ -237,6 +240,11 @@ int enqueue_substep(Batch &b, Group &g, int s, bool remap_after, bool advance, h
 void launch_mf(const Group &g, const qlk::MFArgs &m, hipStream_t st);
 int launch_noise(Group &g, double2 *u, bool use_clock, double t, double dt, bool noise, bool remap, hipStream_t st);
 qlk::MFArgs mf_args(const Batch &b, const Group &g);
+// the caller's layout: fluctuation fields per mode, mean fields, and the
+// first internal mean-field slot the caller's mean field 0 is
+inline int ext_nlin(const Batch &b) { return b.hd ? 2 : 4; }
+inline int ext_nmf(const Batch &b) { return b.hd ? 2 : b.nMF; }
+inline int ext_mf0(const Batch &b) { return b.hd ? 2 : 0; }
 int refresh_profiles(Batch &b, Group &g, hipStream_t st, bool rec = false);
 int run_steps(Batch &b, int nsteps, double *t_inout);
 // defined in ql_adjoint.hip

@@ -183,3 +183,30 @@ def test_batch_bad_run_index():
         b.get_state(-1)
     with pytest.raises(QLError):
         b.set_config(256, 256, 512)  # no NZ=256 run in this set
+
+
+@pytest.mark.parametrize("model,NX,NY,NZ", [(0, 2, 2, 32), (0, 32, 32, 64), (1, 36, 60, 64), (0, 64, 64, 64),
+                                            (0, 64, 128, 128), (2, 8, 8, 32), (2, 64, 64, 128), (2, 64, 128, 128)])
+def test_states_come_back_as_they_went(model, NX, NY, NZ):
+    """Downloads in one, two, several and more than eight pieces (2 MiB each), HD_fullU's
+    two fields out of the internal four, and from two threads on one context: bit for
+    bit what was uploaded."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    from ql_dns_amd.capi import QLContext
+    from ql_dns_amd.ic import mode_tables
+    from ql_dns_amd.params import QLParams
+    p = QLParams(model=model, NX=NX, NY=NY, NZ=NZ)
+    c = QLContext(p)
+    rng = np.random.default_rng(NX * NZ + model)
+    lin, mf, kx0 = c.get_state()
+    lin = rng.standard_normal(lin.shape) + 1j * rng.standard_normal(lin.shape)
+    lin[mode_tables(p)[1] == 0, ::2, 0] = 0.0  # the compressive slots
+    mf = rng.standard_normal(mf.shape) + 1j * rng.standard_normal(mf.shape)
+    kx0 = kx0 + rng.standard_normal(kx0.shape)
+    c.set_state(lin, mf, kx0)
+    with ThreadPoolExecutor(2) as pool:
+        for got in [f.result() for f in [pool.submit(c.get_state) for _ in range(4)]]:
+            for x, y in zip(got, (lin, mf, kx0)):
+                assert np.array_equal(x, y)
+    c.close()
