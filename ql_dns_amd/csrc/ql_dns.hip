@@ -641,22 +641,37 @@ void set_split(const Batch &b, const Group &g, qlk::ModeArgs &a)
     a.hi = g.hi;
 }
 
-// the precision flags from the mode amplitudes of the current state: always
-// (clocked = false: after the state changed outside the steps), or inside a
-// step when the group's clock is at a multiple of SPLIT_EVERY steps
-void launch_flags(const Batch &b, const Group &g, bool clocked, hipStream_t st)
+// the precision flags from the mode amplitudes of the current state
+int launch_flags(const Batch &b, const Group &g, hipStream_t st)
 {
-    const qlk::Clock *ck = clocked ? g.clock : nullptr;
-    qlk::k_amp_modes<<<g.modes, 64, 0, st>>>(g.u, g.nz, g.amp, ck, SPLIT_EVERY);
-    qlk::k_amp_flags<<<g.nruns, qlk::AMP_NT, 0, st>>>(g.amp, g.rp, b.amp_tau, g.hi, ck, SPLIT_EVERY);
+    qlk::k_amp_modes<<<g.modes, 64, 0, st>>>(g.u, g.nz, g.amp);
+    qlk::k_amp_flags<<<g.nruns, qlk::AMP_NT, 0, st>>>(g.amp, g.rp, b.amp_tau, g.hi);
+    QL_HIP(hipGetLastError());
+    return QL_OK;
 }
 
 int prime_split(Batch &b, Group &g, hipStream_t st)
 {
     if (!split_active(b, g) || !g.amp_stale) return QL_OK;
-    launch_flags(b, g, false, st);
-    QL_HIP(hipGetLastError());
+    QL_RC(launch_flags(b, g, st));
     g.amp_stale = false;
+    return QL_OK;
+}
+
+// Before step n (steps since the integrator was set up) the flags are set again
+// where n is a multiple of SPLIT_EVERY; returns how many of nsteps steps may
+// follow before the next time.  The host counts the steps, so the launches stand
+// between replays (inside the replay graphs, where each step had to look at the
+// device clock, the two launches took 4 us of every step: 64 steps of
+// 128x128x256 25.0 -> 24.8 ms).
+int set_flags(Batch &b, int n, int nsteps, int *run)
+{
+    *run = nsteps;
+    for (Group &g : b.groups) {
+        if (!split_active(b, g)) continue;
+        if (n % SPLIT_EVERY == 0) QL_RC(launch_flags(b, g, b.s));
+        *run = std::min(nsteps, SPLIT_EVERY - n % SPLIT_EVERY);
+    }
     return QL_OK;
 }
 
@@ -885,15 +900,11 @@ int enqueue_substep(Batch &b, Group &g, int s, bool remap_after, bool advance, h
 }
 
 // nsteps whole steps (main.cpp:108-123, noise off: Step, t += dt when advance
-// is set, remap) of one group: with mixed precision the clocked flag refresh,
-// then the substeps
+// is set, remap) of one group
 int enqueue_group_steps(Batch &b, Group &g, int nsteps, bool remap, bool advance, hipStream_t st)
 {
-    for (int n = 0; n < nsteps; ++n) {
-        if (split_active(b, g)) launch_flags(b, g, true, st);
-        QL_HIP(hipGetLastError());
+    for (int n = 0; n < nsteps; ++n)
         for (int s = 1; s <= 3; ++s) QL_RC(enqueue_substep(b, g, s, remap && s == 3, advance, st));
-    }
     return QL_OK;
 }
 
@@ -923,7 +934,6 @@ int set_clock(Batch &b, double t)
     c.t_prev = b.t_prev;
     c.t_init = b.t_init;
     c.old_init = b.old_init;
-    c.nstep = b.nstep;
     c.dt = b.dt;
     c.dt_last = b.dt_last;
     for (Group &g : b.groups)
@@ -947,7 +957,6 @@ int set_clock_runs(Batch &b, const double *t_runs)
             c.t_prev = b.rt_prev[r];
             c.t_init = b.t_init;
             c.old_init = b.old_init;
-            c.nstep = b.nstep;
             c.dt = b.dt;
             c.dt_last = b.rdt_last[r];
         }
@@ -1019,11 +1028,14 @@ int run_steps(Batch &b, int nsteps, double *t_runs)
     if (per_run) QL_RC(set_clock_runs(b, t_runs));
     else QL_RC(set_clock(b, t));
     QL_RC(prime_split_all(b));
-    if (b.timing) {
-        QL_RC(enqueue_steps(b, nsteps, true, true));
-    } else if (nsteps > 0) {
-        QL_RC(ensure_graphs(b));
-        int left = nsteps;
+    if (!b.timing && nsteps > 0) QL_RC(ensure_graphs(b));
+    for (int done = 0, n = 0; done < nsteps; done += n) {
+        QL_RC(set_flags(b, b.nstep + done, nsteps - done, &n));
+        if (b.timing) {
+            QL_RC(enqueue_steps(b, n, true, true));
+            continue;
+        }
+        int left = n;
         for (int k = 0; k < 5; ++k)
             for (; left >= GRAPH_LEVELS[k]; left -= GRAPH_LEVELS[k]) QL_HIP(hipGraphLaunch(b.graphs[k], b.s));
     }
@@ -1594,6 +1606,8 @@ int ql_step(ql_ctx *c, double t, double *dt_out)
     Batch &b = c->bt.b;
     QL_RC(set_clock(b, t));
     QL_RC(prime_split_all(b));
+    int one = 1;
+    QL_RC(set_flags(b, b.nstep, 1, &one));
     QL_RC(enqueue_steps(b, 1, false, false));
     b.t_prev = t;
     b.old_init = 0;

@@ -82,7 +82,7 @@ struct WgInfo {
 // taken, dt_last the one taken last
 struct Clock {
     double t, t_prev, t_init;
-    int old_init, nstep;  // nstep: steps since the integrator was set up
+    int old_init;
     double dt, dt_last;
 };
 
@@ -270,7 +270,6 @@ __device__ __forceinline__ void clock_advance(Clock *c)
     c->t = rn_add(t, dt);
     c->dt_last = dt;
     c->old_init = 0;
-    c->nstep += 1;
 }
 
 // ---------------------------------------------------------------------------
@@ -353,13 +352,10 @@ __device__ __forceinline__ void neumaier(double &s, double &e, double v)
     }
 }
 
-// mixed precision: every `every` steps of the clock (always when clock is
-// null), max |value| of each mode's state, one wavefront per mode
+// mixed precision: max |value| of each mode's state, one wavefront per mode
 [[maybe_unused]] static __global__ __launch_bounds__(64) void k_amp_modes(const double2 *__restrict__ u, int nz,
-                                                                          float *__restrict__ amp,
-                                                                          const Clock *__restrict__ clock, int every)
+                                                                          float *__restrict__ amp)
 {
-    if (clock && clock->nstep % every != 0) return;
     const size_t i = blockIdx.x;
     float m = 0.0f;
     for (int k = threadIdx.x; k < 2 * nz; k += 64) m = fmaxf(m, amp2(u[i * 4 * nz + k], u[i * 4 * nz + 2 * nz + k]));
@@ -372,10 +368,8 @@ __device__ __forceinline__ void neumaier(double &s, double &e, double v)
 constexpr int AMP_NT = 1024;
 [[maybe_unused]] static __global__ __launch_bounds__(AMP_NT) void k_amp_flags(const float *__restrict__ amp,
                                                                              const RunParams *__restrict__ runs,
-                                                                             double tau, unsigned char *__restrict__ hi,
-                                                                             const Clock *__restrict__ clock, int every)
+                                                                             double tau, unsigned char *__restrict__ hi)
 {
-    if (clock && clock->nstep % every != 0) return;
     __shared__ float red[AMP_NT / 64];
     const RunParams &rp = runs[blockIdx.x];
     const int tid = threadIdx.x;

@@ -151,7 +151,7 @@ struct Group {
 // fraction of its run's largest (measured at 128x128x256 over 2000 steps: 29
 // of 8128 modes in FP64 and the mean fields, drives and energies within 3e-9
 // of the FP64 run, against 1.7e-6 with every mode in FP32); the flags are
-// set again every SPLIT_EVERY steps of the clock (a mode's amplitude changes
+// set again every SPLIT_EVERY steps (a mode's amplitude changes
 // by a few per cent over that many steps) and after a state upload.  Remaps
 // and driving noise leave them: a zeroed mode gives zeros in either
 // precision, and the noise is small against the modes that set the flags
@@ -169,7 +169,7 @@ struct Staging;  // ql_state_out.hpp
 struct Batch {
     int model = 0, integrator = 0, precision = 0, device = 0, nMF = 4;
     double amp_tau = MIXED_AMP_TAU;  // mixed precision: FP64 from this fraction of a run's largest mode
-    int nstep = 0;                   // steps since the integrator was set up (the device clock's count)
+    int nstep = 0;                   // steps since the integrator was set up
     // HD_fullU runs on the MHD_FullQlin kernels with the magnetic fields zero;
     // at the boundary they have 2 fluctuation fields (u, zeta) and 2 mean
     // fields (Ux, Uy, internal slots 2 and 3)
