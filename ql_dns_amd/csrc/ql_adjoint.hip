@@ -117,11 +117,9 @@ int load_ck(Batch &b, const AdjState::Ck &c, double2 *u, double2 *mf, double *mf
     b.dt_last = c.dt_last;
     b.old_init = c.old_init;
     qlk::MFArgs m = mf_args(b, g);
-    m.mode = qlk::MODE_PROFILES;
     m.mf = mf;
     m.mfz = mfz;
-    m.mfn_out = g.mfN1;
-    launch_mf(g, m, b.s);
+    launch_profiles(b, g, m, b.s);
     QL_HIP(hipGetLastError());
     return QL_OK;
 }

@@ -420,7 +420,7 @@ int create_batch(Batch &b, const ql_params *ps, int nruns)
         QL_HIP(hipMemcpy(g.kzv, r0.h_kz.data(), sizeof(double) * g.nz, hipMemcpyHostToDevice));
         QL_HIP(hipMemcpy(g.tw, htw.data(), sizeof(double2) * g.NZ, hipMemcpyHostToDevice));
         QL_HIP(hipMemcpy(g.tw32, htw32.data(), sizeof(float2) * g.NZ, hipMemcpyHostToDevice));
-        const Shape sh = default_shape(g.NZ, b.model, b.precision, g.nruns, g.modes);
+        const Shape sh = default_shape(g.NZ, b.precision, g.nruns, g.modes);
         QL_RC(configure(b, g, sh.line, sh.target));
         g.tail = sh.tail;
         for (const qlk::RunParams &rp : g.h_rp)
@@ -751,25 +751,36 @@ const double2 *mf_after_substep(const Batch &b, const Group &g, int s)
 int own_rows(const Group &g) { return g.nruns == 1 && g.h_rp[0].nwg2 == 0 ? g.h_rp[0].nwg : 0; }
 
 template <int NZ>
-void launch_fused_tail_t(const Group &g, const qlk::MFArgs &m, const double *part, hipStream_t st)
+void launch_fused_tail_t(const Group &g, const qlk::MFArgs &m, bool cn, const double *part, hipStream_t st)
 {
     const dim3 grid(m.nMF, g.nruns);
     if (m.model == QL_MODEL_MHD_BQLIN) {
-        if (m.mode == qlk::MODE_CN) qlk::k_mf_fused<NZ, qlk::MODE_CN, 1><<<grid, qlk::MFF_T, 0, st>>>(m, part, own_rows(g));
+        if (cn) qlk::k_mf_fused<NZ, qlk::MODE_CN, 1><<<grid, qlk::MFF_T, 0, st>>>(m, part, own_rows(g));
         else qlk::k_mf_fused<NZ, qlk::MODE_ELIN, 1><<<grid, qlk::MFF_T, 0, st>>>(m, part, own_rows(g));
     } else {
-        if (m.mode == qlk::MODE_CN) qlk::k_mf_fused<NZ, qlk::MODE_CN, 0><<<grid, qlk::MFF_T, 0, st>>>(m, part, own_rows(g));
+        if (cn) qlk::k_mf_fused<NZ, qlk::MODE_CN, 0><<<grid, qlk::MFF_T, 0, st>>>(m, part, own_rows(g));
         else qlk::k_mf_fused<NZ, qlk::MODE_ELIN, 0><<<grid, qlk::MFF_T, 0, st>>>(m, part, own_rows(g));
     }
 }
 
-void launch_fused_tail(const Group &g, const qlk::MFArgs &m, const double *part, hipStream_t st)
+void launch_fused_tail(const Group &g, const qlk::MFArgs &m, bool cn, const double *part, hipStream_t st)
 {
     switch (g.NZ) {
-    case 32: launch_fused_tail_t<32>(g, m, part, st); break;
-    case 64: launch_fused_tail_t<64>(g, m, part, st); break;
-    default: launch_fused_tail_t<128>(g, m, part, st); break;
+    case 32: launch_fused_tail_t<32>(g, m, cn, part, st); break;
+    case 64: launch_fused_tail_t<64>(g, m, cn, part, st); break;
+    default: launch_fused_tail_t<128>(g, m, cn, part, st); break;
     }
+}
+
+// the real-space profiles of the mean fields m.mf (and with m.rec their maxima):
+// in the kernel that forms them in a substep, so that they have its bits
+void launch_profiles(const Batch &b, const Group &g, qlk::MFArgs m, hipStream_t st)
+{
+    m.mode = qlk::MODE_PROFILES;
+    m.mfn_out = g.mfN1;
+    const bool lines = b.model == QL_MODEL_MHD_BQLIN && fused_tail(b, g);
+    if (!lines || m.rec) launch_mf(g, m, st);
+    if (lines) launch_fused_tail(g, m, b.integrator == QL_INT_RK3CN, nullptr, st);
 }
 
 // mode kernel -> column reduction of its partials -> mean-field kernel; the
@@ -812,7 +823,7 @@ int enqueue_sequence(Batch &b, Group &g, const qlk::ModeArgs &a, const qlk::MFAr
     }
     tm_cur = LaunchTiming{};
     if (fused_tail(b, g) && (m.mode == qlk::MODE_ELIN || m.mode == qlk::MODE_CN)) {
-        launch_fused_tail(g, m, a.partials, st);
+        launch_fused_tail(g, m, m.mode == qlk::MODE_CN, a.partials, st);
         QL_HIP(hipGetLastError());
     } else {
         qlk::k_reduce_cols<<<dim3((ncols + qlk::RED_CW - 1) / qlk::RED_CW, g.nruns), qlk::NT, 0, st>>>(
@@ -828,10 +839,8 @@ int enqueue_sequence(Batch &b, Group &g, const qlk::ModeArgs &a, const qlk::MFAr
 int refresh_profiles(Batch &b, Group &g, hipStream_t st, bool rec)
 {
     qlk::MFArgs m = mf_args(b, g);
-    m.mode = qlk::MODE_PROFILES;
     if (rec) m.rec = 1;
-    m.mfn_out = g.mfN1;
-    launch_mf(g, m, st);
+    launch_profiles(b, g, m, st);
     QL_HIP(hipGetLastError());
     return QL_OK;
 }

@@ -731,6 +731,10 @@ __global__ __launch_bounds__(NT) void k_meanfield(MFArgs a)
 // (a.mf_in -> a.mf).  Substep updates with fixed steps and no CFL records only
 // (the profile maxima and HD_fullU's records combine the fields).  A set of one
 // run passes its row count and physics as launch arguments (own_rows, a.ph1).
+// With a.mode MODE_PROFILES it forms the profile lines of the mean fields read
+// and nothing else: for MHD_BQlin, whose lines k_meanfield rounds differently
+// (the compiler contracts products by their number of uses), the profiles of
+// an uploaded or restored state then have the bits a substep would leave.
 // ---------------------------------------------------------------------------
 constexpr int MFF_T = 1024;          // threads per workgroup
 constexpr int RED_CH = NT / RED_CW;  // row chunks per column, as k_reduce_cols
@@ -797,6 +801,7 @@ __global__ __launch_bounds__(MFF_T) void k_mf_fused(MFArgs a, const double *__re
         r1[q] = act ? min(nrows, r0[q] + per) : r0[q];
         s[q] = e[q] = 0.0;
     }
+    const bool lines_only = MODEL == 1 && a.mode == MODE_PROFILES;
     auto add_rows = [&](auto batch) {
         constexpr int B = decltype(batch)::value;
         for (int j = 0; j < per; j += B) {
@@ -814,8 +819,10 @@ __global__ __launch_bounds__(MFF_T) void k_mf_fused(MFArgs a, const double *__re
                 for (int k = 0; k < B; ++k) neumaier(s[q], e[q], v[q][k]);
         }
     };
-    if (per <= RED_FEW) add_rows(std::integral_constant<int, RED_FEW>{});
-    else add_rows(std::integral_constant<int, RED_BATCH>{});
+    if (!lines_only) {
+        if (per <= RED_FEW) add_rows(std::integral_constant<int, RED_FEW>{});
+        else add_rows(std::integral_constant<int, RED_BATCH>{});
+    }
 #pragma unroll
     for (int q = 0; q < NP; ++q) {
         const int pq = tid + q * MFF_T;
@@ -830,35 +837,40 @@ __global__ __launch_bounds__(MFF_T) void k_mf_fused(MFArgs a, const double *__re
         sh.sprev[tid] = pv;
     }
     if (tid < nslot) sh.smf[tid] = mv;
-    if (a.advance && f == 0 && tid == 0) clock_advance(a.clock + run);
-    __syncthreads();
-    if (tid < NZ) {
-        double t = 0.0, te = 0.0;
-        for (int k0 = 0; k0 < RED_CH && k0 * per < nrows; k0 += RED_FEW)  // the chunks that hold rows
-#pragma unroll
-            for (int k = k0; k < k0 + RED_FEW; ++k) {
-                neumaier(t, te, sh.red[k][tid]);
-                te += sh.red2[k][tid];
-            }
-        sh.ssum[tid] = t + te;
-    }
-    __syncthreads();
     const PadIO<NZ, double2> pad{sh.pad};
-    {
-        const double *S = sh.ssum;
-        const auto ld = [S](int, int j) { return make_double2(S[j], 0.0); };
-        fft_pass_io<NZ, 1, false, PL::R1, 1, false, MFF_T>(sh.tw, ld, pad);
-        fft_pass_io<NZ, 1, false, PL::R2, PL::R1, false, MFF_T>(sh.tw, pad, BufIO<NZ, double2>{sh.line});
-    }
-    if (tid < NZD) {
-        double2 Dv, N, Mn;
-        mf_slot<NZD, HALF, MODE, MODEL>(f, tid, sh.line, sh.skz, sh.smf, ph, a.mfn_prev != nullptr, sh.sprev[tid],
-                                        a.linC, a.nlc1, a.nlc2, Dv, N, Mn);
-        const size_t k = mo + (size_t)f * NZD + tid;
-        a.drive[k] = Dv;
-        a.mfn_out[k] = N;
-        a.mf[k] = Mn;
-        sh.smfn[tid] = Mn;
+    if (lines_only) {
+        __syncthreads();
+        if (tid < NZD) sh.smfn[tid] = sh.smf[f * NZD + tid];
+    } else {
+        if (a.advance && f == 0 && tid == 0) clock_advance(a.clock + run);
+        __syncthreads();
+        if (tid < NZ) {
+            double t = 0.0, te = 0.0;
+            for (int k0 = 0; k0 < RED_CH && k0 * per < nrows; k0 += RED_FEW)  // the chunks that hold rows
+    #pragma unroll
+                for (int k = k0; k < k0 + RED_FEW; ++k) {
+                    neumaier(t, te, sh.red[k][tid]);
+                    te += sh.red2[k][tid];
+                }
+            sh.ssum[tid] = t + te;
+        }
+        __syncthreads();
+        {
+            const double *S = sh.ssum;
+            const auto ld = [S](int, int j) { return make_double2(S[j], 0.0); };
+            fft_pass_io<NZ, 1, false, PL::R1, 1, false, MFF_T>(sh.tw, ld, pad);
+            fft_pass_io<NZ, 1, false, PL::R2, PL::R1, false, MFF_T>(sh.tw, pad, BufIO<NZ, double2>{sh.line});
+        }
+        if (tid < NZD) {
+            double2 Dv, N, Mn;
+            mf_slot<NZD, HALF, MODE, MODEL>(f, tid, sh.line, sh.skz, sh.smf, ph, a.mfn_prev != nullptr, sh.sprev[tid],
+                                            a.linC, a.nlc1, a.nlc2, Dv, N, Mn);
+            const size_t k = mo + (size_t)f * NZD + tid;
+            a.drive[k] = Dv;
+            a.mfn_out[k] = N;
+            a.mf[k] = Mn;
+            sh.smfn[tid] = Mn;
+        }
     }
     __syncthreads();
     // the field's real-space profile lines (k_meanfield's lines 2f, 2f + 1;

@@ -70,9 +70,8 @@ inline int mb_for(int NZ, int line) { return (line == LINE_WAVE || NZ >= line) ?
 //                  which saves a launch (2-4 us per step); with more rows (NZ =
 //                  64, 504 rows: 78.4 against 77.5) or longer ones (NZ = 128, 252
 //                  rows: 116 against 109; 60 rows: 55.2 against 53.0) its
-//                  workgroups read too much each.  Not MHD_BQlin's, whose
-//                  profile lines the two tails round differently: a run continued
-//                  from its saved state must give the same bits.
+//                  workgroups read too much each (36x60x64 MHD_BQlin with noise, 100 CN
+//                  steps: 5.46 -> 5.24 ms).
 // Groups of more than SMALL_SET runs fill the chip and share it with the other
 // groups: there eight (four) modes per pass and two launches measured best (48
 // runs: 160.0 us per step; wavefront kernel at NZ = 64 164.0, one-launch tail
@@ -81,10 +80,10 @@ constexpr int SMALL_SET = 4, SMALL_MODES = 512, TAIL_ONE = 16384;
 struct Shape {
     int line, target, tail;
 };
-inline Shape default_shape(int NZ, int model, int precision, int nruns, int modes)
+inline Shape default_shape(int NZ, int precision, int nruns, int modes)
 {
     const bool small = precision == QL_PREC_FP64 && nruns <= SMALL_SET;
-    const int tail = small && NZ <= 64 && model != QL_MODEL_MHD_BQLIN ? 1 : 0;
+    const int tail = small && NZ <= 64 ? 1 : 0;
     if (NZ >= 128) return Shape{LINE_WAVE, 256, tail};
     if (small && (NZ == 64 || modes <= SMALL_MODES)) {
         const int target = modes / 4 < 64 ? 64 : (modes / 4 < 256 ? modes / 4 : 256);
@@ -237,7 +236,7 @@ struct SubBuffers {
 };
 int enqueue_substep(Batch &b, Group &g, int s, bool remap_after, bool advance, hipStream_t st,
                     const SubBuffers *bf = nullptr);
-void launch_mf(const Group &g, const qlk::MFArgs &m, hipStream_t st);
+void launch_profiles(const Batch &b, const Group &g, qlk::MFArgs m, hipStream_t st);
 int launch_noise(Group &g, double2 *u, bool use_clock, double t, double dt, bool noise, bool remap, hipStream_t st);
 qlk::MFArgs mf_args(const Batch &b, const Group &g);
 // the caller's layout: fluctuation fields per mode, mean fields, and the

@@ -184,3 +184,27 @@ def test_partial_row_counts_match_oracle(NZ, rows):
     assert np.array_equal(out[0][3], kx0)
     for got, want in ((out[0][1], lin), (out[0][2], mf), (out[0][4], o.drive())):
         assert rel_err(got, want) < 1e-10
+
+
+@pytest.mark.parametrize("integrator", [0, 1])
+@pytest.mark.parametrize("model,NZ", [(1, 32), (1, 64), (1, 128), (0, 64)])
+def test_uploaded_state_continues_bitwise(model, NZ, integrator):
+    """The profiles formed from an uploaded state, or around a CFL call, have the bits
+    that the one-launch tail leaves: a run interrupted by both continues as one that
+    was not."""
+    from ql_dns_amd.capi import QLContext
+    from ql_dns_amd.ic import initial_state
+    p = _p(model=model, integrator=integrator, NX=16, NY=16, NZ=NZ, Ly=1.0)
+    out = []
+    for stop in (False, True):
+        c = QLContext(p)
+        c.set_tail(NZ, 1)
+        c.set_state(*initial_state(p))
+        c.linear_ops_init(0.0)
+        t = c.steps(5, 0.0)
+        if stop:
+            c.set_state(*c.get_state())
+            c.calculate_cfl()
+        out.append((c.steps(5, t),) + tuple(c.get_state()) + (c.drive(),))
+        c.close()
+    _equal(*out)
