@@ -404,3 +404,34 @@ def test_variable_steps_adjoint_matches_frozen_step_differences():
         Lm = _loss_parts(p, *_frozen_run(p.replace(**{name: base - h}), lin0, mf0, dts), alpha)[0]
         fd = (Lp - Lm) / (2 * h)
         assert abs(gpar[k] - fd) <= TOL * abs(fd), f"d/d{name}: adjoint {gpar[k]!r} fd {fd!r}"
+
+
+@pytest.mark.parametrize("NX,NY,NZ", [(46, 46, 128), (34, 34, 256), (4, 2, 32), (2, 2, 64)])
+def test_adjoint_of_many_and_few_modes(NX, NY, NZ):
+    """More groups of modes than the reverse mode kernel has workgroups (512), so that
+    a workgroup takes several and the last one part of a group, and fewer modes than
+    one group holds: one state direction and q, the bars above."""
+    from ql_dns_amd.capi import QLContext
+    from ql_dns_amd.ic import initial_state
+    p = _p(NX=NX, NY=NY, NZ=NZ, Ly=1.0, B0z=0.03, nu=1 / 1500, eta=1 / 1200)
+    n, every = 4, 3
+    lin0, mf0 = initial_state(p)
+    alpha = 0.01 / max(float((np.abs(lin0) ** 2).sum()), 1.0)
+    c = QLContext(p)
+    c.set_state(lin0, mf0)
+    c.linear_ops_init(0.0)
+    c.adjoint_forward(n, every, 0.0)
+    linT, mfT, _ = c.get_state()
+    _, g_lin, g_mf = _loss_parts(p, linT, mfT, alpha)
+    gl0, gm0, gpar = c.adjoint_backward(g_lin, g_mf)
+    c.close()
+    rng = np.random.default_rng(11)
+    vl = (rng.standard_normal(lin0.shape) + 1j * rng.standard_normal(lin0.shape)) * np.sqrt(np.mean(np.abs(lin0) ** 2))
+    vl[::NY // 2, 0::2, 0] = 0
+    vm = (rng.standard_normal(mf0.shape) + 1j * rng.standard_normal(mf0.shape)) * np.sqrt(np.mean(np.abs(mf0) ** 2))
+    ad = float(np.sum(gl0.real * vl.real + gl0.imag * vl.imag) + np.sum(gm0.real * vm.real + gm0.imag * vm.imag))
+    L = [_loss_parts(p, *_run(p, lin0 + s * EPS * vl, mf0 + s * EPS * vm, n), alpha)[0] for s in (1, -1)]
+    assert abs(ad - (L[0] - L[1]) / (2 * EPS)) <= TOL * abs(ad)
+    h = EPS * p.q
+    L = [_loss_parts(p, *_run(p.replace(q=p.q + s * h), lin0, mf0, n), alpha)[0] for s in (1, -1)]
+    assert abs(gpar[0] - (L[0] - L[1]) / (2 * h)) <= TOL * abs(gpar[0])

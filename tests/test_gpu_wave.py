@@ -260,3 +260,30 @@ def test_z_lines_in_registers_match_oracle(model, NZ, NX, NY, target):
     for a, b in zip(g.rhs(0.37, 0.011), o.rhs(0.37, 0.011)):
         assert rel_err(a, b) < 1e-12
     assert rel_err(g.drive(), o.drive()) < 1e-12
+
+
+@pytest.mark.parametrize("model", [0, 1, 2])
+@pytest.mark.parametrize("NX,NY,NZ,runs", [(2, 2, 32, 1), (32, 32, 32, 1), (34, 32, 32, 1), (2, 2, 64, 1), (10, 6, 64, 1),
+                                           (8, 8, 32, 4), (8, 8, 32, 5), (8, 6, 64, 4), (8, 6, 64, 5)])
+def test_default_shapes_match_oracle(model, NX, NY, NZ, runs):
+    """Shapes and tails as a context chooses them, on both sides of the rule's lines
+    (512 modes at NZ = 32, sets of four and of five runs) and for the fewest modes."""
+    from ql_dns_amd.capi import QLBatch
+    from ql_dns_amd.ic import initial_state
+    from oracle.oracle import Oracle
+    ps = [_params(model=model, NX=NX, NY=NY, NZ=NZ, q=1.5 - 0.05 * r) for r in range(runs)]
+    st = [initial_state(p, seed=30 + r) for r, p in enumerate(ps)]
+    b = QLBatch(ps)
+    for r, s in enumerate(st):
+        b.set_state(r, *s)
+    b.linear_ops_init(0.0)
+    t = b.steps(6, 0.0)
+    for r in {0, runs - 1}:
+        o = Oracle.from_params(ps[r], nthreads=8)
+        o.set_state(*st[r])
+        o.linear_ops_init(0.0)
+        assert o.steps(6, 0.0) == t
+        (lo, mo, ko), (lg, mg, kg) = o.get_state(), b.get_state(r)
+        assert np.array_equal(kg, ko)
+        assert rel_err(mg, mo) < TOL and rel_err(lg, lo) < TOL
+    b.close()
