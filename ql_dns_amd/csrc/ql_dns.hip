@@ -38,6 +38,9 @@ int fail(int code, const char *fmt, ...)
     vsnprintf(buf, sizeof(buf), fmt, ap);
     va_end(ap);
     g_err = buf;
+    // the runtime keeps a failed call's error until it is asked for it: without
+    // this the launch checks of the next calls would report it once more
+    if (code == QL_ERR_HIP) (void)hipGetLastError();
     return code;
 }
 

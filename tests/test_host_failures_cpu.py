@@ -1,0 +1,110 @@
+"""What libql_dns.so's host code does when a runtime call fails, without a GPU:
+the library runs on tests/cpp/hip_on_host.cpp, which serves its HIP calls from
+host memory (kernels do nothing) and makes chosen ones fail.  Every scenario
+runs in a process of its own."""
+import ctypes
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("hip_on_host") / "hip_on_host.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Werror", "-o", so,
+                    os.path.join(HERE, "cpp", "hip_on_host.cpp")], check=True)
+    return so
+
+
+def scenario(runtime, name, *args):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), runtime, name] + [str(a) for a in args],
+                       stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=300)
+    assert r.returncode == 0 and "scenario done" in r.stdout, r.stdout
+
+
+# ---------------------------------------------------------------------------
+# in the scenario's process
+# ---------------------------------------------------------------------------
+class Host:
+    """The stand-in runtime's controls."""
+
+    def __init__(self, so):
+        # ahead of the library's own dependencies in symbol lookup
+        self.L = ctypes.CDLL(so, mode=ctypes.RTLD_GLOBAL)
+        for f in ("hoh_live", "hoh_limit"):
+            getattr(self.L, f).restype = ctypes.c_size_t
+        for f in ("hoh_races", "hoh_bad", "hoh_null_waits", "hoh_mallocs", "hoh_host_live", "hoh_sizes"):
+            getattr(self.L, f).restype = ctypes.c_long
+        for f in ("hoh_fail_malloc", "hoh_fail_host", "hoh_fail_new"):
+            getattr(self.L, f).argtypes = [ctypes.c_long]
+        self.L.hoh_limit.argtypes = [ctypes.c_size_t]
+        self.L.hoh_sizes.argtypes = [ctypes.POINTER(ctypes.c_size_t), ctypes.c_long]
+
+    def __getattr__(self, name):
+        return getattr(self.L, "hoh_" + name)
+
+    def sizes(self):
+        n = self.L.hoh_sizes(None, 0)
+        a = (ctypes.c_size_t * n)()
+        self.L.hoh_sizes(a, n)
+        return list(a)
+
+    def clean(self):
+        """No copy outside its buffer and none that a late clearing could undo."""
+        assert self.bad() == 0 and self.races() == 0, (self.bad(), self.races())
+
+
+def _state(c, seed=3):
+    rng = np.random.default_rng(seed)
+    lin = rng.standard_normal((c.nxy, c.nLin, c.nz)) + 1j * rng.standard_normal((c.nxy, c.nLin, c.nz))
+    lin[::c.params.NY // 2, 0::2, 0] = 0
+    return lin, rng.standard_normal((c.nMF, c.nz)) + 0j
+
+
+def _context(**kw):
+    from ql_dns_amd.capi import QLContext
+    from ql_dns_amd.params import QLParams
+    kw.setdefault("NX", 8)
+    kw.setdefault("NY", 6)
+    kw.setdefault("NZ", 32)
+    c = QLContext(QLParams(**kw))
+    c.set_state(*_state(c))
+    c.linear_ops_init(0.0)
+    return c
+
+
+def _fails(f, *args):
+    from ql_dns_amd.capi import QLError
+    try:
+        f(*args)
+    except QLError as e:
+        assert e.code == -2 and "out of memory" in str(e), e
+        return True
+    return False
+
+
+def s_error_is_reported_once(host):
+    c = _context()
+    c.adjoint_forward(4, 2, 0.0)
+    host.fail_malloc(1)
+    assert _fails(c.adjoint_backward)
+    # the calls after it launch kernels and check for their errors, not for an old one
+    c.steps(3)
+    c.get_state()
+
+
+# ---------------------------------------------------------------------------
+def test_a_failed_allocation_is_reported_once(runtime):
+    scenario(runtime, "error_is_reported_once")
+
+
+if __name__ == "__main__":
+    sys.path.insert(0, os.path.dirname(HERE))
+    host_ = Host(sys.argv[1])
+    globals()["s_" + sys.argv[2]](host_, *[int(a) for a in sys.argv[3:]])
+    print("scenario done")
