@@ -48,11 +48,19 @@ struct AdjState {
     double *gsums = nullptr, *gpart = nullptr, *grows = nullptr, *gpar_mf = nullptr, *gpar = nullptr;
 };
 
+// The buffers outlive a call that fails, so each of the three kinds (a
+// checkpoint, the segment's, the adjoint's) is there as a whole or not at all:
+// its first pointer tells
 namespace {
 void free_ck(AdjState::Ck &c) { dfree(c.u), dfree(c.mf), dfree(c.kx0), dfree(c.pm); }
 void free_segment(AdjState *A)
 {
     dfree(A->st_u), dfree(A->st_mf), dfree(A->st_kx0), dfree(A->st_pre), dfree(A->st_mfz);
+}
+void free_adjoint(AdjState *A)
+{
+    dfree(A->gu), dfree(A->gnp), dfree(A->gM), dfree(A->gnmp);
+    dfree(A->gsums), dfree(A->gpart), dfree(A->grows), dfree(A->gpar_mf), dfree(A->gpar);
 }
 }  // namespace
 
@@ -62,8 +70,7 @@ void adj_release(Batch &b)
     if (!A) return;
     for (auto &c : A->ck) free_ck(c);
     free_segment(A);
-    dfree(A->gu), dfree(A->gnp), dfree(A->gM), dfree(A->gnmp);
-    dfree(A->gsums), dfree(A->gpart), dfree(A->grows), dfree(A->gpar_mf), dfree(A->gpar);
+    free_adjoint(A);
     delete A;
     b.adj = nullptr;
 }
@@ -231,6 +238,43 @@ int adj_fit(Batch &b, int nsteps, int every, bool noise)
     return QL_OK;
 }
 
+// one segment's states, mean fields and profiles: all of them or none
+int alloc_segment(AdjState *A, const Group &g, size_t nl, size_t nm)
+{
+    const size_t K = A->every;
+    const int rc = [&]() -> int {
+        QL_RC(dalloc(&A->st_u, nl * (3 * K + 1)));
+        QL_RC(dalloc(&A->st_mf, nm * (3 * K + 1)));
+        QL_RC(dalloc(&A->st_kx0, (size_t)g.modes * K));
+        // zeroed: MHD_BQlin writes 3 of the 8 profile lines
+        QL_RC(dalloc(&A->st_mfz, (size_t)8 * g.NZ * (3 * K + 1)));
+        if (g.noise) QL_RC(dalloc(&A->st_pre, nl * K));
+        return QL_OK;
+    }();
+    if (rc != QL_OK) free_segment(A);
+    return rc;
+}
+
+// the adjoint state, its sums and W partial rows: all of them or none
+int alloc_adjoint(AdjState *A, const Group &g, size_t nl, size_t nm, int W)
+{
+    const size_t ncols = 8 * g.NZ + qlk::NGP;
+    const int rc = [&]() -> int {
+        QL_RC(dalloc(&A->gu, nl));
+        QL_RC(dalloc(&A->gnp, nl));
+        QL_RC(dalloc(&A->gM, nm));
+        QL_RC(dalloc(&A->gnmp, nm));
+        QL_RC(dalloc(&A->gsums, (size_t)4 * g.NZ));  // zeroed: MHD_BQlin fills 2 of the 4 lines
+        QL_RC(dalloc(&A->gpart, (size_t)W * ncols));
+        QL_RC(dalloc(&A->grows, ncols));
+        QL_RC(dalloc(&A->gpar_mf, (size_t)qlk::NGP));
+        QL_RC(dalloc(&A->gpar, (size_t)qlk::NGP));
+        return QL_OK;
+    }();
+    if (rc != QL_OK) free_adjoint(A);
+    return rc;
+}
+
 int adjoint_forward(Batch &b, int nsteps, int every, double *t_inout)
 {
     QL_RC(check_adjoint(b, "ql_adjoint_forward"));
@@ -265,26 +309,8 @@ int adjoint_backward(Batch &b, const double *g_lin, const double *g_mf, double *
     const size_t nl = (size_t)nxy * 4 * nz, nm = (size_t)b.nMF * nz;
     const int MB = qlk::NT / NZ;  // modes per pass of the reverse mode kernel
     const int W = std::min((nxy + MB - 1) / MB, ADJ_GMAX);
-    const int ncols = 8 * NZ + qlk::NGP;
-    if (!A->st_u) {
-        QL_RC(dalloc(&A->st_u, nl * (3 * K + 1)));
-        QL_RC(dalloc(&A->st_mf, nm * (3 * K + 1)));
-        QL_RC(dalloc(&A->st_kx0, (size_t)nxy * K));
-        // zeroed: MHD_BQlin writes 3 of the 8 profile lines
-        QL_RC(dalloc(&A->st_mfz, (size_t)8 * NZ * (3 * K + 1)));
-        if (g.noise) QL_RC(dalloc(&A->st_pre, nl * K));
-    }
-    if (!A->gpar) {
-        QL_RC(dalloc(&A->gu, nl));
-        QL_RC(dalloc(&A->gnp, nl));
-        QL_RC(dalloc(&A->gM, nm));
-        QL_RC(dalloc(&A->gnmp, nm));
-        QL_RC(dalloc(&A->gsums, (size_t)4 * NZ));  // zeroed: MHD_BQlin fills 2 of the 4 lines
-        QL_RC(dalloc(&A->gpart, (size_t)W * ncols));
-        QL_RC(dalloc(&A->grows, (size_t)ncols));
-        QL_RC(dalloc(&A->gpar_mf, (size_t)qlk::NGP));
-        QL_RC(dalloc(&A->gpar, (size_t)qlk::NGP));
-    }
+    if (!A->st_u) QL_RC(alloc_segment(A, g, nl, nm));
+    if (!A->gu) QL_RC(alloc_adjoint(A, g, nl, nm, W));
     // HD_fullU runs the MHD_FullQlin kernels with b = B = 0 on the internal
     // four-field layout: its caller's (ux, zeta) and (Ux, Uy) gradients sit at
     // fields 0, 1 and mean-field slots 2, 3, the others are zero

@@ -98,7 +98,48 @@ def s_error_is_reported_once(host):
     c.get_state()
 
 
+def _gradient(c, n=7, every=3):
+    c.adjoint_forward(n, every, 0.0)
+    c.adjoint_backward()
+
+
+def _noisy_context(model):
+    c = _context(model=model, NZ=64)
+    c.set_noise(2.0)  # the driven step's buffer among the segment's
+    return c
+
+
+def s_backward_buffers(host, model):
+    # the allocations of a backward, and what is allocated after one
+    c = _noisy_context(model)
+    c.adjoint_forward(7, 3, 0.0)
+    n0 = host.mallocs()
+    c.adjoint_backward()
+    nalloc, sizes = host.mallocs() - n0, host.sizes()
+    c.close()
+    assert nalloc > 10 and host.live() == 0
+    for k in range(1, nalloc + 1):
+        c = _noisy_context(model)
+        c.adjoint_forward(7, 3, 0.0)
+        host.fail_malloc(k)
+        assert _fails(c.adjoint_backward), k
+        c.adjoint_backward()  # the same backward again, with memory to be had
+        assert host.sizes() == sizes, k
+        _gradient(c)
+        assert host.sizes() == sizes, k
+        c.close()
+        assert host.live() == 0 and host.host_live() == 0, k
+    host.clean()
+
+
 # ---------------------------------------------------------------------------
+@pytest.mark.parametrize("model", [0, 1, 2])
+def test_backward_after_a_failed_allocation(runtime, model):
+    """Whichever of a gradient's buffers could not be had, the same backward and
+    the next gradient find all of them, and none is lost."""
+    scenario(runtime, "backward_buffers", model)
+
+
 def test_a_failed_allocation_is_reported_once(runtime):
     scenario(runtime, "error_is_reported_once")
 
