@@ -89,16 +89,25 @@ int check_adjoint(const Batch &b, const char *who)
     return QL_OK;
 }
 
-int save_ck(Batch &b, AdjState::Ck &c, double t)
+// a checkpoint's buffers: all of them or none
+int alloc_ck(AdjState::Ck &c, const Group &g, size_t nl, size_t nm)
 {
-    Group &g = b.groups[0];
-    const size_t nl = (size_t)g.modes * 4 * g.nz, nm = (size_t)b.nMF * g.nz;
-    if (!c.u) {
+    const int rc = [&]() -> int {
         QL_RC(dalloc(&c.u, nl));
         QL_RC(dalloc(&c.mf, nm));
         QL_RC(dalloc(&c.kx0, g.modes));
         QL_RC(dalloc(&c.pm, (size_t)qlk::PM_STRIDE));
-    }
+        return QL_OK;
+    }();
+    if (rc != QL_OK) free_ck(c);
+    return rc;
+}
+
+int save_ck(Batch &b, AdjState::Ck &c, double t)
+{
+    Group &g = b.groups[0];
+    const size_t nl = (size_t)g.modes * 4 * g.nz, nm = (size_t)b.nMF * g.nz;
+    if (!c.u) QL_RC(alloc_ck(c, g, nl, nm));
     QL_HIP(hipMemcpyAsync(c.u, g.u, sizeof(double2) * nl, hipMemcpyDeviceToDevice, b.s));
     QL_HIP(hipMemcpyAsync(c.mf, g.mf, sizeof(double2) * nm, hipMemcpyDeviceToDevice, b.s));
     QL_HIP(hipMemcpyAsync(c.kx0, g.kx0, sizeof(double) * g.modes, hipMemcpyDeviceToDevice, b.s));

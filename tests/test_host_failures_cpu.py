@@ -88,6 +88,15 @@ def _fails(f, *args):
     return False
 
 
+def _fails_state(f, *args):
+    from ql_dns_amd.capi import QL_ERR_STATE, QLError
+    try:
+        f(*args)
+    except QLError as e:
+        return e.code == QL_ERR_STATE
+    return False
+
+
 def s_error_is_reported_once(host):
     c = _context()
     c.adjoint_forward(4, 2, 0.0)
@@ -132,7 +141,33 @@ def s_backward_buffers(host, model):
     host.clean()
 
 
+def s_checkpoints(host):
+    c = _context()
+    n0 = host.mallocs()
+    c.adjoint_forward(7, 2, 0.0)
+    nalloc, sizes = host.mallocs() - n0, host.sizes()
+    c.close()
+    assert nalloc > 15 and host.live() == 0
+    for k in range(1, nalloc + 1):
+        c = _context()
+        host.fail_malloc(k)
+        assert _fails(c.adjoint_forward, 7, 2, 0.0), k
+        assert _fails_state(c.adjoint_backward), k  # no forward has completed
+        c.adjoint_forward(7, 2, 0.0)
+        assert host.sizes() == sizes, k
+        c.adjoint_backward()
+        c.close()
+        assert host.live() == 0, k
+    host.clean()
+
+
 # ---------------------------------------------------------------------------
+def test_forward_after_a_failed_allocation(runtime):
+    """Whichever buffer of a checkpoint could not be had, the next forward on the
+    context finds all of them."""
+    scenario(runtime, "checkpoints")
+
+
 @pytest.mark.parametrize("model", [0, 1, 2])
 def test_backward_after_a_failed_allocation(runtime, model):
     """Whichever of a gradient's buffers could not be had, the same backward and
