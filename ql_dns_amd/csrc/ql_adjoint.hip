@@ -103,11 +103,24 @@ int alloc_ck(AdjState::Ck &c, const Group &g, size_t nl, size_t nm)
     return rc;
 }
 
-int save_ck(Batch &b, AdjState::Ck &c, double t)
+// checkpoint k of the forward
+int save_ck(Batch &b, int k, double t)
 {
+    AdjState *A = b.adj;
+    AdjState::Ck &c = A->ck[k];
     Group &g = b.groups[0];
     const size_t nl = (size_t)g.modes * 4 * g.nz, nm = (size_t)b.nMF * g.nz;
-    if (!c.u) QL_RC(alloc_ck(c, g, nl, nm));
+    if (!c.u) {
+        int rc = alloc_ck(c, g, nl, nm);
+        if (rc != QL_OK && (A->st_u || A->gu)) {
+            // what an earlier backward left makes way
+            QL_HIP(hipStreamSynchronize(b.s));
+            free_segment(A);
+            free_adjoint(A);
+            rc = alloc_ck(c, g, nl, nm);
+        }
+        QL_RC(rc);
+    }
     QL_HIP(hipMemcpyAsync(c.u, g.u, sizeof(double2) * nl, hipMemcpyDeviceToDevice, b.s));
     QL_HIP(hipMemcpyAsync(c.mf, g.mf, sizeof(double2) * nm, hipMemcpyDeviceToDevice, b.s));
     QL_HIP(hipMemcpyAsync(c.kx0, g.kx0, sizeof(double) * g.modes, hipMemcpyDeviceToDevice, b.s));
@@ -293,11 +306,11 @@ int adjoint_forward(Batch &b, int nsteps, int every, double *t_inout)
     A->t_init = b.t_init;
     double t = *t_inout;
     for (int sg = 0; sg < A->nseg; ++sg) {
-        QL_RC(save_ck(b, A->ck[sg], t));
+        QL_RC(save_ck(b, sg, t));
         const int n = std::min(every, nsteps - sg * every);
         QL_RC(run_steps(b, n, &t));
     }
-    QL_RC(save_ck(b, A->ck[A->nseg], t));
+    QL_RC(save_ck(b, A->nseg, t));
     QL_HIP(hipStreamSynchronize(b.s));
     A->valid = true;
     *t_inout = t;

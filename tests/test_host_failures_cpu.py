@@ -161,7 +161,29 @@ def s_checkpoints(host):
     host.clean()
 
 
+def s_room_for_checkpoints(host):
+    c = _context()
+    c.adjoint_forward(40, 2, 0.0)
+    need = host.live()
+    c.close()
+    c = _context()
+    _gradient(c, 4, 2)
+    host.limit(need)  # just what the forward takes on a new context
+    c.adjoint_forward(40, 2, 0.0)
+    assert host.live() <= need
+    host.limit(1 << 40)
+    c.adjoint_backward()
+    c.close()
+    assert host.live() == 0
+    host.clean()
+
+
 # ---------------------------------------------------------------------------
+def test_longer_forward_after_a_gradient_takes_no_more_memory(runtime):
+    """The buffers an earlier backward left make way for checkpoints."""
+    scenario(runtime, "room_for_checkpoints")
+
+
 def test_forward_after_a_failed_allocation(runtime):
     """Whichever buffer of a checkpoint could not be had, the next forward on the
     context finds all of them."""
