@@ -132,8 +132,8 @@ int save_ck(Batch &b, int k, double t)
     return QL_OK;
 }
 
-// the state and clock history of a checkpoint, the state into u, mf and the
-// profiles mfz
+// the state, step record and clock history of a checkpoint, the state into u, mf
+// and the profiles mfz
 int load_ck(Batch &b, const AdjState::Ck &c, double2 *u, double2 *mf, double *mfz)
 {
     Group &g = b.groups[0];
@@ -148,6 +148,7 @@ int load_ck(Batch &b, const AdjState::Ck &c, double2 *u, double2 *mf, double *mf
     qlk::MFArgs m = mf_args(b, g);
     m.mf = mf;
     m.mfz = mfz;
+    m.rec = 0;  // the record is the checkpoint's: HD_fullU's holds the drives of its last rhs
     launch_profiles(b, g, m, b.s);
     QL_HIP(hipGetLastError());
     return QL_OK;
