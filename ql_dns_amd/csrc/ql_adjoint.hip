@@ -37,6 +37,7 @@ struct AdjState {
         int old_init = 0;
     };
     std::vector<Ck> ck;
+    double2 *drive = nullptr;  // of the forward's last right-hand side (no segment reads them)
     double t_init = 0.0;
     // substep states, mean fields and profiles of one segment; with driving
     // noise also each step's state after substep 3 before the noise and the
@@ -69,6 +70,7 @@ void adj_release(Batch &b)
     AdjState *A = b.adj;
     if (!A) return;
     for (auto &c : A->ck) free_ck(c);
+    dfree(A->drive);
     free_segment(A);
     free_adjoint(A);
     delete A;
@@ -312,6 +314,10 @@ int adjoint_forward(Batch &b, int nsteps, int every, double *t_inout)
         QL_RC(run_steps(b, n, &t));
     }
     QL_RC(save_ck(b, A->nseg, t));
+    const Group &g = b.groups[0];
+    const size_t nm = (size_t)b.nMF * g.nz;
+    if (!A->drive) QL_RC(dalloc(&A->drive, nm));
+    QL_HIP(hipMemcpyAsync(A->drive, g.drive, sizeof(double2) * nm, hipMemcpyDeviceToDevice, b.s));
     QL_HIP(hipStreamSynchronize(b.s));
     A->valid = true;
     *t_inout = t;
@@ -488,6 +494,7 @@ int adjoint_backward(Batch &b, const double *g_lin, const double *g_mf, double *
     QL_RC(launch_adj_mf(NZ, b.model, aa, b.s));
     // leave the context at the forward's final state
     QL_RC(load_ck(b, A->ck[A->nseg], g.u, g.mf, g.mfz));
+    QL_HIP(hipMemcpyAsync(g.drive, A->drive, sizeof(double2) * nm, hipMemcpyDeviceToDevice, b.s));
     double gp[qlk::NGP];
     QL_RC(state_out(*b.out, b.s, A->gu, nxy, ext_nlin(b) * nz, 4 * nz, g_lin0, A->gM + (size_t)ext_mf0(b) * nz,
                     ext_nmf(b) * nz, g_mf0, A->gpar, qlk::NGP, gp));

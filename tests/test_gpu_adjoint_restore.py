@@ -108,3 +108,21 @@ def test_hd_variable_steps_adjoint_matches_frozen_step_differences():
         L = [loss(*frozen(p.replace(**{name: getattr(p, name) + s * h}), lin0, mf0)) for s in (1, -1)]
         fd = (L[0] - L[1]) / (2 * h)
         assert abs(gpar[k] - fd) <= TOL * abs(fd), f"d/d{name}: adjoint {gpar[k]!r} fd {fd!r}"
+
+
+@pytest.mark.parametrize("model,integrator,dt", [(0, 1, 0.004), (1, 0, 0.004), (2, 1, 0.004), (0, 0, -0.05), (2, 1, -0.05)])
+def test_drives_after_a_gradient_are_the_forwards(model, integrator, dt):
+    """The drives and what the diagnostics read are those of the forward's last
+    right-hand side, not of the segment recomputed last."""
+    from ql_dns_amd.ic import initial_state
+    p = _p(model=model, integrator=integrator, dt=dt, CFL=1.0)
+    lin, mf = initial_state(p, amp=0.05)
+    c = _start(p, lin, mf)
+    t = c.adjoint_forward(7, 3, 0.0)
+    want = (c.drive(), c.drive_real(), c.mf_real(), c.diagnostics(t), c.calculate_cfl())
+    l, m, _ = c.get_state()
+    c.adjoint_backward(1e-3 * l, m)
+    got = (c.drive(), c.drive_real(), c.mf_real(), c.diagnostics(t), c.calculate_cfl())
+    c.close()
+    for a, b in zip(want, got):
+        assert np.array_equal(a, b)
