@@ -1368,6 +1368,7 @@ int tune(Batch &b, int trial_steps, double *best_ms_out)
         }
         g.dft = best_dft;
         g.tail = best_tail;
+        g.own_shape = true;
         if (rc == QL_OK) rc = configure(b, g, best_line, best_target);
         total_best += best;
     }
@@ -1957,12 +1958,19 @@ int ql_batch_set_transform(ql_batch *bt, int NZ, int transform)
         if (g.NZ != NZ) continue;
         if (transform != QL_TRANSFORM_FFT && transform != QL_TRANSFORM_DFT_MFMA)
             return fail(QL_ERR_ARG, "ql_batch_set_transform: unknown transform %d", transform);
-        if (transform == QL_TRANSFORM_DFT_MFMA && !dft_ok(g.NZ, b.precision, g.line))
+        // the wavefront kernel has no matrix-core variant: a group that is on it by
+        // default only moves to the workgroup kernel, and back with the radix transforms
+        Shape sh{g.line, g.target, g.tail};
+        if (!g.own_shape) {
+            sh = default_shape(g.NZ, b.precision, g.nruns, g.modes);
+            if (transform == QL_TRANSFORM_DFT_MFMA && sh.line == LINE_WAVE) sh = Shape{DEFAULT_LINE, DEFAULT_TARGET, sh.tail};
+        }
+        if (transform == QL_TRANSFORM_DFT_MFMA && !dft_ok(g.NZ, b.precision, sh.line))
             return fail(QL_ERR_ARG,
                         "ql_batch_set_transform: the matrix-core transform needs FP64, NZ 32 or 64 and line 128 "
-                        "or 256 (NZ %d, line %d)", g.NZ, g.line);
+                        "or 256 (NZ %d, line %d)", g.NZ, sh.line);
         g.dft = transform;
-        return configure(b, g, g.line, g.target);
+        return configure(b, g, sh.line, sh.target);
     }
     return fail(QL_ERR_ARG, "ql_batch_set_transform: no group with NZ = %d", NZ);
 }
@@ -2045,7 +2053,10 @@ int ql_batch_set_config(ql_batch *bt, int NZ, int line, int target)
     if (target < 1) return fail(QL_ERR_ARG, "ql_batch_set_config: target=%d < 1", target);
     Batch &b = bt->b;
     for (Group &g : b.groups)
-        if (g.NZ == NZ) return configure(b, g, line, target);
+        if (g.NZ == NZ) {
+            g.own_shape = true;
+            return configure(b, g, line, target);
+        }
     return fail(QL_ERR_ARG, "ql_batch_set_config: no runs with NZ=%d", NZ);
 }
 

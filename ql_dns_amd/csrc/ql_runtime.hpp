@@ -112,6 +112,7 @@ struct Group {
     int NZ = 0, nz = 0, nruns = 0, modes = 0;
     std::vector<int> run_ids;
     int line = DEFAULT_LINE, target = DEFAULT_TARGET;
+    bool own_shape = false;  // the shape was asked for (ql_batch_set_config) or tuned: not default_shape's
     int dft = 0;  // 1: the workgroup kernel's transforms as matrix-core products (ql_dft.hpp)
     int MB = 1, W = 0, part_cap = 0, wg_cap = 0;
     hipStream_t s = nullptr;  // own stream (sets with several groups)

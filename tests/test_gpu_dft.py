@@ -102,3 +102,29 @@ def test_tuner_times_the_matrix_core_candidate():
         lg, mg, _ = b.get_state(r)
         assert rel_err(mg, mo) < TOL and rel_err(lg, lo) < TOL
     b.close()
+
+
+@pytest.mark.parametrize("model", [0, 1, 2])
+@pytest.mark.parametrize("NZ", [32, 64])
+def test_dft_on_a_default_shape_matches_oracle(model, NZ):
+    """Without a shape asked for (small FP64 sets are on the wavefront kernel by
+    default, which has no matrix-core variant)."""
+    from ql_dns_amd.capi import QLContext
+    from ql_dns_amd.ic import initial_state
+    from ql_dns_amd.params import QLParams
+    from oracle.oracle import Oracle
+    p = QLParams(model=model, NX=8, NY=8, NZ=NZ, B0z=0.02, Ly=1.0)
+    lin, mf = initial_state(p)
+    o, g = Oracle.from_params(p, nthreads=8), QLContext(p)
+    for x in (o, g):
+        x.set_state(lin, mf)
+        x.linear_ops_init(0.0)
+    assert g.steps(4, 0.0) == o.steps(4, 0.0)  # replay graphs of the default shape exist
+    g.set_transform(NZ, DFT)
+    assert g.config()[0]["transform"] == DFT
+    to, tg = o.steps(26, 4 * p.dt), g.steps(26, 4 * p.dt)
+    assert tg == to
+    (lo, mo, ko), (lg, mg, kg) = o.get_state(), g.get_state()
+    assert np.array_equal(kg, ko)
+    assert rel_err(mg, mo) < TOL and rel_err(lg, lo) < TOL
+    assert rel_err(g.drive(), o.drive()) < TOL

@@ -1,7 +1,8 @@
-"""What libql_dns.so's host code does when a runtime call fails, without a GPU:
-the library runs on tests/cpp/hip_on_host.cpp, which serves its HIP calls from
-host memory (kernels do nothing) and makes chosen ones fail.  Every scenario
-runs in a process of its own."""
+"""libql_dns.so's host code without a GPU: what it does when a runtime call fails,
+what it allocates and waits for, and which launch shapes it takes.  The library
+runs on tests/cpp/hip_on_host.cpp, which serves its HIP calls from host memory
+(kernels do nothing) and makes chosen ones fail.  Every scenario runs in a
+process of its own."""
 import ctypes
 import os
 import subprocess
@@ -178,7 +179,52 @@ def s_room_for_checkpoints(host):
     host.clean()
 
 
+def _refused(f, *args):
+    from ql_dns_amd.capi import QLError
+    try:
+        f(*args)
+    except QLError as e:
+        return e.code == -1
+    return False
+
+
+def s_transform_on_default_shape(host):
+    from ql_dns_amd.capi import QLBatch
+    from ql_dns_amd.params import QLParams
+    for model in (0, 1, 2):
+        for NZ in (32, 64):
+            c = _context(model=model, NZ=NZ)
+            before = c.config()[0]
+            assert before["line"] == 64 and before["transform"] == 0
+            c.set_transform(NZ, 1)
+            assert c.config()[0]["transform"] == 1 and c.config()[0]["line"] == 256
+            c.steps(2)
+            c.set_transform(NZ, 0)
+            assert c.config()[0] == before
+            # a shape that was asked for stays
+            c.set_config(NZ, 64, 128)
+            assert _refused(c.set_transform, NZ, 1)
+            assert c.config()[0]["line"] == 64 and c.config()[0]["transform"] == 0
+            c.set_config(NZ, 128, 512)
+            c.set_transform(NZ, 1)
+            c.set_transform(NZ, 0)
+            assert c.config()[0]["line"] == 128 and c.config()[0]["transform"] == 0
+            c.close()
+    b = QLBatch([QLParams(NX=8, NY=8, NZ=NZ) for NZ in (32, 64, 64)])
+    b.set_transform(64, 1)
+    assert [g["transform"] for g in b.config()] == [0, 1] and [g["line"] for g in b.config()] == [64, 256]
+    b.close()
+    for kw in (dict(NZ=128), dict(NZ=32, precision=1)):
+        assert _refused(_context(**kw).set_transform, kw["NZ"], 1)
+
+
 # ---------------------------------------------------------------------------
+def test_matrix_core_transform_on_a_default_shape(runtime):
+    """ql_batch_set_transform takes a set no shape was asked for: it moves to the
+    workgroup kernel, which has the variant, and back."""
+    scenario(runtime, "transform_on_default_shape")
+
+
 def test_longer_forward_after_a_gradient_takes_no_more_memory(runtime):
     """The buffers an earlier backward left make way for checkpoints."""
     scenario(runtime, "room_for_checkpoints")
