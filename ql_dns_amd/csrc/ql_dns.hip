@@ -288,6 +288,7 @@ int configure(Batch &b, Group &g, int line, int target)
     g.target = target;
     g.MB = MB;
     g.W = W;
+    g.tail = g.own_tail >= 0 ? g.own_tail : default_tail(b.precision, g);
     drop_graphs(b);
     return QL_OK;
 }
@@ -425,9 +426,6 @@ int create_batch(Batch &b, const ql_params *ps, int nruns)
         QL_HIP(hipMemcpy(g.tw32, htw32.data(), sizeof(float2) * g.NZ, hipMemcpyHostToDevice));
         const Shape sh = default_shape(g.NZ, b.precision, g.nruns, g.modes);
         QL_RC(configure(b, g, sh.line, sh.target));
-        g.tail = sh.tail;
-        for (const qlk::RunParams &rp : g.h_rp)
-            if (rp.nwg * g.NZ > TAIL_ONE) g.tail = 0;
     }
     return QL_OK;
 }
@@ -1367,7 +1365,7 @@ int tune(Batch &b, int trial_steps, double *best_ms_out)
             if (rc) break;
         }
         g.dft = best_dft;
-        g.tail = best_tail;
+        g.own_tail = best_tail;
         g.own_shape = true;
         if (rc == QL_OK) rc = configure(b, g, best_line, best_target);
         total_best += best;
@@ -1960,10 +1958,10 @@ int ql_batch_set_transform(ql_batch *bt, int NZ, int transform)
             return fail(QL_ERR_ARG, "ql_batch_set_transform: unknown transform %d", transform);
         // the wavefront kernel has no matrix-core variant: a group that is on it by
         // default only moves to the workgroup kernel, and back with the radix transforms
-        Shape sh{g.line, g.target, g.tail};
+        Shape sh{g.line, g.target};
         if (!g.own_shape) {
             sh = default_shape(g.NZ, b.precision, g.nruns, g.modes);
-            if (transform == QL_TRANSFORM_DFT_MFMA && sh.line == LINE_WAVE) sh = Shape{DEFAULT_LINE, DEFAULT_TARGET, sh.tail};
+            if (transform == QL_TRANSFORM_DFT_MFMA && sh.line == LINE_WAVE) sh = Shape{DEFAULT_LINE, DEFAULT_TARGET};
         }
         if (transform == QL_TRANSFORM_DFT_MFMA && !dft_ok(g.NZ, b.precision, sh.line))
             return fail(QL_ERR_ARG,
@@ -1987,7 +1985,7 @@ int ql_batch_set_tail(ql_batch *bt, int NZ, int tail)
             return fail(QL_ERR_ARG,
                         "ql_batch_set_tail: the one-launch tail needs fixed steps, NZ <= 128 and at most %ld "
                         "partial rows per run (NZ %d)", TAIL_MAX_ROWS_NZ / g.NZ, g.NZ);
-        g.tail = tail;
+        g.own_tail = tail;
         return configure(b, g, g.line, g.target);
     }
     return fail(QL_ERR_ARG, "ql_batch_set_tail: no group with NZ = %d", NZ);

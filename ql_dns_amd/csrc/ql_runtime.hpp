@@ -66,30 +66,21 @@ inline int mb_for(int NZ, int line) { return (line == LINE_WAVE || NZ >= line) ?
 //                  against 82.7);
 //   few modes      at least 64 workgroups, then four modes each: fewer rows for
 //                  the tail to sum (32x32x64: 124 workgroups 39.9, 248 41.8);
-//   tail           one launch at NZ <= 64 and at most TAIL_ONE / NZ rows per run,
-//                  which saves a launch (2-4 us per step); with more rows (NZ =
-//                  64, 504 rows: 78.4 against 77.5) or longer ones (NZ = 128, 252
-//                  rows: 116 against 109; 60 rows: 55.2 against 53.0) its
-//                  workgroups read too much each (36x60x64 MHD_BQlin with noise, 100 CN
-//                  steps: 5.46 -> 5.24 ms).
 // Groups of more than SMALL_SET runs fill the chip and share it with the other
 // groups: there eight (four) modes per pass and two launches measured best (48
 // runs: 160.0 us per step; wavefront kernel at NZ = 64 164.0, one-launch tail
 // 166-172; at 8 runs the one-launch tail won, 97.6 -> 79.0).
-constexpr int SMALL_SET = 4, SMALL_MODES = 512, TAIL_ONE = 16384;
+constexpr int SMALL_SET = 4, SMALL_MODES = 512;
 struct Shape {
-    int line, target, tail;
+    int line, target;
 };
+inline bool small_set(int precision, int nruns) { return precision == QL_PREC_FP64 && nruns <= SMALL_SET; }
 inline Shape default_shape(int NZ, int precision, int nruns, int modes)
 {
-    const bool small = precision == QL_PREC_FP64 && nruns <= SMALL_SET;
-    const int tail = small && NZ <= 64 ? 1 : 0;
-    if (NZ >= 128) return Shape{LINE_WAVE, 256, tail};
-    if (small && (NZ == 64 || modes <= SMALL_MODES)) {
-        const int target = modes / 4 < 64 ? 64 : (modes / 4 < 256 ? modes / 4 : 256);
-        return Shape{LINE_WAVE, target, tail};
-    }
-    return Shape{DEFAULT_LINE, DEFAULT_TARGET, tail};
+    if (NZ >= 128) return Shape{LINE_WAVE, 256};
+    if (small_set(precision, nruns) && (NZ == 64 || modes <= SMALL_MODES))
+        return Shape{LINE_WAVE, modes / 4 < 64 ? 64 : (modes / 4 < 256 ? modes / 4 : 256)};
+    return Shape{DEFAULT_LINE, DEFAULT_TARGET};
 }
 // the matrix-core transform (QL_TRANSFORM_DFT_MFMA): FP64 workgroup kernel, NZ 32 and 64
 inline bool dft_ok(int NZ, int precision, int line)
@@ -121,8 +112,9 @@ struct Group {
     double2 *mf = nullptr, *mfN1 = nullptr, *mfN2 = nullptr, *drive = nullptr, *tw = nullptr;
     // the substep tail as one launch (k_mf_fused) where it applies; it writes
     // the mean fields of substeps 1 and 2 to mfc1, mfc2 and those of substep 3
-    // to mf, so mf holds them at the end of every step
-    int tail = 0;
+    // to mf, so mf holds them at the end of every step.  own_tail: asked for
+    // (ql_batch_set_tail) or tuned, -1: the rule's for the shape (default_tail)
+    int tail = 0, own_tail = -1;
     double2 *mfc1 = nullptr, *mfc2 = nullptr;
     float2 *tw32 = nullptr;
     double *kx0 = nullptr, *ky = nullptr, *kzv = nullptr, *mfz = nullptr, *part = nullptr, *sums = nullptr;
@@ -146,6 +138,22 @@ struct Group {
     unsigned char *hi = nullptr;     // [modes] the modes the companion takes
     bool amp_stale = true;           // a state was uploaded (or the fraction changed) since the flags were set
 };
+
+// The substep tail of a group whose shape is set: one launch for small FP64 sets
+// at NZ <= 64 and at most TAIL_ONE / NZ rows per run, which saves a launch (2-4 us
+// per step; 36x60x64 MHD_BQlin with noise, 100 CN steps: 5.46 -> 5.24 ms).  With more
+// rows its workgroups read too much each: us per step of 64x64x64 with one launch
+// and with two, 252 rows 48.1 and 48.1, 504 rows 64.1 and 60.5, 1008 rows 74.3 and
+// 61.5.  Rows of NZ = 128 are too long: 252 of them 116 and 109, 60 of them 55.2
+// and 53.0.
+constexpr int TAIL_ONE = 16384;
+inline int default_tail(int precision, const Group &g)
+{
+    if (!small_set(precision, g.nruns) || g.NZ > 64) return 0;
+    for (const qlk::RunParams &rp : g.h_rp)
+        if ((rp.nwg + rp.nwg2) * g.NZ > TAIL_ONE) return 0;
+    return 1;
+}
 
 // mixed precision: a mode runs in FP64 when its amplitude reaches this
 // fraction of its run's largest (measured at 128x128x256 over 2000 steps: 29

@@ -218,7 +218,47 @@ def s_transform_on_default_shape(host):
         assert _refused(_context(**kw).set_transform, kw["NZ"], 1)
 
 
+def s_tail_follows_the_shape(host):
+    from ql_dns_amd.params import QLParams
+    c = _context(NX=36, NY=60, NZ=64)
+
+    def tail(line, target):
+        c.set_config(64, line, target)
+        g = c.config()[0]
+        return g["tail"], g["workgroups"] * 64
+
+    start = c.config()[0]
+    assert start["tail"] == 1
+    # one launch up to 16384 / NZ rows, two above, whatever the shape before
+    for line, target in ((64, 256), (256, 512), (128, 4096), (64, 256), (64, 1 << 30), (128, 256), (64, 512)):
+        t, rows = tail(line, target)
+        assert t == (1 if rows <= 16384 else 0), (line, target, rows)
+    # a tail that was asked for stays as far as it fits (65536 / NZ rows)
+    c.set_tail(64, 1)
+    assert tail(64, 512)[0] == 1 and tail(64, 1 << 30)[0] == 0 and tail(64, 512)[0] == 1
+    c.set_tail(64, 0)
+    assert tail(64, 256)[0] == 0
+    c.close()
+    # never by rule: variable steps, larger sets, mixed precision, NZ above 64
+    for kw in (dict(NZ=64, dt=-0.01), dict(NZ=64, precision=1), dict(NZ=128)):
+        c = _context(**kw)
+        c.set_config(kw["NZ"], 64, 64)
+        assert c.config()[0]["tail"] == 0
+        c.close()
+    from ql_dns_amd.capi import QLBatch
+    b = QLBatch([QLParams(NX=8, NY=8, NZ=32)] * 5)
+    b.set_config(32, 64, 64)
+    assert b.config()[0]["tail"] == 0
+    b.close()
+
+
 # ---------------------------------------------------------------------------
+def test_default_tail_follows_the_shape(runtime):
+    """The one-launch tail a set has by default is a matter of the shape it has now,
+    not of the one it was created with."""
+    scenario(runtime, "tail_follows_the_shape")
+
+
 def test_matrix_core_transform_on_a_default_shape(runtime):
     """ql_batch_set_transform takes a set no shape was asked for: it moves to the
     workgroup kernel, which has the variant, and back."""
