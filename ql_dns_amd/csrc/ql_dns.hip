@@ -275,15 +275,16 @@ int configure(Batch &b, Group &g, int line, int target)
     const int ncols = (b.nMF) * g.NZ;
     if (W + W2 > g.wg_cap) {
         dfree(g.wg), dfree(g.wg2), dfree(g.part);
-        QL_RC(dalloc(&g.wg, W + W2));
-        QL_RC(dalloc(&g.wg2, W + W2));
-        QL_RC(dalloc(&g.part, (size_t)(W + W2) * ncols));
+        QL_RC(dalloc_queued(&g.wg, W + W2));
+        QL_RC(dalloc_queued(&g.wg2, W + W2));
+        QL_RC(dalloc_queued(&g.part, (size_t)(W + W2) * ncols));
         g.wg_cap = W + W2;
     }
     QL_HIP(hipMemcpy(g.wg, wi.data(), sizeof(qlk::WgInfo) * W, hipMemcpyHostToDevice));
     if (W2) QL_HIP(hipMemcpy(g.wg2, wi2.data(), sizeof(qlk::WgInfo) * W2, hipMemcpyHostToDevice));
     g.W2 = W2;
     QL_HIP(hipMemcpy(g.rp, g.h_rp.data(), sizeof(qlk::RunParams) * g.nruns, hipMemcpyHostToDevice));
+    QL_RC(dwait());  // the clearings, these and with a new set all before (the copies have left little to wait for)
     g.line = line;
     g.target = target;
     g.MB = MB;
@@ -357,46 +358,46 @@ int create_batch(Batch &b, const ql_params *ps, int nruns)
     QL_HIP(hipStreamCreateWithFlags(&b.s, hipStreamNonBlocking));
     QL_HIP(hipEventCreateWithFlags(&b.fork, hipEventDisableTiming));
     for (auto &e : b.ev) QL_HIP(hipEventCreate(&e));
-    QL_RC(dalloc(&b.dpart, (size_t)256 * 6));
-    QL_RC(dalloc(&b.dout, (size_t)18));
-    QL_RC(dalloc(&b.mfr_tmp, (size_t)4 * 256));
+    QL_RC(dalloc_queued(&b.dpart, (size_t)256 * 6));
+    QL_RC(dalloc_queued(&b.dout, (size_t)18));
+    QL_RC(dalloc_queued(&b.mfr_tmp, (size_t)4 * 256));
     size_t lin = 0, tail = sizeof(double) * 4 * 256;
     for (const RunInfo &r : b.runs) {
         lin = std::max(lin, sizeof(double2) * r.nxy * ext_nlin(b) * r.nz);
         tail = std::max(tail, sizeof(double2) * 4 * r.nz + sizeof(double) * std::max(r.nxy, qlk::NT));
     }
-    QL_RC(staging_create(&b.out, lin, tail));
+    staging_create(&b.out, lin, tail);
     for (Group &g : b.groups) {
         if (b.groups.size() > 1) {
             QL_HIP(hipStreamCreateWithFlags(&g.s, hipStreamNonBlocking));
             QL_HIP(hipEventCreateWithFlags(&g.join, hipEventDisableTiming));
         }
         const size_t nl = (size_t)g.modes * 4 * g.nz, nm = (size_t)g.nruns * b.nMF * g.nz;
-        QL_RC(dalloc(&g.u, nl));
-        QL_RC(dalloc(&g.N1, nl));
-        QL_RC(dalloc(&g.N2, nl));
-        QL_RC(dalloc(&g.mf, nm));
-        QL_RC(dalloc(&g.mfc1, nm));
-        QL_RC(dalloc(&g.mfc2, nm));
-        QL_RC(dalloc(&g.mfN1, nm));
-        QL_RC(dalloc(&g.mfN2, nm));
-        QL_RC(dalloc(&g.drive, nm));
-        QL_RC(dalloc(&g.tw, g.NZ));
-        QL_RC(dalloc(&g.tw32, g.NZ));
-        QL_RC(dalloc(&g.kx0, g.modes));
-        QL_RC(dalloc(&g.ky, g.modes));
-        QL_RC(dalloc(&g.kzv, g.nz));
-        QL_RC(dalloc(&g.mfz, (size_t)g.nruns * 8 * g.NZ));
-        QL_RC(dalloc(&g.sums, (size_t)g.nruns * b.nMF * g.NZ));
-        QL_RC(dalloc(&g.rp, g.nruns));
-        QL_RC(dalloc(&g.pm, (size_t)g.nruns * qlk::PM_STRIDE));
-        QL_RC(dalloc(&g.mode_run, g.modes));
-        QL_RC(dalloc(&g.np, g.nruns));
-        QL_RC(dalloc(&g.clock, g.nruns));
+        QL_RC(dalloc_queued(&g.u, nl));
+        QL_RC(dalloc_queued(&g.N1, nl));
+        QL_RC(dalloc_queued(&g.N2, nl));
+        QL_RC(dalloc_queued(&g.mf, nm));
+        QL_RC(dalloc_queued(&g.mfc1, nm));
+        QL_RC(dalloc_queued(&g.mfc2, nm));
+        QL_RC(dalloc_queued(&g.mfN1, nm));
+        QL_RC(dalloc_queued(&g.mfN2, nm));
+        QL_RC(dalloc_queued(&g.drive, nm));
+        QL_RC(dalloc_queued(&g.tw, g.NZ));
+        QL_RC(dalloc_queued(&g.tw32, g.NZ));
+        QL_RC(dalloc_queued(&g.kx0, g.modes));
+        QL_RC(dalloc_queued(&g.ky, g.modes));
+        QL_RC(dalloc_queued(&g.kzv, g.nz));
+        QL_RC(dalloc_queued(&g.mfz, (size_t)g.nruns * 8 * g.NZ));
+        QL_RC(dalloc_queued(&g.sums, (size_t)g.nruns * b.nMF * g.NZ));
+        QL_RC(dalloc_queued(&g.rp, g.nruns));
+        QL_RC(dalloc_queued(&g.pm, (size_t)g.nruns * qlk::PM_STRIDE));
+        QL_RC(dalloc_queued(&g.mode_run, g.modes));
+        QL_RC(dalloc_queued(&g.np, g.nruns));
+        QL_RC(dalloc_queued(&g.clock, g.nruns));
         g.split = b.precision == QL_PREC_MIXED;
         if (g.split) {
-            QL_RC(dalloc(&g.amp, g.modes));
-            QL_RC(dalloc(&g.hi, g.modes));
+            QL_RC(dalloc_queued(&g.amp, g.modes));
+            QL_RC(dalloc_queued(&g.hi, g.modes));
         }
         std::vector<double> kx0(g.modes), ky(g.modes);
         std::vector<int> mrun(g.modes);

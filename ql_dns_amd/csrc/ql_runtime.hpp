@@ -212,16 +212,28 @@ struct Batch {
     Staging *out = nullptr;  // pinned memory results leave through
 };
 
+// Device memory, cleared on the null stream, which the contexts' streams (created
+// hipStreamNonBlocking) do not wait for: whoever allocates waits (dwait) before the
+// first copy or launch on them, or the clearing could land after it.  Where many
+// buffers are allocated together one wait serves all (the 30 of a context: 0.24 ms
+// of 0.6 when each waited)
+template <typename T>
+int dalloc_queued(T **p, size_t n)
+{
+    QL_HIP(hipMalloc((void **)p, sizeof(T) * (n ? n : 1)));
+    QL_HIP(hipMemset(*p, 0, sizeof(T) * (n ? n : 1)));
+    return QL_OK;
+}
+inline int dwait()
+{
+    QL_HIP(hipStreamSynchronize(nullptr));
+    return QL_OK;
+}
 template <typename T>
 int dalloc(T **p, size_t n)
 {
-    QL_HIP(hipMalloc((void **)p, sizeof(T) * (n ? n : 1)));
-    // the clearing runs on the null stream, which the contexts' streams (created
-    // hipStreamNonBlocking) do not wait for: without the wait it could land after
-    // the first copy into the buffer
-    QL_HIP(hipMemset(*p, 0, sizeof(T) * (n ? n : 1)));
-    QL_HIP(hipStreamSynchronize(nullptr));
-    return QL_OK;
+    QL_RC(dalloc_queued(p, n));
+    return dwait();
 }
 
 template <typename T>

@@ -55,10 +55,11 @@ constexpr size_t OUT_SLOT = (size_t)2 << 20;
 constexpr int OUT_SLOTS = 8, OUT_THREADED = 3;
 
 // One context's pinned memory: the slots, then a tail for everything but the
-// fluctuations.  Where none can be had, host is null and results take the
-// runtime's own copies.
+// fluctuations, allocated with the first result that leaves through it.  Where
+// none can be had, host stays null and results take the runtime's own copies.
 struct Staging {
     std::mutex mu;  // calls of several threads on one context take turns
+    bool tried = false;
     char *host = nullptr;
     size_t slot = 0, tail = 0;
     int n = 0;
@@ -73,18 +74,26 @@ struct Staging {
 };
 
 // sized for the largest run's fluctuations (lin bytes) and tail
-inline int staging_create(Staging **out, size_t lin, size_t tail)
+inline void staging_create(Staging **out, size_t lin, size_t tail)
 {
     std::unique_ptr<Staging> s(new Staging);
     s->slot = std::min((lin + 255) / 256 * 256, OUT_SLOT);
     s->n = (int)std::min<size_t>((lin + s->slot - 1) / s->slot, OUT_SLOTS);
     s->tail = (tail + 255) / 256 * 256;
-    if (hipHostMalloc((void **)&s->host, s->slot * s->n + s->tail, hipHostMallocCoherent) != hipSuccess) {
-        (void)hipGetLastError();
-        s->host = nullptr;
-    }
-    for (int k = 0; k < s->n; ++k) QL_HIP(hipEventCreateWithFlags(&s->ev[k], hipEventDisableTiming));
     *out = s.release();
+}
+
+// the memory, and the events of several slots (with mu held)
+inline int staging_get(Staging &s)
+{
+    if (s.tried) return QL_OK;
+    for (int k = 0; s.n > 1 && k < s.n; ++k)
+        if (!s.ev[k]) QL_HIP(hipEventCreateWithFlags(&s.ev[k], hipEventDisableTiming));
+    if (hipHostMalloc((void **)&s.host, s.slot * s.n + s.tail, hipHostMallocCoherent) != hipSuccess) {
+        (void)hipGetLastError();
+        s.host = nullptr;
+    }
+    s.tried = true;
     return QL_OK;
 }
 
@@ -99,6 +108,7 @@ inline int state_out(Staging &sg, hipStream_t st, const double2 *u, int rows, in
     if (!k) nk = 0;
     const size_t row_bytes = sizeof(double2) * rowlen, mf_bytes = sizeof(double2) * nmf, k_bytes = sizeof(double) * nk;
     std::lock_guard<std::mutex> lock(sg.mu);
+    QL_RC(staging_get(sg));
     if (!sg.host || mf_bytes + k_bytes > sg.tail || (rows && row_bytes > sg.slot)) {
         if (rows)
             QL_HIP(hipMemcpy2DAsync(lin, row_bytes, u, sizeof(double2) * rowstride, row_bytes, rows,
