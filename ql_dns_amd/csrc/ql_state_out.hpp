@@ -15,7 +15,6 @@
 #include <memory>
 #include <mutex>
 #include <thread>
-#include <vector>
 
 #include "ql_runtime.hpp"
 
@@ -152,8 +151,11 @@ inline int state_out(Staging &sg, hipStream_t st, const double2 *u, int rows, in
     } else {
         std::atomic<int> ready{0}, next{0};
         std::atomic<bool> stop{false};
-        std::vector<std::atomic<int>> done(np);
-        for (auto &d : done) d.store(0, std::memory_order_relaxed);
+        // per slot, one past the last piece copied out of it (nothing here takes
+        // memory but the threads, which are done without where there is none: no
+        // exception may leave a call)
+        std::atomic<int> copied[OUT_SLOTS];
+        for (auto &d : copied) d.store(0, std::memory_order_relaxed);
         // a worker takes the next piece, waits until it has arrived and copies it
         auto work = [&]() {
             for (int c; (c = next.fetch_add(1)) < np;) {
@@ -162,16 +164,17 @@ inline int state_out(Staging &sg, hipStream_t st, const double2 *u, int rows, in
                     std::this_thread::yield();
                 }
                 copy(c);
-                done[c].store(1, std::memory_order_release);
+                copied[c % sg.n].store(c + 1, std::memory_order_release);
             }
         };
-        std::vector<std::thread> pool;
-        int issued = 0;
+        std::thread pool[OUT_SLOTS];
+        int workers = 0, issued = 0;
         auto run = [&]() -> int {
             for (int c = 0; c < np; ++c) {
                 // slots are filled again once they have been copied out
                 while (issued < np && issued < c + sg.n) {
-                    if (issued >= sg.n && !done[issued - sg.n].load(std::memory_order_acquire)) {
+                    if (issued >= sg.n &&
+                        copied[issued % sg.n].load(std::memory_order_acquire) != issued - sg.n + 1) {
                         if (issued > c) break;
                         std::this_thread::yield();
                         continue;
@@ -182,15 +185,16 @@ inline int state_out(Staging &sg, hipStream_t st, const double2 *u, int rows, in
                         // the first pieces are on their way: start the workers
                         const unsigned cpus = std::max(1u, std::thread::hardware_concurrency());
                         try {
-                            while ((int)pool.size() < std::min<int>(std::min(np, OUT_SLOTS), cpus)) pool.emplace_back(work);
+                            for (; workers < std::min<int>(std::min(np, OUT_SLOTS), cpus); ++workers)
+                                pool[workers] = std::thread(work);
                         } catch (...) {  // no more threads: those there are, or none, do it
                         }
                     }
                 }
                 QL_HIP(hipEventSynchronize(sg.ev[c % sg.n]));
-                if (pool.empty()) {
+                if (!workers) {
                     copy(c);
-                    done[c].store(1, std::memory_order_release);
+                    copied[c % sg.n].store(c + 1, std::memory_order_release);
                 } else {
                     ready.store(c + 1, std::memory_order_release);
                 }
@@ -199,7 +203,7 @@ inline int state_out(Staging &sg, hipStream_t st, const double2 *u, int rows, in
         };
         const int rc = run();
         if (rc != QL_OK) stop.store(true);
-        for (std::thread &t : pool) t.join();
+        for (int k = 0; k < workers; ++k) pool[k].join();
         if (rc != QL_OK) return rc;
     }
     if (nmf) std::memcpy(mf, sg.tail_ptr(), mf_bytes);

@@ -47,7 +47,9 @@ class Host:
         self.L.hoh_sizes.argtypes = [ctypes.POINTER(ctypes.c_size_t), ctypes.c_long]
 
     def __getattr__(self, name):
-        return getattr(self.L, "hoh_" + name)
+        f = getattr(self.L, "hoh_" + name)
+        setattr(self, name, f)
+        return f
 
     def sizes(self):
         n = self.L.hoh_sizes(None, 0)
@@ -285,7 +287,51 @@ def s_creation(host):
     b.close()
 
 
+def _downloads(c, lin, mf, kx0, before=lambda: None, after=lambda: None):
+    """get_state with nothing but the call itself between before() and after()."""
+    from ql_dns_amd.capi import _dp
+    got = np.zeros_like(lin), np.zeros_like(mf), np.zeros_like(kx0)
+    args = [c._h] + [_dp(a) for a in got]
+    before()
+    rc = c._L.ql_get_state(*args)
+    after()
+    c._check(rc)
+    for a, b in zip(got, (lin, mf, kx0)):
+        assert np.array_equal(a, b)
+
+
+def s_downloads(host, NX, NZ, model):
+    from ql_dns_amd.ic import mode_tables
+    from ql_dns_amd.params import QLParams
+    kw = dict(NX=NX, NY=NX, NZ=NZ, model=model)
+    kx0 = mode_tables(QLParams(**kw))[0]
+    c = _context(**kw)
+    lin, mf = _state(c)
+    for _ in range(3):
+        _downloads(c, lin, mf, kx0)
+    # no memory for what the copying takes on the host, a thread's start included
+    for k in range(1, 13):
+        _downloads(c, lin, mf, kx0, lambda: host.fail_new(k), lambda: host.fail_new(0))
+    c.close()
+    # no pinned memory, at the first result and after
+    host.fail_host(1)
+    c = _context(**kw)
+    _downloads(c, lin, mf, kx0)
+    _downloads(c, lin, mf, kx0)
+    assert host.host_live() == 0
+    c.steps(1)  # and the failure is not reported by a later call
+    c.close()
+    host.clean()
+
+
 # ---------------------------------------------------------------------------
+@pytest.mark.parametrize("NX,NZ,model", [(6, 32, 0), (34, 256, 0), (34, 256, 2), (70, 256, 0), (70, 256, 2)])
+def test_results_arrive_whole_or_without_an_exception(runtime, NX, NZ, model):
+    """States of one piece, of a few and of more than there are slots, in both
+    layouts: the same values whatever the host has no memory for."""
+    scenario(runtime, "downloads", NX, NZ, model)
+
+
 def test_creation_waits_once_and_pins_nothing(runtime):
     """A new context waits for the clearing of its buffers as a whole, not for each
     (30 waits took 0.24 ms of a small context's 0.6), and has no pinned memory."""
