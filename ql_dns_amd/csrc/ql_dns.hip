@@ -222,7 +222,6 @@ int comp_nwg(int nxy)
 // near-equal contiguous ranges
 int configure(Batch &b, Group &g, int line, int target)
 {
-    if (g.dft && !dft_ok(g.NZ, b.precision, line)) g.dft = 0;  // the shape has no matrix-core variant
     // the tables are rewritten below: nothing queued may still read them
     QL_RC(sync_all(b));
     const int MB = mb_for(g.NZ, line);
@@ -230,8 +229,9 @@ int configure(Batch &b, Group &g, int line, int target)
     for (int id : g.run_ids) total += (b.runs[id].nxy + MB - 1) / MB;
     const long gpw = std::max<long>(1, (total + target - 1) / target);
     std::vector<qlk::WgInfo> wi;
+    std::vector<qlk::RunParams> h_rp = g.h_rp;
     for (int k = 0; k < g.nruns; ++k) {
-        qlk::RunParams &rp = g.h_rp[k];
+        qlk::RunParams &rp = h_rp[k];
         const int ng = (rp.nxy + MB - 1) / MB;
         const int nw = (int)((ng + gpw - 1) / gpw);
         rp.wg_off = (int)wi.size();
@@ -253,10 +253,10 @@ int configure(Batch &b, Group &g, int line, int target)
     // (the wavefront kernel takes its flagged modes in FP64 itself,
     // k_wave_mix, and has no companion)
     std::vector<qlk::WgInfo> wi2;
-    for (qlk::RunParams &rp : g.h_rp) rp.wg_off2 = rp.nwg2 = 0;
+    for (qlk::RunParams &rp : h_rp) rp.wg_off2 = rp.nwg2 = 0;
     if (g.split && line != LINE_WAVE) {
         for (int k = 0; k < g.nruns; ++k) {
-            qlk::RunParams &rp = g.h_rp[k];
+            qlk::RunParams &rp = h_rp[k];
             const int nw2 = comp_nwg(rp.nxy);
             rp.wg_off2 = W + (int)wi2.size();
             rp.nwg2 = nw2;
@@ -274,12 +274,22 @@ int configure(Batch &b, Group &g, int line, int target)
     const int W2 = (int)wi2.size();
     const int ncols = (b.nMF) * g.NZ;
     if (W + W2 > g.wg_cap) {
-        dfree(g.wg), dfree(g.wg2), dfree(g.part);
-        QL_RC(dalloc_queued(&g.wg, W + W2));
-        QL_RC(dalloc_queued(&g.wg2, W + W2));
-        QL_RC(dalloc_queued(&g.part, (size_t)(W + W2) * ncols));
+        // the group keeps its shape, whose buffers these are, where the new ones
+        // cannot be had
+        qlk::WgInfo *wg = nullptr, *wg2 = nullptr;
+        double *part = nullptr;
+        const int rc = [&]() -> int {
+            QL_RC(dalloc_queued(&wg, W + W2));
+            QL_RC(dalloc_queued(&wg2, W + W2));
+            QL_RC(dalloc_queued(&part, (size_t)(W + W2) * ncols));
+            return QL_OK;
+        }();
+        if (rc == QL_OK) std::swap(g.wg, wg), std::swap(g.wg2, wg2), std::swap(g.part, part);
+        dfree(wg), dfree(wg2), dfree(part);
+        QL_RC(rc);
         g.wg_cap = W + W2;
     }
+    g.h_rp.swap(h_rp);
     QL_HIP(hipMemcpy(g.wg, wi.data(), sizeof(qlk::WgInfo) * W, hipMemcpyHostToDevice));
     if (W2) QL_HIP(hipMemcpy(g.wg2, wi2.data(), sizeof(qlk::WgInfo) * W2, hipMemcpyHostToDevice));
     g.W2 = W2;
@@ -289,6 +299,7 @@ int configure(Batch &b, Group &g, int line, int target)
     g.target = target;
     g.MB = MB;
     g.W = W;
+    if (!dft_ok(g.NZ, b.precision, line)) g.dft = 0;  // the shape has no matrix-core variant
     g.tail = g.own_tail >= 0 ? g.own_tail : default_tail(b.precision, g);
     drop_graphs(b);
     return QL_OK;
@@ -1968,8 +1979,11 @@ int ql_batch_set_transform(ql_batch *bt, int NZ, int transform)
             return fail(QL_ERR_ARG,
                         "ql_batch_set_transform: the matrix-core transform needs FP64, NZ 32 or 64 and line 128 "
                         "or 256 (NZ %d, line %d)", g.NZ, sh.line);
+        const int was = g.dft;
         g.dft = transform;
-        return configure(b, g, sh.line, sh.target);
+        const int rc = configure(b, g, sh.line, sh.target);
+        if (rc != QL_OK) g.dft = was;
+        return rc;
     }
     return fail(QL_ERR_ARG, "ql_batch_set_transform: no group with NZ = %d", NZ);
 }
@@ -1986,8 +2000,11 @@ int ql_batch_set_tail(ql_batch *bt, int NZ, int tail)
             return fail(QL_ERR_ARG,
                         "ql_batch_set_tail: the one-launch tail needs fixed steps, NZ <= 128 and at most %ld "
                         "partial rows per run (NZ %d)", TAIL_MAX_ROWS_NZ / g.NZ, g.NZ);
+        const int was = g.own_tail;
         g.own_tail = tail;
-        return configure(b, g, g.line, g.target);
+        const int rc = configure(b, g, g.line, g.target);
+        if (rc != QL_OK) g.own_tail = was;
+        return rc;
     }
     return fail(QL_ERR_ARG, "ql_batch_set_tail: no group with NZ = %d", NZ);
 }
@@ -2053,8 +2070,9 @@ int ql_batch_set_config(ql_batch *bt, int NZ, int line, int target)
     Batch &b = bt->b;
     for (Group &g : b.groups)
         if (g.NZ == NZ) {
+            QL_RC(configure(b, g, line, target));
             g.own_shape = true;
-            return configure(b, g, line, target);
+            return QL_OK;
         }
     return fail(QL_ERR_ARG, "ql_batch_set_config: no runs with NZ=%d", NZ);
 }

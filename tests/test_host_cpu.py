@@ -324,7 +324,34 @@ def s_downloads(host, NX, NZ, model):
     host.clean()
 
 
+def s_shape_without_memory(host, precision):
+    c = _context(NX=36, NY=60, NZ=64, precision=precision)
+    before, sizes = c.config(), host.sizes()
+    n0 = host.mallocs()
+    c.set_config(64, 128, 1 << 30)
+    nalloc = host.mallocs() - n0
+    after = c.config()
+    c.close()
+    assert nalloc == 3 and after != before
+    for k in range(1, nalloc + 1):
+        c = _context(NX=36, NY=60, NZ=64, precision=precision)
+        host.fail_malloc(k)
+        assert _fails(c.set_config, 64, 128, 1 << 30), k
+        assert c.config() == before and host.sizes() == sizes, k  # the shape it had, buffers and all
+        c.steps(1)
+        c.set_config(64, 128, 1 << 30)
+        assert c.config() == after
+        c.close()
+    host.clean()
+    assert host.live() == 0
+
+
 # ---------------------------------------------------------------------------
+@pytest.mark.parametrize("precision", [0, 1])
+def test_a_shape_there_is_no_memory_for_changes_nothing(runtime, precision):
+    scenario(runtime, "shape_without_memory", precision)
+
+
 @pytest.mark.parametrize("NX,NZ,model", [(6, 32, 0), (34, 256, 0), (34, 256, 2), (70, 256, 0), (70, 256, 2)])
 def test_results_arrive_whole_or_without_an_exception(runtime, NX, NZ, model):
     """States of one piece, of a few and of more than there are slots, in both
