@@ -1300,6 +1300,7 @@ int tune(Batch &b, int trial_steps, double *best_ms_out)
     struct Snap {
         double2 *u = nullptr, *mf = nullptr, *drive = nullptr;
         double *kx0 = nullptr, *pm = nullptr;
+        bool whole = false;  // holds the group's state
     };
     std::vector<Snap> snaps(b.groups.size());
     int rc = QL_OK;
@@ -1317,6 +1318,7 @@ int tune(Batch &b, int trial_steps, double *best_ms_out)
             hipMemcpyAsync(sn.drive, g.drive, sizeof(double2) * nm, hipMemcpyDeviceToDevice, b.s) != hipSuccess ||
             hipMemcpyAsync(sn.kx0, g.kx0, sizeof(double) * g.modes, hipMemcpyDeviceToDevice, b.s) != hipSuccess)
             rc = fail(QL_ERR_HIP, "tune: state snapshot failed");
+        sn.whole = rc == QL_OK;
     }
     double total_best = 0.0;
     const bool timing = b.timing;
@@ -1391,7 +1393,7 @@ int tune(Batch &b, int trial_steps, double *best_ms_out)
         Group &g = b.groups[gi];
         Snap &sn = snaps[gi];
         const size_t nl = (size_t)g.modes * 4 * g.nz, nm = (size_t)g.nruns * b.nMF * g.nz;
-        if (sn.u && sn.mf && sn.drive && sn.kx0) {
+        if (sn.whole) {
             if (hipMemcpyAsync(g.u, sn.u, sizeof(double2) * nl, hipMemcpyDeviceToDevice, b.s) != hipSuccess ||
                 hipMemcpyAsync(g.mf, sn.mf, sizeof(double2) * nm, hipMemcpyDeviceToDevice, b.s) != hipSuccess ||
                 hipMemcpyAsync(g.drive, sn.drive, sizeof(double2) * nm, hipMemcpyDeviceToDevice, b.s) != hipSuccess ||
@@ -1400,8 +1402,8 @@ int tune(Batch &b, int trial_steps, double *best_ms_out)
             g.amp_stale = true;
             if (rc == QL_OK) rc = refresh_profiles(b, g, b.s);
             // after the refresh, which rewrites the current-state maxima
-            if (sn.pm && hipMemcpyAsync(g.pm, sn.pm, sizeof(double) * g.nruns * qlk::PM_STRIDE,
-                                        hipMemcpyDeviceToDevice, b.s) != hipSuccess)
+            if (hipMemcpyAsync(g.pm, sn.pm, sizeof(double) * g.nruns * qlk::PM_STRIDE, hipMemcpyDeviceToDevice,
+                               b.s) != hipSuccess)
                 if (rc == QL_OK) rc = fail(QL_ERR_HIP, "tune: state restore failed");
         }
     }

@@ -346,7 +346,38 @@ def s_shape_without_memory(host, precision):
     assert host.live() == 0
 
 
+def s_tune_without_memory(host):
+    from ql_dns_amd.capi import QLBatch
+    from ql_dns_amd.params import QLParams
+    ps = [QLParams(NX=8, NY=6, NZ=NZ) for NZ in (32, 64)]
+    states = []
+    for r, p in enumerate(ps):
+        c = _context(NX=8, NY=6, NZ=p.NZ)
+        states.append(_state(c, r))
+        c.close()
+    for k in range(0, 11):  # five buffers per group
+        b = QLBatch(ps)
+        for r, st in enumerate(states):
+            b.set_state(r, *st)
+        live = host.live()
+        if k:
+            host.fail_malloc(k)
+            assert _fails(b.tune, 1), k
+            assert host.live() == live, k
+        else:
+            b.tune(1)
+        for r, (lin, mf) in enumerate(states):
+            l, m, _ = b.get_state(r)
+            assert np.array_equal(l, lin) and np.array_equal(m, mf), (k, r)
+        b.close()
+    host.clean()
+
+
 # ---------------------------------------------------------------------------
+def test_tuning_there_is_no_memory_for_keeps_the_state(runtime):
+    scenario(runtime, "tune_without_memory")
+
+
 @pytest.mark.parametrize("precision", [0, 1])
 def test_a_shape_there_is_no_memory_for_changes_nothing(runtime, precision):
     scenario(runtime, "shape_without_memory", precision)
