@@ -174,9 +174,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_
     const int tid = threadIdx.x;
     const Phys ph = a.ph;
     const double q = ph.q, Om = ph.omega, B0z = ph.B0z;
-    // d L / d coefficient and d L / d x of a dissipation operator coef * op(x),
-    // x = -kx^2 - ky^2 + kz2: -|x|^p for MHD_FullQlin, x itself for MHD_BQlin
-    const auto opv = [&](double x) { return BQ ? x : neg_abs_pow(x, ph.vo2); };
+    // d op / d x of a dissipation operator coef op(x), x = -kx^2 - ky^2 + kz2: -|x|^p
+    // for MHD_FullQlin, x itself for MHD_BQlin
     const auto opd = [&](double x) { return BQ ? 1.0 : neg_abs_pow_d(x, ph.vo2); };
     const double qt = to_sgpr(rn_mul(q, a.ts)), qdtl = to_sgpr(rn_mul(q, a.dtl));
     const double qt_old = to_sgpr(rn_mul(q, a.tso)), qdtl_old = to_sgpr(rn_mul(q, a.dtlo));
@@ -271,17 +270,20 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_
                     dxo_dq = (a.tso + a.dtlo) * ky;
                 }
             }
+            // the operators and their derivatives, which the pairs share
+            const double opn = P::op(xn, ph), dpn = opd(xn);
+            const double opo = MODE == MODE_CN ? P::op(xo, ph) : 0.0, dpo = MODE == MODE_CN ? opd(xo) : 0.0;
 #pragma unroll
             for (int pr = 0; pr < 2; ++pr) {
                 const double coef = pr == 0 ? ph.nu : ph.eta;
-                const double Ln = P::lin(pr, kxn, ky, kz2, ph);
+                const double Ln = P::lin(pr, opn, ph);
                 double gLn = 0.0, gLo = 0.0;
                 // factors of the update and of the two right-hand sides in it
                 double e, d = 1.0;
                 if constexpr (MODE == MODE_ELIN) {
                     e = exp(a.linC * Ln);
                 } else {
-                    const double Lo = a.oinit ? P::lin_init(pr, kxo, lap2, ph) : P::lin(pr, kxo_e, ky, kz2, ph);
+                    const double Lo = P::lin(pr, opo, ph);
                     d = 1.0 / (1.0 - a.linC * Ln);
                     e = (1 + a.linC * Lo) * d;
                 }
@@ -306,11 +308,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_
                     }
                 }
                 // L = coef * op(x): coefficient and kx(t) = kx0 + q t ky dependence
-                const double gc = gLn * opv(xn) + (MODE == MODE_CN ? gLo * opv(xo) : 0.0);
+                const double gc = gLn * opn + (MODE == MODE_CN ? gLo * opo : 0.0);
                 if (pr == 0) gnu += gc;
                 else geta += gc;
-                gq += gLn * coef * opd(xn) * (-2.0 * kxn) * ((a.ts + a.dtl) * ky);
-                if (MODE == MODE_CN) gq += gLo * coef * opd(xo) * (-2.0 * kxo_e) * dxo_dq;
+                gq += gLn * coef * dpn * (-2.0 * kxn) * ((a.ts + a.dtl) * ky);
+                if (MODE == MODE_CN) gq += gLo * coef * dpo * (-2.0 * kxo_e) * dxo_dq;
             }
             const double ilapF = (i == 0 && im == 0) ? 1.0 : 1.0 / (-kx * kx + lap2);
             if constexpr (!BQ) {

@@ -644,11 +644,20 @@ __device__ __forceinline__ void mode_wave_body(const ModeArgs &a)
                     for (int f = 0; f < 2 * P::NPAIR; ++f) np[f] = a.n_prev ? a.n_prev[off + f * NZD] : make_double2(0.0, 0.0);
                 }
                 const CC *T = bufc + m;
+                const double kxn = kx + qdtl * ky;
+                const double opn = P::op((-kxn * kxn - ky * ky) + kz2, ph);
+                double opo = 0.0;
+                if constexpr (MODE == MODE_CN) {
+                    // the "old" operator is the one of the previous substep (or
+                    // linearOPs_Init at t0)
+                    const double kxo = rn_add(kx0, rn_mul(qt_old, ky)), kxe = kxo + qdtl_old * ky;
+                    opo = P::op(st.oinit ? -kxo * kxo + lap2 : (-kxe * kxe - ky * ky) + kz2, ph);
+                }
     #pragma unroll
                 for (int pr = 0; pr < P::NPAIR; ++pr) {
                     double2 N0, N1;
                     P::rhs_pair(pr, T, LL::TLD, U0, U1, U2, U3, kx, ky, kzk, ilapF, ph, N0, N1);
-                    const double Ln = P::lin(pr, kx + qdtl * ky, ky, kz2, ph);
+                    const double Ln = P::lin(pr, opn, ph);
                     const size_t off0 = off + (2 * pr) * NZD, off1 = off0 + NZD;
                     if constexpr (MODE == MODE_RHS) {
                         if (a.n_out) {
@@ -672,15 +681,8 @@ __device__ __forceinline__ void mode_wave_body(const ModeArgs &a)
                         un0 = cscale(e, cadd(s0, u0));
                         un1 = cscale(e, cadd(s1, u1));
                     } else {
-                        // RK3CN.cpp:105-107, :141-143, :177-179; the "old" operator is
-                        // the one of the previous substep (or linearOPs_Init at t0)
-                        double Lo;
-                        const double kxo = rn_add(kx0, rn_mul(qt_old, ky));
-                        if (st.oinit) {
-                            Lo = P::lin_init(pr, kxo, lap2, ph);
-                        } else {
-                            Lo = P::lin(pr, kxo + qdtl_old * ky, ky, kz2, ph);
-                        }
+                        // RK3CN.cpp:105-107, :141-143, :177-179
+                        const double Lo = P::lin(pr, opo, ph);
                         const double denom = 1.0 / (1.0 - linC * Ln);
                         const double c1 = nlc1 * denom, co = (1 + linC * Lo) * denom;
                         double2 s0 = cscale(c1, N0), s1 = cscale(c1, N1);
