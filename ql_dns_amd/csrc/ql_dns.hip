@@ -489,6 +489,28 @@ void launch_mode_m(const Batch &b, const Group &g, const qlk::ModeArgs &a, hipSt
     }
 }
 
+// Whether the wavefront kernel of MHD_BQlin, whose eight lines take the most
+// registers and LDS, runs in its second variant (ALT; us per RK3CN_Elin step, ALT
+// against the first variant):
+//   NZ = 32   more workgroups than CUs: without the loads ahead of a mode (126
+//             registers instead of 155) two workgroups fit on a CU (48x48x32: 282
+//             workgroups 45.1 against 50.9, 564 56.0 against 63.4; 226 38.5 against
+//             37.3).  Not FP32 alone, which fits twice as it is;
+//   NZ = 256  few modes, where a mode's latency is the bound: z lines through LDS
+//             and no early loads (16x16 72.6 against 74.5, 32x32 79.0 against 81.2,
+//             64x64 131.2 against 129.5; FP32 alone, at two wavefronts per SIMD
+//             instead of one, up to more modes: 64x64 116.3 against 119.0, 128x128
+//             314.3 against 303.3)
+constexpr int CUS = 256, ALT_MODES = 512, ALT_MODES32 = 4096;
+bool wave_alt(const Batch &b, const Group &g, const qlk::ModeArgs &a)
+{
+    if (b.model != QL_MODEL_MHD_BQLIN) return false;
+    const bool mixed = b.precision == QL_PREC_MIXED, fp32 = mixed && a.split != qlk::SPLIT_LO;
+    if (g.NZ == 32) return !fp32 && g.W > CUS;
+    if (g.NZ == 256) return fp32 ? g.modes <= ALT_MODES32 : !mixed && g.modes <= ALT_MODES;
+    return false;
+}
+
 template <int NZ, int MODE>
 void launch_wave_m(const Batch &b, const Group &g, const qlk::ModeArgs &a, hipStream_t st)
 {
@@ -496,19 +518,22 @@ void launch_wave_m(const Batch &b, const Group &g, const qlk::ModeArgs &a, hipSt
     constexpr int TF = qlk::mode_waves<qlk::ModelFull>(NZ) * qlk::WAVE;
     constexpr int TH = qlk::mode_waves<qlk::ModelHD>(NZ) * qlk::WAVE;
     constexpr int TB = qlk::mode_waves<qlk::ModelBQ>(NZ) * qlk::WAVE;
-    const bool bq = b.model == QL_MODEL_MHD_BQLIN;
+    const bool bq = b.model == QL_MODEL_MHD_BQLIN, alt = wave_alt(b, g, a);
     // HD_fullU: the velocity-only policy (its magnetic fields are zero)
     if (b.precision == QL_PREC_MIXED && a.split == qlk::SPLIT_LO) {
         // flagged modes in FP64, the others in FP32, in one launch
         if (b.hd) launch_k(qlk::k_wave_mix<NZ, qlk::ModelHD, MODE>, g.W, TH, st, tm, a);
+        else if (alt) launch_k(qlk::k_wave_mix<NZ, qlk::ModelBQ, MODE, NZ == 32>, g.W, TB, st, tm, a);
         else if (bq) launch_k(qlk::k_wave_mix<NZ, qlk::ModelBQ, MODE>, g.W, TB, st, tm, a);
         else launch_k(qlk::k_wave_mix<NZ, qlk::ModelFull, MODE>, g.W, TF, st, tm, a);
     } else if (b.precision == QL_PREC_MIXED) {
         if (b.hd) launch_k(qlk::k_wave32<NZ, qlk::ModelHD, MODE>, g.W, TH, st, tm, a);
+        else if (alt) launch_k(qlk::k_wave32<NZ, qlk::ModelBQ, MODE, NZ == 256>, g.W, TB, st, tm, a);
         else if (bq) launch_k(qlk::k_wave32<NZ, qlk::ModelBQ, MODE>, g.W, TB, st, tm, a);
         else launch_k(qlk::k_wave32<NZ, qlk::ModelFull, MODE>, g.W, TF, st, tm, a);
     } else {
         if (b.hd) launch_k(qlk::k_wave64<NZ, qlk::ModelHD, MODE>, g.W, TH, st, tm, a);
+        else if (alt) launch_k(qlk::k_wave64<NZ, qlk::ModelBQ, MODE, NZ == 32 || NZ == 256>, g.W, TB, st, tm, a);
         else if (bq) launch_k(qlk::k_wave64<NZ, qlk::ModelBQ, MODE>, g.W, TB, st, tm, a);
         else launch_k(qlk::k_wave64<NZ, qlk::ModelFull, MODE>, g.W, TF, st, tm, a);
     }

@@ -334,7 +334,8 @@ struct WaveCompactDst {
 
 // MIXW (C = float2): mixed precision in one launch, each mode in FP64 when
 // its flag is set and in FP32 otherwise (no companion launch)
-template <int NZ, class P, class C, int MODE, int NW, bool SPL, bool MIXW = false>
+// ALT: the second variant of MHD_BQlin (wave_alt, beside its launch)
+template <int NZ, class P, class C, int MODE, int NW, bool SPL, bool MIXW = false, bool ALT = false>
 __device__ __forceinline__ void mode_wave_body(const ModeArgs &a)
 {
     typedef RealOf<C> R;
@@ -343,7 +344,7 @@ __device__ __forceinline__ void mode_wave_body(const ModeArgs &a)
     // lines at 128 only (at 256, two wavefronts per SIMD, they need more registers
     // than there are: 47.7 against 46.9 us); not the mixed kernel's FP64 modes, which
     // share their sums by z point with its FP32 ones
-    constexpr bool ROWS = sizeof(C) == 16 && !MIXW && (NZ == 128 || (NZ > 128 && P::NPAIR == 2));
+    constexpr bool ROWS = sizeof(C) == 16 && !MIXW && !ALT && (NZ == 128 || (NZ > 128 && P::NPAIR == 2));
     using L = WaveLayout<NZ, P, C, ROWS>;
     using PL = Plan2<NZ>;
     constexpr int NZD = D::nz;
@@ -372,7 +373,7 @@ __device__ __forceinline__ void mode_wave_body(const ModeArgs &a)
     // the registers are there (100 CN steps of 36x60x64 MHD_BQlin with noise 5.93 ->
     // 5.75 ms, the gradient of 200 steps of 32x32x64 30.05 -> 29.48); with more
     // slots they are not (200 steps of 64x128x128 21.8 -> 27.9 ms)
-    constexpr bool AHEAD = KI == 1 && (!SPL || MIXW);
+    constexpr bool AHEAD = KI == 1 && (!SPL || MIXW) && !ALT;
     double kxl = 0.0, kyl = 0.0;
     double2 ua[4], na[4];
     auto load_ahead = [&](int l) {
@@ -472,17 +473,19 @@ __device__ __forceinline__ void mode_wave_body(const ModeArgs &a)
             // opaque: keeps what depends on the lane (the profile loads) inside the
             // mode loop instead of in registers across it
             int ln = lane;
-            if constexpr (ROWS || NZ >= 256) asm volatile("" : "+v"(ln));
+            if constexpr (ROWS || (NZ >= 256 && !ALT)) asm volatile("" : "+v"(ln));
             const double kx0 = to_sgpr(AHEAD ? kxl : a.kx0[i]), ky = to_sgpr(AHEAD ? kyl : a.ky[i]);
             const double kx = to_sgpr(rn_add(kx0, rn_mul(qt, ky)));  // kx(t), MHD_FullQlin.cpp:727
             const size_t row = (size_t)i * 4 * NZD;
 
             // B: 1/lap2, 1/lapF and the base spectral fields (MHD_FullQlin.cpp:220-221,
             // 722-738), fac1D folded in
-            // (the loads of every slot of the lane together: one latency)
+            // (the loads of every slot of the lane together, one latency; ALT at
+            // several slots: each slot's before its use)
+            constexpr bool SLOTS = ALT && KI > 1;
             double2 ub[KI][4];
     #pragma unroll
-            for (int k = 0; k < KI; ++k) {
+            for (int k = 0; k < KI && !SLOTS; ++k) {
                 const size_t o = row + min(lane + k * WAVE, NZD - 1);
     #pragma unroll
                 for (int f = 0; f < 4; ++f) {
@@ -496,6 +499,11 @@ __device__ __forceinline__ void mode_wave_body(const ModeArgs &a)
                 if (k > 0) __builtin_amdgcn_sched_barrier(0);  // one slot at a time (registers)
                 const int m = lane + k * WAVE;
                 if (KI * WAVE == NZD || m < NZD) {
+                    if constexpr (SLOTS) {
+    #pragma unroll
+                        for (int f = 0; f < 4; ++f)
+                            ub[k][f] = f < 2 * P::NPAIR ? a.u[row + f * NZD + m] : make_double2(0.0, 0.0);
+                    }
                     const double2 u0 = ub[k][0], u1 = ub[k][1], u2 = ub[k][2], u3 = ub[k][3];
                     const double kzk = skz[m], kz2 = -(kzk * kzk);
                     const bool zero = (ky == 0.0 && m == 0);
@@ -510,7 +518,7 @@ __device__ __forceinline__ void mode_wave_body(const ModeArgs &a)
             // forward transforms where registers are left for them: at one wavefront
             // per SIMD (128x128x256: 114.6 -> 104.3 us) and for HD_fullU's half state at
             // NZ = 128 (17.2 -> 16.8); elsewhere they spill (33.6 against 24.3 us at NZ = 128)
-            constexpr bool EARLY = P::NPAIR == 1 ? ROWS && NZ == 128 : NZ >= 256;
+            constexpr bool EARLY = P::NPAIR == 1 ? ROWS && NZ == 128 : NZ >= 256 && !ALT;
             double2 uf[EARLY ? KI : 1][4], nf[EARLY ? KI : 1][4];
             auto load_early = [&]() {
     #pragma unroll
@@ -754,23 +762,23 @@ template <class P>
 constexpr int mode_waves(int NZ) { return NZ >= 256 && P::NPAIR == 2 ? 4 : 8; }
 template <class P>
 constexpr int wave_occ(int NZ) { return NZ >= 256 && P::NPAIR == 2 ? 1 : 2; }
-template <int NZ, class P, int MODE>
+template <int NZ, class P, int MODE, bool ALT = false>
 __global__ __launch_bounds__(mode_waves<P>(NZ) * WAVE) __attribute__((amdgpu_waves_per_eu(wave_occ<P>(NZ))))
 void k_wave64(ModeArgs a)
 {
-    mode_wave_body<NZ, P, double2, MODE, mode_waves<P>(NZ), false>(a);
+    mode_wave_body<NZ, P, double2, MODE, mode_waves<P>(NZ), false, false, ALT>(a);
 }
-template <int NZ, class P, int MODE>
+template <int NZ, class P, int MODE, bool ALT = false>
 __global__ __launch_bounds__(mode_waves<P>(NZ) * WAVE) __attribute__((amdgpu_waves_per_eu(wave_occ<P>(NZ))))
 void k_wave32(ModeArgs a)
 {
-    mode_wave_body<NZ, P, float2, MODE, mode_waves<P>(NZ), true>(a);
+    mode_wave_body<NZ, P, float2, MODE, mode_waves<P>(NZ), true, false, ALT>(a);
 }
-template <int NZ, class P, int MODE>
+template <int NZ, class P, int MODE, bool ALT = false>
 __global__ __launch_bounds__(mode_waves<P>(NZ) * WAVE) __attribute__((amdgpu_waves_per_eu(wave_occ<P>(NZ))))
 void k_wave_mix(ModeArgs a)
 {
-    mode_wave_body<NZ, P, float2, MODE, mode_waves<P>(NZ), true, true>(a);
+    mode_wave_body<NZ, P, float2, MODE, mode_waves<P>(NZ), true, true, ALT>(a);
 }
 
 }  // namespace qlk

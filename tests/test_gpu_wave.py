@@ -287,3 +287,56 @@ def test_default_shapes_match_oracle(model, NX, NY, NZ, runs):
         assert np.array_equal(kg, ko)
         assert rel_err(mg, mo) < TOL and rel_err(lg, lo) < TOL
     b.close()
+
+
+@pytest.mark.parametrize("integrator", [1, 0])
+@pytest.mark.parametrize("NX,NZ,line,target", [
+    (34, 32, 64, 200), (34, 32, 64, 1 << 30), (48, 32, 64, 400),  # one workgroup per CU, and more
+    (4, 256, 64, 256), (32, 256, 64, 256), (34, 256, 64, 256)])   # up to 512 modes, and more
+def test_both_variants_of_bqlin_match_oracle(integrator, NX, NZ, line, target):
+    """MHD_BQlin's wavefront kernel on both sides of the rule between its variants:
+    the right-hand side and steps."""
+    from ql_dns_amd.capi import QLContext
+    from ql_dns_amd.ic import initial_state
+    from ql_dns_amd.params import QLParams
+    from oracle.oracle import Oracle
+    p = QLParams(model=1, integrator=integrator, NX=NX, NY=NX, NZ=NZ, Ly=1.0)
+    lin, mf = initial_state(p)
+    o, g = Oracle.from_params(p, nthreads=8), QLContext(p)
+    g.set_config(NZ, line, target)
+    for x in (o, g):
+        x.set_state(lin, mf)
+        x.linear_ops_init(0.0)
+    for a, b in zip(g.rhs(0.1, 0.01), o.rhs(0.1, 0.01)):
+        assert rel_err(a, b) < 1e-10
+    assert g.steps(4, 0.0) == o.steps(4, 0.0)
+    (lo, mo, ko), (lg, mg, kg) = o.get_state(), g.get_state()
+    assert np.array_equal(kg, ko)
+    assert rel_err(mg, mo) < 1e-10 and rel_err(lg, lo) < 1e-10
+    assert rel_err(g.drive(), o.drive()) < 1e-10
+
+
+@pytest.mark.parametrize("NX,NZ,target,tau", [(34, 32, 200, 0.0), (34, 32, 1 << 30, 0.0), (34, 32, 1 << 30, 2.0),
+                                              (16, 256, 256, 2.0), (92, 256, 256, 2.0), (16, 256, 256, 0.0)])
+def test_both_variants_of_bqlin_in_mixed_precision(NX, NZ, target, tau):
+    """Against FP64 within the mixed-precision bars (drives and mean fields 1e-6,
+    fluctuations 1e-5), with the split and without (tau > 1)."""
+    from ql_dns_amd.capi import QLContext
+    from ql_dns_amd.ic import initial_state
+    from ql_dns_amd.params import QLParams
+    p = QLParams(model=1, NX=NX, NY=NX, NZ=NZ)
+    lin, mf = initial_state(p)
+    out = []
+    for precision in (0, 1):
+        c = QLContext(p.replace(precision=precision))
+        c.set_config(NZ, 64, target)
+        if precision and tau:
+            c.mixed_split(tau)
+        c.set_state(lin, mf)
+        c.linear_ops_init(0.0)
+        c.steps(8, 0.0)
+        out.append(c.get_state()[:2] + (c.drive(),))
+        c.close()
+    (la, ma, da), (lb, mb, db) = out
+    assert not np.array_equal(la, lb)
+    assert rel_err(mb, ma) < 1e-6 and rel_err(db, da) < 1e-6 and rel_err(lb, la) < 1e-5
