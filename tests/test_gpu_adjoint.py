@@ -435,3 +435,46 @@ def test_adjoint_of_many_and_few_modes(NX, NY, NZ):
     h = EPS * p.q
     L = [_loss_parts(p, *_run(p.replace(q=p.q + s * h), lin0, mf0, n), alpha)[0] for s in (1, -1)]
     assert abs(gpar[0] - (L[0] - L[1]) / (2 * h)) <= TOL * abs(gpar[0])
+
+
+@pytest.mark.parametrize("model,integrator,NX,NZ,noise", [
+    (1, 1, 46, 128, False), (1, 0, 34, 256, False), (1, 1, 34, 256, True), (2, 0, 46, 128, False), (2, 1, 34, 256, True),
+    (0, 0, 46, 128, True)])
+def test_adjoint_of_many_modes_in_every_model(model, integrator, NX, NZ, noise):
+    """Past the reverse mode kernel's 512 workgroups, where a workgroup takes several
+    groups of modes in turn and reuses what MHD_BQlin sums over a mode's wavefronts:
+    one state direction, q and nu, the bars above."""
+    from ql_dns_amd.capi import QLContext
+    from ql_dns_amd.ic import initial_state
+    p = _p(model=model, NX=NX, NY=NX, NZ=NZ, Ly=1.0, B0z=0.03 if model == 0 else 0.0, integrator=integrator,
+           nu=1 / 1500, eta=1 / 1200)
+    assert p.nxy > 512 * (256 // NZ)
+    drive = dict(f_noise=2.0, seed=0x5EED0012) if noise else None
+    n, every = 4, 3
+    lin0, mf0 = initial_state(p)
+    alpha = 0.01 / float((np.abs(lin0) ** 2).sum())
+    c = QLContext(p)
+    if drive:
+        c.set_noise(**drive)
+    c.set_state(lin0, mf0)
+    c.linear_ops_init(0.0)
+    c.adjoint_forward(n, every, 0.0)
+    linT, mfT, _ = c.get_state()
+    _, g_lin, g_mf = _loss_parts(p, linT, mfT, alpha)
+    gl0, gm0, gpar = c.adjoint_backward(g_lin, g_mf)
+    c.close()
+    rng = np.random.default_rng(13)
+    vl = (rng.standard_normal(lin0.shape) + 1j * rng.standard_normal(lin0.shape)) * np.sqrt(np.mean(np.abs(lin0) ** 2))
+    if model != 1:
+        vl[::p.NY // 2, 0::2, 0] = 0
+    vm = (rng.standard_normal(mf0.shape) + 1j * rng.standard_normal(mf0.shape)) * np.sqrt(np.mean(np.abs(mf0) ** 2))
+    ad = float(np.sum(gl0.real * vl.real + gl0.imag * vl.imag) + np.sum(gm0.real * vm.real + gm0.imag * vm.imag))
+    L = [_loss_parts(p, *_run(p, lin0 + s * EPS * vl, mf0 + s * EPS * vm, n, drive), alpha)[0] for s in (1, -1)]
+    assert abs(ad - (L[0] - L[1]) / (2 * EPS)) <= TOL * abs(ad)
+    for k, name in ((0, "q"), (2, "nu")):
+        h = EPS * getattr(p, name)
+        L = [_loss_parts(p, *_run(p.replace(**{name: getattr(p, name) + s * h}), lin0, mf0, n, drive), alpha)[0]
+             for s in (1, -1)]
+        if np.spacing(L[0]) / (2 * h) > TOL * abs(gpar[k]):
+            continue  # one rounding of the loss already moves the difference by more than the bar
+        assert abs(gpar[k] - (L[0] - L[1]) / (2 * h)) <= TOL * abs(gpar[k]), name
