@@ -372,12 +372,7 @@ int create_batch(Batch &b, const ql_params *ps, int nruns)
     QL_RC(dalloc_queued(&b.dpart, (size_t)256 * 6));
     QL_RC(dalloc_queued(&b.dout, (size_t)18));
     QL_RC(dalloc_queued(&b.mfr_tmp, (size_t)4 * 256));
-    size_t lin = 0, tail = sizeof(double) * 4 * 256;
-    for (const RunInfo &r : b.runs) {
-        lin = std::max(lin, sizeof(double2) * r.nxy * ext_nlin(b) * r.nz);
-        tail = std::max(tail, sizeof(double2) * 4 * r.nz + sizeof(double) * std::max(r.nxy, qlk::NT));
-    }
-    staging_create(&b.out, lin, tail);
+    b.out = new Staging;
     for (Group &g : b.groups) {
         if (b.groups.size() > 1) {
             QL_HIP(hipStreamCreateWithFlags(&g.s, hipStreamNonBlocking));

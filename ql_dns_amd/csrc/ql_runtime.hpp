@@ -209,7 +209,7 @@ struct Batch {
     std::vector<hipEvent_t> tpool;
     size_t tused = 0;
     AdjState *adj = nullptr;
-    Staging *out = nullptr;  // pinned memory results leave through
+    Staging *out = nullptr;  // results leave through it (ql_state_out.hpp)
 };
 
 // Device memory, cleared on the null stream, which the contexts' streams (created

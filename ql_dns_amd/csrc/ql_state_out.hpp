@@ -12,7 +12,6 @@
 #pragma once
 #include <atomic>
 #include <cstring>
-#include <memory>
 #include <mutex>
 #include <thread>
 
@@ -53,48 +52,92 @@ namespace qlh {
 constexpr size_t OUT_SLOT = (size_t)2 << 20;
 constexpr int OUT_SLOTS = 8, OUT_THREADED = 3;
 
-// One context's pinned memory: the slots, then a tail for everything but the
-// fluctuations, allocated with the first result that leaves through it.  Where
-// none can be had, host stays null and results take the runtime's own copies.
+// Pinned memory for results on their way: lent to one download at a time and kept
+// for the next one of any handle, since new pinned pages cost more than a download
+// where they are first touched.  First state of a handle, us, with memory of its
+// own -> lent (pageable copies): 36x60x64 1350 -> 200 (1370), 64x64x128 1740 -> 550
+// (2840), 64x128x128 2290 -> 1030 (1850), 128x128x256 3840 -> 2520 (8900).  At most
+// PINNED_KEPT buffers wait here, and with the last handle they go.  Two sizes:
+// records and small states take the small one.
+constexpr int PINNED_KEPT = 4;
+constexpr size_t PINNED_SMALL = (size_t)512 << 10, PINNED_LARGE = OUT_SLOT * OUT_SLOTS + ((size_t)1 << 20);
+
+struct PinnedPool {
+    struct Buffer {
+        char *host = nullptr;
+        size_t size = 0;
+    };
+    std::mutex mu;
+    int handles = 0, kept = 0;
+    Buffer buf[PINNED_KEPT];
+
+    void open()
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        ++handles;
+    }
+    void close()
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        if (--handles > 0) return;
+        for (; kept > 0; --kept) (void)hipHostFree(buf[kept - 1].host);
+    }
+    // the smallest kept buffer of at least size bytes, or a new one (host null:
+    // none can be had)
+    Buffer take(size_t size)
+    {
+        size = size <= PINNED_SMALL ? PINNED_SMALL : std::max(size, PINNED_LARGE);
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            int best = -1;
+            for (int k = 0; k < kept; ++k)
+                if (buf[k].size >= size && (best < 0 || buf[k].size < buf[best].size)) best = k;
+            if (best >= 0) {
+                const Buffer b = buf[best];
+                buf[best] = buf[--kept];
+                return b;
+            }
+        }
+        Buffer b;
+        b.size = size;
+        if (hipHostMalloc((void **)&b.host, size, hipHostMallocCoherent | hipHostMallocPortable) != hipSuccess) {
+            (void)hipGetLastError();
+            b.host = nullptr;
+        }
+        return b;
+    }
+    void give(const Buffer &b)
+    {
+        if (!b.host) return;
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            if (kept < PINNED_KEPT && handles > 0 && b.size <= PINNED_LARGE) {
+                buf[kept++] = b;
+                return;
+            }
+        }
+        (void)hipHostFree(b.host);
+    }
+};
+// one per process, never destroyed: handles may be released while it ends
+inline PinnedPool &pinned_pool()
+{
+    static PinnedPool *const p = new PinnedPool;
+    return *p;
+}
+
+// One handle's part in it
 struct Staging {
-    std::mutex mu;  // calls of several threads on one context take turns
-    bool tried = false;
-    char *host = nullptr;
-    size_t slot = 0, tail = 0;
-    int n = 0;
-    hipEvent_t ev[OUT_SLOTS] = {};
-    char *tail_ptr() const { return host + slot * n; }
+    std::mutex mu;  // calls of several threads on one handle take turns
+    hipEvent_t ev[OUT_SLOTS] = {};  // with the first result of several pieces
+    Staging() { pinned_pool().open(); }
     ~Staging()
     {
         for (hipEvent_t e : ev)
             if (e) (void)hipEventDestroy(e);
-        if (host) (void)hipHostFree(host);
+        pinned_pool().close();
     }
 };
-
-// sized for the largest run's fluctuations (lin bytes) and tail
-inline void staging_create(Staging **out, size_t lin, size_t tail)
-{
-    std::unique_ptr<Staging> s(new Staging);
-    s->slot = std::min((lin + 255) / 256 * 256, OUT_SLOT);
-    s->n = (int)std::min<size_t>((lin + s->slot - 1) / s->slot, OUT_SLOTS);
-    s->tail = (tail + 255) / 256 * 256;
-    *out = s.release();
-}
-
-// the memory, and the events of several slots (with mu held)
-inline int staging_get(Staging &s)
-{
-    if (s.tried) return QL_OK;
-    for (int k = 0; s.n > 1 && k < s.n; ++k)
-        if (!s.ev[k]) QL_HIP(hipEventCreateWithFlags(&s.ev[k], hipEventDisableTiming));
-    if (hipHostMalloc((void **)&s.host, s.slot * s.n + s.tail, hipHostMallocCoherent) != hipSuccess) {
-        (void)hipGetLastError();
-        s.host = nullptr;
-    }
-    s.tried = true;
-    return QL_OK;
-}
 
 // rows of rowlen values, rowstride apart from u on, to lin; nmf values to mf and
 // nk doubles to k (each left out where its destination is null), in stream
@@ -106,9 +149,27 @@ inline int state_out(Staging &sg, hipStream_t st, const double2 *u, int rows, in
     if (!mf) nmf = 0;
     if (!k) nk = 0;
     const size_t row_bytes = sizeof(double2) * rowlen, mf_bytes = sizeof(double2) * nmf, k_bytes = sizeof(double) * nk;
+    const int per = rows ? (int)std::min<size_t>(OUT_SLOT / row_bytes, rows) : 0;
+    const int np = rows ? (rows + per - 1) / per : 0;  // pieces
+    const int n = std::max(1, std::min(np, OUT_SLOTS));  // slots
+    const size_t slot = (per * row_bytes + 255) / 256 * 256;
     std::lock_guard<std::mutex> lock(sg.mu);
-    QL_RC(staging_get(sg));
-    if (!sg.host || mf_bytes + k_bytes > sg.tail || (rows && row_bytes > sg.slot)) {
+    for (int k = 0; np > 1 && k < n; ++k)
+        if (!sg.ev[k]) QL_HIP(hipEventCreateWithFlags(&sg.ev[k], hipEventDisableTiming));
+    // the slots, then everything but the fluctuations
+    struct Lent {
+        PinnedPool::Buffer b;
+        hipStream_t st;
+        bool whole = false;  // nothing queued writes it any more
+        ~Lent()
+        {
+            if (!whole) (void)hipStreamSynchronize(st);
+            pinned_pool().give(b);
+        }
+    } lent{pinned_pool().take(slot * n + mf_bytes + k_bytes), st};
+    char *const host = lent.b.host, *const tail = host + slot * n;
+    if (!host) {
+        lent.whole = true;
         if (rows)
             QL_HIP(hipMemcpy2DAsync(lin, row_bytes, u, sizeof(double2) * rowstride, row_bytes, rows,
                                     hipMemcpyDeviceToHost, st));
@@ -117,31 +178,29 @@ inline int state_out(Staging &sg, hipStream_t st, const double2 *u, int rows, in
         QL_HIP(hipStreamSynchronize(st));
         return QL_OK;
     }
-    const int per = rows ? (int)std::min<size_t>(sg.slot / row_bytes, rows) : 0;
-    const int np = rows ? (rows + per - 1) / per : 0;  // pieces
     auto issue = [&](int c) -> int {
         qlk::StateOut a{};
         a.u = u + (size_t)c * per * rowstride;
         a.rows = rows ? std::min(per, rows - c * per) : 0;
         a.rowlen = rowlen;
         a.rowstride = rowstride;
-        a.dst = reinterpret_cast<double2 *>(sg.host + sg.slot * (c % sg.n));
+        a.dst = reinterpret_cast<double2 *>(host + slot * (c % n));
         if (c == 0) {
             a.mf = mf_src;
             a.nmf = nmf;
-            a.dst_mf = reinterpret_cast<double2 *>(sg.tail_ptr());
+            a.dst_mf = reinterpret_cast<double2 *>(tail);
             a.k = k_src;
             a.nk = nk;
-            a.dst_k = reinterpret_cast<double *>(sg.tail_ptr() + mf_bytes);
+            a.dst_k = reinterpret_cast<double *>(tail + mf_bytes);
         }
         const int work = std::max(std::max(a.rows * rowlen, a.nmf), a.nk);
         qlk::k_state_out<<<std::max(1, std::min((work + qlk::NT - 1) / qlk::NT, 512)), qlk::NT, 0, st>>>(a);
         QL_HIP(hipGetLastError());
-        if (np > 1) QL_HIP(hipEventRecord(sg.ev[c % sg.n], st));
+        if (np > 1) QL_HIP(hipEventRecord(sg.ev[c % n], st));
         return QL_OK;
     };
     auto copy = [&](int c) {
-        std::memcpy(static_cast<char *>(lin) + (size_t)c * per * row_bytes, sg.host + sg.slot * (c % sg.n),
+        std::memcpy(static_cast<char *>(lin) + (size_t)c * per * row_bytes, host + slot * (c % n),
                     row_bytes * std::min(per, rows - c * per));
     };
     if (np <= 1) {
@@ -164,7 +223,7 @@ inline int state_out(Staging &sg, hipStream_t st, const double2 *u, int rows, in
                     std::this_thread::yield();
                 }
                 copy(c);
-                copied[c % sg.n].store(c + 1, std::memory_order_release);
+                copied[c % n].store(c + 1, std::memory_order_release);
             }
         };
         std::thread pool[OUT_SLOTS];
@@ -172,16 +231,16 @@ inline int state_out(Staging &sg, hipStream_t st, const double2 *u, int rows, in
         auto run = [&]() -> int {
             for (int c = 0; c < np; ++c) {
                 // slots are filled again once they have been copied out
-                while (issued < np && issued < c + sg.n) {
-                    if (issued >= sg.n &&
-                        copied[issued % sg.n].load(std::memory_order_acquire) != issued - sg.n + 1) {
+                while (issued < np && issued < c + n) {
+                    if (issued >= n &&
+                        copied[issued % n].load(std::memory_order_acquire) != issued - n + 1) {
                         if (issued > c) break;
                         std::this_thread::yield();
                         continue;
                     }
                     QL_RC(issue(issued));
                     ++issued;
-                    if (c == 0 && np >= OUT_THREADED && issued == std::min(np, sg.n)) {
+                    if (c == 0 && np >= OUT_THREADED && issued == std::min(np, n)) {
                         // the first pieces are on their way: start the workers
                         const unsigned cpus = std::max(1u, std::thread::hardware_concurrency());
                         try {
@@ -191,10 +250,10 @@ inline int state_out(Staging &sg, hipStream_t st, const double2 *u, int rows, in
                         }
                     }
                 }
-                QL_HIP(hipEventSynchronize(sg.ev[c % sg.n]));
+                QL_HIP(hipEventSynchronize(sg.ev[c % n]));
                 if (!workers) {
                     copy(c);
-                    copied[c % sg.n].store(c + 1, std::memory_order_release);
+                    copied[c % n].store(c + 1, std::memory_order_release);
                 } else {
                     ready.store(c + 1, std::memory_order_release);
                 }
@@ -206,8 +265,9 @@ inline int state_out(Staging &sg, hipStream_t st, const double2 *u, int rows, in
         for (int k = 0; k < workers; ++k) pool[k].join();
         if (rc != QL_OK) return rc;
     }
-    if (nmf) std::memcpy(mf, sg.tail_ptr(), mf_bytes);
-    if (nk) std::memcpy(k, sg.tail_ptr() + mf_bytes, k_bytes);
+    lent.whole = true;
+    if (nmf) std::memcpy(mf, tail, mf_bytes);
+    if (nk) std::memcpy(k, tail + mf_bytes, k_bytes);
     return QL_OK;
 }
 

@@ -268,11 +268,17 @@ def s_creation(host):
         c.get_state()
         assert host.host_live() == 1
         c.get_state()
-        c.diagnostics(0.0)
         assert host.host_live() == 1
+        d = QLContext(QLParams(**kw))
+        d.get_state()
+        assert host.host_live() == 1  # the next handle's results take what is there
+        c.close()
+        c = d
+        c.diagnostics(0.0)
+        assert host.host_live() <= 2
         host.clean()
         c.close()
-        assert host.live() == 0 and host.host_live() == 0
+        assert host.live() == 0 and host.host_live() == 0  # and it goes with the last
     n = host.null_waits()
     b = QLBatch([QLParams(NX=8, NY=8, NZ=(32, 64, 128)[k % 3]) for k in range(12)])
     assert host.null_waits() - n <= 4
@@ -314,13 +320,16 @@ def s_downloads(host, NX, NZ, model):
         _downloads(c, lin, mf, kx0, lambda: host.fail_new(k), lambda: host.fail_new(0))
     c.close()
     # no pinned memory, at the first result and after
-    host.fail_host(1)
     c = _context(**kw)
-    _downloads(c, lin, mf, kx0)
-    _downloads(c, lin, mf, kx0)
-    assert host.host_live() == 0
+    held = host.host_live()
+    for k in range(3):
+        host.fail_host(1)
+        _downloads(c, lin, mf, kx0)
+    assert host.host_live() == held
+    host.fail_host(0)
     c.steps(1)  # and the failure is not reported by a later call
     c.close()
+    assert host.host_live() == 0
     host.clean()
 
 
@@ -373,7 +382,36 @@ def s_tune_without_memory(host):
     host.clean()
 
 
+def s_threads(host):
+    from threading import Thread
+    cs = [_context(NX=NX, NY=NX, NZ=NZ) for NX, NZ in ((6, 32), (34, 256), (34, 256), (70, 256), (24, 256), (8, 64))]
+    want = [c.get_state() for c in cs]
+    bad = []
+
+    def work(k):
+        for _ in range(12):
+            if not all(np.array_equal(a, b) for a, b in zip(cs[k].get_state(), want[k])):
+                bad.append(k)
+
+    ts = [Thread(target=work, args=(k % len(cs),)) for k in range(2 * len(cs))]  # two threads per context
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad
+    for n, c in enumerate(cs):
+        assert 1 <= host.host_live() <= 4
+        c.close()
+    assert host.host_live() == 0
+    host.clean()
+
+
 # ---------------------------------------------------------------------------
+def test_downloads_of_several_threads(runtime):
+    """Threads on one context take turns, threads on several have memory of their own."""
+    scenario(runtime, "threads")
+
+
 def test_tuning_there_is_no_memory_for_keeps_the_state(runtime):
     scenario(runtime, "tune_without_memory")
 
