@@ -95,11 +95,11 @@ int check_adjoint(const Batch &b, const char *who)
 int alloc_ck(AdjState::Ck &c, const Group &g, size_t nl, size_t nm)
 {
     const int rc = [&]() -> int {
-        QL_RC(dalloc(&c.u, nl));
-        QL_RC(dalloc(&c.mf, nm));
-        QL_RC(dalloc(&c.kx0, g.modes));
-        QL_RC(dalloc(&c.pm, (size_t)qlk::PM_STRIDE));
-        return QL_OK;
+        QL_RC(dalloc_queued(&c.u, nl));
+        QL_RC(dalloc_queued(&c.mf, nm));
+        QL_RC(dalloc_queued(&c.kx0, g.modes));
+        QL_RC(dalloc_queued(&c.pm, (size_t)qlk::PM_STRIDE));
+        return dwait();
     }();
     if (rc != QL_OK) free_ck(c);
     return rc;
@@ -268,13 +268,13 @@ int alloc_segment(AdjState *A, const Group &g, size_t nl, size_t nm)
 {
     const size_t K = A->every;
     const int rc = [&]() -> int {
-        QL_RC(dalloc(&A->st_u, nl * (3 * K + 1)));
-        QL_RC(dalloc(&A->st_mf, nm * (3 * K + 1)));
-        QL_RC(dalloc(&A->st_kx0, (size_t)g.modes * K));
+        QL_RC(dalloc_queued(&A->st_u, nl * (3 * K + 1)));
+        QL_RC(dalloc_queued(&A->st_mf, nm * (3 * K + 1)));
+        QL_RC(dalloc_queued(&A->st_kx0, (size_t)g.modes * K));
         // zeroed: MHD_BQlin writes 3 of the 8 profile lines
-        QL_RC(dalloc(&A->st_mfz, (size_t)8 * g.NZ * (3 * K + 1)));
-        if (g.noise) QL_RC(dalloc(&A->st_pre, nl * K));
-        return QL_OK;
+        QL_RC(dalloc_queued(&A->st_mfz, (size_t)8 * g.NZ * (3 * K + 1)));
+        if (g.noise) QL_RC(dalloc_queued(&A->st_pre, nl * K));
+        return dwait();
     }();
     if (rc != QL_OK) free_segment(A);
     return rc;
@@ -285,16 +285,16 @@ int alloc_adjoint(AdjState *A, const Group &g, size_t nl, size_t nm, int W)
 {
     const size_t ncols = 8 * g.NZ + qlk::NGP;
     const int rc = [&]() -> int {
-        QL_RC(dalloc(&A->gu, nl));
-        QL_RC(dalloc(&A->gnp, nl));
-        QL_RC(dalloc(&A->gM, nm));
-        QL_RC(dalloc(&A->gnmp, nm));
-        QL_RC(dalloc(&A->gsums, (size_t)4 * g.NZ));  // zeroed: MHD_BQlin fills 2 of the 4 lines
-        QL_RC(dalloc(&A->gpart, (size_t)W * ncols));
-        QL_RC(dalloc(&A->grows, ncols));
-        QL_RC(dalloc(&A->gpar_mf, (size_t)qlk::NGP));
-        QL_RC(dalloc(&A->gpar, (size_t)qlk::NGP));
-        return QL_OK;
+        QL_RC(dalloc_queued(&A->gu, nl));
+        QL_RC(dalloc_queued(&A->gnp, nl));
+        QL_RC(dalloc_queued(&A->gM, nm));
+        QL_RC(dalloc_queued(&A->gnmp, nm));
+        QL_RC(dalloc_queued(&A->gsums, (size_t)4 * g.NZ));  // zeroed: MHD_BQlin fills 2 of the 4 lines
+        QL_RC(dalloc_queued(&A->gpart, (size_t)W * ncols));
+        QL_RC(dalloc_queued(&A->grows, ncols));
+        QL_RC(dalloc_queued(&A->gpar_mf, (size_t)qlk::NGP));
+        QL_RC(dalloc_queued(&A->gpar, (size_t)qlk::NGP));
+        return dwait();
     }();
     if (rc != QL_OK) free_adjoint(A);
     return rc;

@@ -382,6 +382,20 @@ def s_tune_without_memory(host):
     host.clean()
 
 
+def s_gradient_waits(host):
+    c = _noisy_context(0)
+    c.adjoint_forward(4, 2, 0.0)
+    n = host.null_waits()
+    c.adjoint_backward()
+    assert host.null_waits() - n <= 2
+    n = host.null_waits()
+    c.adjoint_forward(6, 1, 0.0)  # four checkpoints more
+    assert host.null_waits() - n <= 4
+    c.adjoint_backward()
+    host.clean()
+    c.close()
+
+
 def s_threads(host):
     from threading import Thread
     cs = [_context(NX=NX, NY=NX, NZ=NZ) for NX, NZ in ((6, 32), (34, 256), (34, 256), (70, 256), (24, 256), (8, 64))]
@@ -407,6 +421,10 @@ def s_threads(host):
 
 
 # ---------------------------------------------------------------------------
+def test_gradients_wait_once_per_group_of_buffers(runtime):
+    scenario(runtime, "gradient_waits")
+
+
 def test_downloads_of_several_threads(runtime):
     """Threads on one context take turns, threads on several have memory of their own."""
     scenario(runtime, "threads")
