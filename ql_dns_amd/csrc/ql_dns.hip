@@ -431,7 +431,7 @@ int create_batch(Batch &b, const ql_params *ps, int nruns)
         QL_HIP(hipMemcpy(g.kzv, r0.h_kz.data(), sizeof(double) * g.nz, hipMemcpyHostToDevice));
         QL_HIP(hipMemcpy(g.tw, htw.data(), sizeof(double2) * g.NZ, hipMemcpyHostToDevice));
         QL_HIP(hipMemcpy(g.tw32, htw32.data(), sizeof(float2) * g.NZ, hipMemcpyHostToDevice));
-        const Shape sh = default_shape(g.NZ, b.precision, g.nruns, g.modes);
+        const Shape sh = default_shape(g.NZ, b.model, b.hd, b.precision, g.nruns, g.modes);
         QL_RC(configure(b, g, sh.line, sh.target));
     }
     return QL_OK;
@@ -1994,7 +1994,7 @@ int ql_batch_set_transform(ql_batch *bt, int NZ, int transform)
         // default only moves to the workgroup kernel, and back with the radix transforms
         Shape sh{g.line, g.target};
         if (!g.own_shape) {
-            sh = default_shape(g.NZ, b.precision, g.nruns, g.modes);
+            sh = default_shape(g.NZ, b.model, b.hd, b.precision, g.nruns, g.modes);
             if (transform == QL_TRANSFORM_DFT_MFMA && sh.line == LINE_WAVE) sh = Shape{DEFAULT_LINE, DEFAULT_TARGET};
         }
         if (transform == QL_TRANSFORM_DFT_MFMA && !dft_ok(g.NZ, b.precision, sh.line))

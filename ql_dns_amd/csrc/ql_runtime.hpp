@@ -60,7 +60,11 @@ inline int mb_for(int NZ, int line) { return (line == LINE_WAVE || NZ >= line) ?
 //   NZ >= 128      the wavefront kernel, about one workgroup per CU, for every
 //                  model and precision (64x128x128: 131 -> 109);
 //   NZ = 64        FP64 groups of few runs take it too: 16x16 42.0 -> 36.6,
-//                  32x32 43.7 -> 39.9, 36x60 54.2 -> 45.7, 128x128 113.6 -> 100.4;
+//                  32x32 43.7 -> 39.9, 36x60 54.2 -> 45.7, 128x128 113.6 -> 100.4.
+//                  HD_fullU, with three lines per mode, up to WAVE_MODES_HD modes
+//                  (160x160 108.8 against 113.9, 176x176 127.9 against 124.1, 256x256
+//                  217.2 against 204.5), MHD_BQlin up to WAVE_MODES_BQ (256x256 272.8
+//                  against 281.4, 360x360 528 against 530, 512x512 1030 against 1017);
 //   NZ = 32        up to 512 modes (16x16 41.4 -> 34.6, 32x32 42.3 -> 36.1); beyond
 //                  that eight modes per pass keep more lanes busy (128x128 74.8
 //                  against 82.7);
@@ -70,15 +74,16 @@ inline int mb_for(int NZ, int line) { return (line == LINE_WAVE || NZ >= line) ?
 // groups: there eight (four) modes per pass and two launches measured best (48
 // runs: 160.0 us per step; wavefront kernel at NZ = 64 164.0, one-launch tail
 // 166-172; at 8 runs the one-launch tail won, 97.6 -> 79.0).
-constexpr int SMALL_SET = 4, SMALL_MODES = 512;
+constexpr int SMALL_SET = 4, SMALL_MODES = 512, WAVE_MODES_HD = 14000, WAVE_MODES_BQ = 60000;
 struct Shape {
     int line, target;
 };
 inline bool small_set(int precision, int nruns) { return precision == QL_PREC_FP64 && nruns <= SMALL_SET; }
-inline Shape default_shape(int NZ, int precision, int nruns, int modes)
+inline Shape default_shape(int NZ, int model, bool hd, int precision, int nruns, int modes)
 {
     if (NZ >= 128) return Shape{LINE_WAVE, 256};
-    if (small_set(precision, nruns) && (NZ == 64 || modes <= SMALL_MODES))
+    const int at64 = hd ? WAVE_MODES_HD : (model == QL_MODEL_MHD_BQLIN ? WAVE_MODES_BQ : modes);
+    if (small_set(precision, nruns) && modes <= (NZ == 64 ? at64 : SMALL_MODES))
         return Shape{LINE_WAVE, modes / 4 < 64 ? 64 : (modes / 4 < 256 ? modes / 4 : 256)};
     return Shape{DEFAULT_LINE, DEFAULT_TARGET};
 }

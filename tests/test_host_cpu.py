@@ -220,6 +220,16 @@ def s_transform_on_default_shape(host):
         assert _refused(_context(**kw).set_transform, kw["NZ"], 1)
 
 
+def s_large_boxes(host):
+    from ql_dns_amd.capi import QLContext
+    from ql_dns_amd.params import QLParams
+    for model, NX, line in ((2, 160, 64), (2, 176, 256), (1, 176, 64), (1, 350, 256), (0, 176, 64), (0, 350, 64)):
+        c = QLContext(QLParams(model=model, NX=NX, NY=NX, NZ=64))
+        assert c.config()[0]["line"] == line, (model, NX)
+        assert c.config()[0]["tail"] == (1 if line == 64 else 0)  # 256 workgroups, or 512
+        c.close()
+
+
 def s_tail_follows_the_shape(host):
     from ql_dns_amd.params import QLParams
     c = _context(NX=36, NY=60, NZ=64)
@@ -450,6 +460,11 @@ def test_creation_waits_once_and_pins_nothing(runtime):
     """A new context waits for the clearing of its buffers as a whole, not for each
     (30 waits took 0.24 ms of a small context's 0.6), and has no pinned memory."""
     scenario(runtime, "creation")
+
+
+def test_default_shapes_of_large_boxes(runtime):
+    """At NZ = 64 large boxes of HD_fullU and MHD_BQlin are faster on the workgroup kernel."""
+    scenario(runtime, "large_boxes")
 
 
 def test_default_tail_follows_the_shape(runtime):
