@@ -248,26 +248,31 @@ int ql_batch_tune(ql_batch *b, int trial_steps, double *step_ms);
 /* Transform of the workgroup mode kernel for the NZ group (fftwPlans.h:33-97):
  * the LDS radix passes (QL_TRANSFORM_FFT, the default) or dense complex
  * matrix products on the matrix cores (QL_TRANSFORM_DFT_MFMA: FP64, NZ 32 or
- * 64, line 128 or 256, else QL_ERR_ARG).  ql_batch_tune times both where both
- * exist.  A later ql_batch_set_config keeps it where the new shape has it. */
+ * 64, line 128 or 256, else QL_ERR_ARG; a group nobody has set or tuned a shape
+ * for moves to line 256 with it, and back).  ql_batch_tune times both where
+ * both exist.  A later ql_batch_set_config keeps it where the new shape has
+ * it. */
 enum { QL_TRANSFORM_FFT = 0, QL_TRANSFORM_DFT_MFMA = 1 };
 int ql_batch_set_transform(ql_batch *b, int NZ, int transform);
 /* Substep tail of the NZ group: the column reduction and the mean-field
  * kernel as two launches (QL_TAIL_TWO_KERNELS) or one launch with a workgroup
  * per mean field and run (QL_TAIL_FUSED: fixed steps, NZ <= 128, at most
- * 65536 / NZ partial rows per run, else QL_ERR_ARG; the default for FP64 sets
- * of few runs at NZ <= 64 except MHD_BQlin's).  Both sum the
- * stress / EMF partial rows in the same order: the results are bitwise equal.
+ * 65536 / NZ partial rows per run, else QL_ERR_ARG).  Unless a tail has been
+ * set or tuned, a group has one launch with fixed steps in FP64 at NZ <= 64
+ * with up to four runs of at most 16384 / NZ partial rows each in its current
+ * shape, else two.  Both sum the stress / EMF partial rows in the same order:
+ * the results are bitwise equal for MHD_FullQlin and HD_fullU; MHD_BQlin's
+ * agree to rounding, as between two shapes.
  * No counterpart in the reference (its MPI Allreduce, MHD_FullQlin.cpp:386,
  * followed by the mean-field update, :386-423). */
 enum { QL_TAIL_TWO_KERNELS = 0, QL_TAIL_FUSED = 1 };
 int ql_batch_set_tail(ql_batch *b, int NZ, int tail);
 /* Mixed precision (QL_PREC_MIXED): a mode whose largest |value| reaches tau
- * times the largest of its run runs in FP64 (a companion launch of the FP64
- * kernel before the FP32 one), the others in FP32; the choice is made again
- * every 16 steps of the clock and after each state upload.  Sets tau when
- * tau > 0 (default 0.03; tau <= 0 leaves it; tau > 1, which no mode reaches,
- * runs every mode in FP32 with neither the flags nor the FP64 launch) and
+ * times the largest of its run runs in FP64 (in the same launch at line 64, in
+ * a companion launch before the FP32 one otherwise), the others in FP32; the
+ * choice is made again every 16 steps and after each state upload.  Sets tau
+ * when tau > 0 (default 0.03; tau <= 0 leaves it; tau > 1, which no mode
+ * reaches, runs every mode in FP32 without the flags) and
  * writes to *nfp64 (may be NULL) how many modes of the set reach it for the
  * current state. */
 int ql_batch_mixed_split(ql_batch *b, double tau, int *nfp64);
@@ -278,7 +283,7 @@ enum { QL_CONFIG_INTS = 7 };
 int ql_batch_get_config(const ql_batch *b, int max_groups, int *ngroups, int *cfg);
 /* sets the shape of the NZ group: line in {64, 128, 256}, target >= 1.
  * line 64 selects the kernel with one wavefront per mode (modes per pass 1;
- * every model; at NZ = 256 FP64 only except for HD_fullU, else QL_ERR_ARG) */
+ * every model and precision) */
 int ql_batch_set_config(ql_batch *b, int NZ, int line, int target);
 
 /* ------------------------------------------------------------------------
@@ -305,7 +310,9 @@ int ql_batch_set_config(ql_batch *b, int NZ, int line, int target);
  * gradients as dL/dRe + i dL/dIm), returns dL/d(state before the forward) in
  * g_lin0 / g_mf0 (NULL to skip) and g_par[0..4] = dL/d(q, omega, nu, eta,
  * B0z).  Segments are recomputed from their checkpoints; the context is left
- * at the forward's final state. */
+ * at the forward's final state, its drives and step record included.  The
+ * buffers stay with the context; those of a backward make way where a later
+ * forward's checkpoints need the memory. */
 int ql_adjoint_forward(ql_ctx *ctx, int nsteps, int every, double *t_inout);
 int ql_adjoint_backward(ql_ctx *ctx, const double *g_lin, const double *g_mf, double *g_lin0, double *g_mf0,
                         double g_par[5]);

@@ -70,10 +70,12 @@ inline int mb_for(int NZ, int line) { return (line == LINE_WAVE || NZ >= line) ?
 //                  against 82.7);
 //   few modes      at least 64 workgroups, then four modes each: fewer rows for
 //                  the tail to sum (32x32x64: 124 workgroups 39.9, 248 41.8);
-// Groups of more than SMALL_SET runs fill the chip and share it with the other
-// groups: there eight (four) modes per pass and two launches measured best (48
-// runs: 160.0 us per step; wavefront kernel at NZ = 64 164.0, one-launch tail
-// 166-172; at 8 runs the one-launch tail won, 97.6 -> 79.0).
+// Groups of more than SMALL_SET runs: eight (four) modes per pass and two
+// launches, which measured best where several groups share the chip (48 uneven
+// runs of three NZ: 160.0 us per step; wavefront kernel at NZ = 64 164.0, one-launch
+// tail 166-172).  Not so for a set of one NZ, where one launch takes 5 us less
+// per step at 5 to 48 runs (8 runs of 16x16x32 39.8 and 35.1, with the wavefront
+// kernel 32.8): the tuner finds that.
 constexpr int SMALL_SET = 4, SMALL_MODES = 512, WAVE_MODES_HD = 14000, WAVE_MODES_BQ = 60000;
 struct Shape {
     int line, target;

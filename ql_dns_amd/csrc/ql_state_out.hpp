@@ -48,7 +48,8 @@ namespace qlh {
 
 // Pieces of at most OUT_SLOT bytes, OUT_SLOTS of them in flight; from
 // OUT_THREADED pieces on, copied by up to OUT_SLOTS threads, whose start takes
-// as long as half a piece's copy (pieces of 1 MiB, 16 of them, measured the same)
+// as long as half a piece's copy (a state of 89 MB 2.2 ms; eight pieces of 1 MiB 2.8,
+// of 512 KiB 4.0, sixteen of 512 KiB 3.0)
 constexpr size_t OUT_SLOT = (size_t)2 << 20;
 constexpr int OUT_SLOTS = 8, OUT_THREADED = 3;
 
