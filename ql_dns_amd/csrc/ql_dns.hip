@@ -1353,6 +1353,7 @@ int tune(Batch &b, int trial_steps, double *best_ms_out)
     for (size_t gi = 0; gi < b.groups.size() && rc == QL_OK; ++gi) {
         Group &g = b.groups[gi];
         double best = 1e300;
+        const int line0 = g.line, target0 = g.target, dft0 = g.dft;
         int best_line = g.line, best_target = g.target, best_dft = g.dft, best_tail = g.tail;
         std::vector<std::pair<int, int>> seen;  // (kernel and MB, W) already timed
         for (int cand = 0; cand < 2 * (int)(sizeof(LINES) / sizeof(LINES[0])); ++cand) {
@@ -1398,10 +1399,15 @@ int tune(Batch &b, int trial_steps, double *best_ms_out)
             }
             if (rc) break;
         }
-        g.dft = best_dft;
-        g.own_tail = best_tail;
-        g.own_shape = true;
-        if (rc == QL_OK) rc = configure(b, g, best_line, best_target);
+        if (rc == QL_OK) {
+            g.dft = best_dft;
+            g.own_tail = best_tail;
+            g.own_shape = true;
+            rc = configure(b, g, best_line, best_target);
+        } else {  // the shape it had
+            g.dft = dft0;
+            (void)configure(b, g, line0, target0);
+        }
         total_best += best;
     }
     // the replay graphs of the chosen shapes, captured here, so that the

@@ -368,13 +368,20 @@ def s_shape_without_memory(host, precision):
 def s_tune_without_memory(host):
     from ql_dns_amd.capi import QLBatch
     from ql_dns_amd.params import QLParams
-    ps = [QLParams(NX=8, NY=6, NZ=NZ) for NZ in (32, 64)]
+    ps = [QLParams(NX=8, NY=6, NZ=32), QLParams(NX=20, NY=20, NZ=64)]
     states = []
     for r, p in enumerate(ps):
-        c = _context(NX=8, NY=6, NZ=p.NZ)
+        c = _context(NX=p.NX, NY=p.NY, NZ=p.NZ)
         states.append(_state(c, r))
         c.close()
-    for k in range(0, 11):  # five buffers per group
+    b = QLBatch(ps)
+    shape = b.config()[1]
+    n = host.mallocs()
+    b.tune(1)
+    n = host.mallocs() - n  # five buffers per group, and those of larger shapes
+    assert n > 10
+    b.close()
+    for k in range(0, n + 1):
         b = QLBatch(ps)
         for r, st in enumerate(states):
             b.set_state(r, *st)
@@ -382,7 +389,11 @@ def s_tune_without_memory(host):
         if k:
             host.fail_malloc(k)
             assert _fails(b.tune, 1), k
-            assert host.live() == live, k
+            assert host.live() >= live and (host.live() == live or k > 10), k
+            assert b.config()[1] == shape, k
+            b.set_transform(64, 1)  # the shape is still nobody's
+            b.set_transform(64, 0)
+            assert b.config()[1] == shape, k
         else:
             b.tune(1)
         for r, (lin, mf) in enumerate(states):
@@ -441,6 +452,7 @@ def test_downloads_of_several_threads(runtime):
 
 
 def test_tuning_there_is_no_memory_for_keeps_the_state(runtime):
+    """And the launch shapes."""
     scenario(runtime, "tune_without_memory")
 
 
